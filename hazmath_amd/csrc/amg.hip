@@ -166,7 +166,10 @@ int amg_setup(Hierarchy &H, const DevCSR &A0, AMG_param *param, bool) {
     if (max_levels > HZ_MAX_AMG_LVL) max_levels = HZ_MAX_AMG_LVL;
     H.lv.assign(max_levels, Level{});
     H.lv[0].A = A0;
-    sell_from_csr(H.lv[0].A, H.lv[0].S);
+    // assembled matrices hold structural zeros (8 of the 15 entries of a Kuhn
+    // row): the solve's SELL copies leave them out.  A level without any has
+    // none to pass on to the next one, which then skips the counting pass.
+    sell_from_csr(H.lv[0].A, H.lv[0].S, true);
     int *counts = arena().alloc_n<int>((size_t)A0.n + 1);
     int lvl = 0;
     const int type = param->aggregation_type;
@@ -281,7 +284,7 @@ int amg_setup(Hierarchy &H, const DevCSR &A0, AMG_param *param, bool) {
             build_restriction(n, L.agg, nagg, L.rptr, L.rmem);
             rap_agg(L.A, L.agg, nagg, L.rptr, L.rmem, C.A);
         }
-        sell_from_csr(C.A, C.S);
+        sell_from_csr(C.A, C.S, L.S.nnz < L.A.nnz);
         if (tr) {
             HZ_CHECK(hipStreamSynchronize(stream()));
             t3 = wall_ms();

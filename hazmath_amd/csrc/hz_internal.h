@@ -18,7 +18,7 @@ struct DevCSR {
 // same order as the CSR loops of the reference.
 struct DevSELL {
     int n = 0, nslices = 0;
-    long long nnz = 0;         // stored CSR entries (algorithmic bytes count these, not the padding)
+    long long nnz = 0;         // entries without the padding (algorithmic bytes count these)
     long long nent = 0;        // padded entries
     long long *sptr = nullptr; // nslices+1 offsets
     int *len = nullptr;        // row lengths
@@ -31,6 +31,15 @@ struct DevSELL {
     // cycle's level has them; null otherwise
     unsigned int *pcol = nullptr;
 };
+
+// Entries a round of the masked SELL kernels: 8 where the slices are at most 8
+// wide on average (stored zeros left out: 7-point rows), else 16.  launch takes
+// the count as a std::integral_constant.
+template <class F>
+void by_round(const DevSELL &S, F &&launch) {
+    if (S.nent <= 8LL * kSlice * S.nslices) launch(std::integral_constant<int, 8>{});
+    else launch(std::integral_constant<int, 16>{});
+}
 
 // Device scalars of the PCG (one 256-byte block; host copies it back once per
 // iteration).
@@ -98,7 +107,9 @@ struct LaunchTimer {
 };
 
 // ---- kernels_solve.hip ----------------------------------------------------
-void sell_from_csr(const DevCSR &A, DevSELL &S);
+// drop_zeros: stored off-diagonal zeros are left out (a product with one adds
+// nothing to a row's sum, so every finite result is the same).
+void sell_from_csr(const DevCSR &A, DevSELL &S, bool drop_zeros = false);
 // y = A x ; if dot_out: *dot_out = sum_i y_i * x_i (deterministic).  timer:
 // events around the SpMV kernel itself (not the partials' finalize).
 // cols_only: the PCG's SpMV ahead of an FP32 cycle, which shares only the

@@ -96,10 +96,13 @@ __global__ void k_jp_round(int n, const int *__restrict__ ia, const int *__restr
     if (local && left) atomicAdd(left, local);
 }
 
-__global__ void k_offdiag_count(int n, const int *__restrict__ ia, const int *__restrict__ ja, int *__restrict__ cnt) {
+// Off-diagonal entries a sweep reads: stored zeros are left out (a product with
+// one changes no sum); the colouring sees the whole pattern.
+__global__ void k_offdiag_count(int n, const int *__restrict__ ia, const int *__restrict__ ja,
+                                const double *__restrict__ a, int *__restrict__ cnt) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         int c = 0;
-        for (int k = ia[i]; k < ia[i + 1]; ++k) c += ja[k] != i;
+        for (int k = ia[i]; k < ia[i + 1]; ++k) c += ja[k] != i && a[k] != 0.0;
         cnt[i] = c;
     }
 }
@@ -128,7 +131,7 @@ __global__ void k_gs_fill(int nslices, const int *__restrict__ spos, const int *
             const int j = ja[k];
             if (j == i) {
                 d = a[k];
-            } else {
+            } else if (a[k] != 0.0) {
                 col[base + (long long)k2 * kSlice + lane] = pos_of[j];
                 val[base + (long long)k2 * kSlice + lane] = a[k];
                 ++k2;
@@ -297,7 +300,7 @@ void gs_prepare(const DevCSR &A, GsLevel &G) {
         if (hl == 0) break;
     }
     std::vector<int> color(n), offd(n);
-    k_offdiag_count<<<grid_rows(n), kBlock, 0, st>>>(n, A.ia, A.ja, c1);
+    k_offdiag_count<<<grid_rows(n), kBlock, 0, st>>>(n, A.ia, A.ja, A.val, c1);
     HZ_LAUNCH_CHECK();
     HZ_CHECK(memcpy_sync(color.data(), c0, sizeof(int) * n, hipMemcpyDeviceToHost));
     HZ_CHECK(memcpy_sync(offd.data(), c1, sizeof(int) * n, hipMemcpyDeviceToHost));

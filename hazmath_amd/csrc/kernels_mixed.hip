@@ -120,7 +120,7 @@ __global__ void k_enter(int n, const double *__restrict__ r, int smoother, float
 // One sweep (Jacobi with weight w / L1DIAG) in FP32, optionally with the
 // prolongation x + P xc folded into every x read, optionally writing the
 // result in FP64 (out64) with block partials of sum_i out64_i r64_i.
-template <int kSmoother, bool kProlong, bool kOut64, class MT, bool kKeepCol = false>
+template <int kSmoother, bool kProlong, bool kOut64, class MT, int U, bool kKeepCol = false>
 __global__ __launch_bounds__(kBlock) void k_sweep_m(int n, int nslices, const long long *__restrict__ sptr,
                                                     const int *__restrict__ col, const MT *__restrict__ val,
                                                     float wgt, const int *__restrict__ agg,
@@ -141,28 +141,28 @@ __global__ __launch_bounds__(kBlock) void k_sweep_m(int n, int nslices, const lo
         const MT *v = val + base + lane;
         float t = (r < n) ? b[r] : 0.0f;
         float d = 0.0f;
-        // rounds of 16 entries masked past the slice width (a 15-entry row in one
-        // round): all loads of a round issued before its math
-        constexpr bool kMask = true;
-        constexpr int U = 16;
-        int k = 0;
-        for (; kMask ? (k < wd) : (k + U <= wd); k += U) {
+        // rounds of U entries masked past the slice width (a 15-entry row in one
+        // round of 16): all loads of a round issued before its math
+        for (int k = 0; k < wd; k += U) {
             int cc[U];
             float vv[U], xx[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const bool ok = !kMask || k + u < wd;
+                const bool ok = k + u < wd;
                 cc[u] = ok ? (kKeepCol ? c[(k + u) * kSlice] : ld_nt(c + (k + u) * kSlice)) : -1;
                 vv[u] = ok ? ldv(v + (k + u) * kSlice) : 0.0f;
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) xx[u] = cc[u] >= 0 ? x[cc[u]] : 0.0f;
             if (kProlong) {
+                int gg[U];
+                float xg[U];
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const int g = cc[u] >= 0 ? agg[cc[u]] : HZ_UNPT;
-                    if (g > HZ_UNPT) xx[u] = xx[u] + xc[g];
-                }
+                for (int u = 0; u < U; ++u) gg[u] = cc[u] >= 0 ? agg[cc[u]] : HZ_UNPT;
+#pragma unroll
+                for (int u = 0; u < U; ++u) xg[u] = gg[u] > HZ_UNPT ? xc[gg[u]] : 0.0f;
+#pragma unroll
+                for (int u = 0; u < U; ++u) xx[u] = gg[u] > HZ_UNPT ? xx[u] + xg[u] : xx[u];
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -175,24 +175,6 @@ __global__ __launch_bounds__(kBlock) void k_sweep_m(int n, int nslices, const lo
                     if (cc[u] == r) d = vv[u];
                     else if (cc[u] >= 0) t = t - vv[u] * xx[u];
                 }
-            }
-        }
-        for (; k < wd; ++k) {
-            const int cj = ld_nt(c + k * kSlice);
-            const float a = ldv(v + k * kSlice);
-            float xj = cj >= 0 ? x[cj] : 0.0f;
-            if (kProlong && cj >= 0) {
-                const int g = agg[cj];
-                if (g > HZ_UNPT) xj = xj + xc[g];
-            }
-            if (kSmoother == HZ_SMOOTHER_L1DIAG) {
-                if (cj >= 0) {
-                    t = t - a * xj;
-                    d = d + fabsf(a);
-                }
-            } else {
-                if (cj == r) d = a;
-                else if (cj >= 0) t = t - a * xj;
             }
         }
         if (r < n) {
@@ -221,7 +203,7 @@ __global__ __launch_bounds__(kBlock) void k_sweep_m(int n, int nslices, const lo
     }
 }
 
-template <class MT, class CT>
+template <class MT, class CT, int U>
 __global__ __launch_bounds__(kBlock) void k_residual_m(int n, int nslices, const long long *__restrict__ sptr,
                                                        const CT *__restrict__ col, const MT *__restrict__ val,
                                                        const float *__restrict__ b, const float *__restrict__ x,
@@ -234,8 +216,7 @@ __global__ __launch_bounds__(kBlock) void k_residual_m(int n, int nslices, const
     const int wd = (int)((sptr[s + 1] - base) / kSlice);
     const CT *c = col + col_base<CT>(base, s) + lane;
     const MT *v = val + base + lane;
-    float acc = 0.0f;
-    constexpr int U = 16;   // rounds of 16 masked past the slice width
+    float acc = 0.0f;   // rounds of U masked past the slice width
     for (int k = 0; k < wd; k += U) {
         int cc[U];
         float vv[U], xx[U];
@@ -564,8 +545,10 @@ void launch_sweep_m(const DevSELL &S, const MT *val, float w, const int *agg, co
     // shares the column indices: they are loaded with ordinary loads and stay
     // in the last-level cache for it (PCG SpMV 81 -> 69 us, FP32-cycle PCG
     // 20.8 -> 20.4 ms at 128^3)
-    k_sweep_m<kSm, kPro, kOut, MT, kOut><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, val, w, agg,
-                                                                         xc, b, x, xout, out64, r64, partials);
+    by_round(S, [&](auto u) {
+        k_sweep_m<kSm, kPro, kOut, MT, decltype(u)::value, kOut><<<grid, kBlock, 0, stream()>>>(
+            S.n, S.nslices, S.sptr, S.col, val, w, agg, xc, b, x, xout, out64, r64, partials);
+    });
     HZ_LAUNCH_CHECK();
 }
 
@@ -716,22 +699,20 @@ void residual_m(const DevSELL &S, const LowMatrix &M, const float *b, const floa
         else
             k_residual_grp_m<G, unsigned short><<<g, kBlock, 0, stream()>>>(
                 S.n, A->ia, A->ja, static_cast<const unsigned short *>(M.csr), b, x, w);
-    } else if (M.kind == kLowF32) {
-        const float *v = static_cast<const float *>(M.sell);
-        if (dcol)
-            k_residual_m<float, unsigned int><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, dcol, v,
-                                                                             b, x, w);
-        else
-            k_residual_m<float, int><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, v, b, x,
-                                                                    w);
     } else {
-        const unsigned short *v = static_cast<const unsigned short *>(M.sell);
-        if (dcol)
-            k_residual_m<unsigned short, unsigned int><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, dcol, v,
-                                                                                      b, x, w);
-        else
-            k_residual_m<unsigned short, int><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col,
-                                                                              v, b, x, w);
+        by_round(S, [&](auto u) {
+            constexpr int U = decltype(u)::value;
+            auto go = [&](auto *v) {
+                using MT = std::remove_const_t<std::remove_pointer_t<decltype(v)>>;
+                if (dcol)
+                    k_residual_m<MT, unsigned int, U><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, dcol, v, b,
+                                                                                     x, w);
+                else
+                    k_residual_m<MT, int, U><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, v, b, x, w);
+            };
+            if (M.kind == kLowF32) go(static_cast<const float *>(M.sell));
+            else go(static_cast<const unsigned short *>(M.sell));
+        });
     }
     HZ_LAUNCH_CHECK();
 }

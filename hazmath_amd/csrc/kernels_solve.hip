@@ -43,6 +43,61 @@ __global__ void k_slice_width(int n, const int *__restrict__ ia, long long *__re
 // rest) -- what k_smoother_diag computes from the SELL copy -- and the first
 // stored diagonal entry (dcsr_getdiag, which the strength graph reads).
 constexpr int kSellStage = 1024;
+
+// Slice widths without the stored off-diagonal zeros (k_sell_fill<true> leaves
+// them out).  A wave loads its slice's entries coalesced, 64 at a time, keeps
+// one bit an entry in LDS, and each lane counts its row's bits; the column of
+// a zero entry is looked at to keep diagonal ones.  kept: entries kept, over
+// kKeptParts counters in lines of their own (with one counter for all waves
+// its atomics took 70 of the 97 us at 438,976 rows).
+constexpr int kKeptParts = 32, kKeptStride = 8;
+__global__ __launch_bounds__(kBlock) void k_slice_width_nz(int n, const int *__restrict__ ia,
+                                                           const int *__restrict__ ja,
+                                                           const double *__restrict__ val,
+                                                           long long *__restrict__ wcount, int nslices,
+                                                           unsigned long long *__restrict__ kept) {
+    __shared__ unsigned long long bits[kSlicesPerBlock][kSellStage / kWave];
+    const int wv = threadIdx.x / kWave;
+    const int s = blockIdx.x * kSlicesPerBlock + wv;
+    const int lane = threadIdx.x % kWave;
+    if (s >= nslices) return;
+    const int e0 = ia[s * kSlice], e1 = ia[min(n, (s + 1) * kSlice)];
+    const bool staged = e1 - e0 <= kSellStage;
+    if (staged) {
+        double v[kSellStage / kWave];
+#pragma unroll
+        for (int c = 0; c < kSellStage / kWave; ++c) {
+            const int e = e0 + c * kWave + lane;
+            v[c] = e < e1 ? ld_nt(val + e) : 0.0;
+        }
+#pragma unroll
+        for (int c = 0; c < kSellStage / kWave; ++c) {
+            const unsigned long long m = __ballot(v[c] != 0.0);
+            if (lane == 0) bits[wv][c] = m;
+        }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the masks are this wave's own
+    __builtin_amdgcn_wave_barrier();
+    const int r = s * kSlice + lane;
+    int len = 0;
+    if (r < n)
+        for (int k = ia[r]; k < ia[r + 1]; ++k) {
+            const bool nz = staged ? (bits[wv][(k - e0) / kWave] >> ((k - e0) % kWave)) & 1ull : val[k] != 0.0;
+            len += nz || ja[k] == r;
+        }
+    int widest = len;
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+        widest = max(widest, __shfl_xor(widest, off, kWave));
+        len += __shfl_xor(len, off, kWave);
+    }
+    if (lane == 0) {
+        wcount[s] = (long long)widest * kSlice;
+        if (len) atomicAdd(kept + (s % kKeptParts) * kKeptStride, (unsigned long long)len);
+    }
+}
+
+template <bool kDropZeros>
 __global__ __launch_bounds__(kBlock) void k_sell_fill(int n, const int *__restrict__ ia, const int *__restrict__ ja,
                                                       const double *__restrict__ val,
                                                       const long long *__restrict__ sptr, int *__restrict__ scol,
@@ -70,27 +125,32 @@ __global__ __launch_bounds__(kBlock) void k_sell_fill(int n, const int *__restri
     if (!active) return;
     const long long base = sptr[s];
     const int w = (int)((sptr[s + 1] - base) / kSlice);
-    const int beg = (r < n) ? ia[r] : 0;
-    const int len = (r < n) ? ia[r + 1] - beg : 0;
+    const int end = (r < n) ? ia[r + 1] : 0;
+    int q = (r < n) ? ia[r] : 0;
     double l1 = 0.0, dj = 0.0, df = 0.0;
     bool seen = false;
     for (int k = 0; k < w; ++k) {
         const long long e = base + (long long)k * kSlice + lane;
-        if (k < len) {
-            const int q = beg + k;
-            const int j = staged ? s_col[wv][q - e0] : ja[q];
-            const double a = staged ? s_val[wv][q - e0] : val[q];
-            scol[e] = j;
-            sval[e] = a;
+        int j = -1;
+        double a = 0.0;
+        for (; q < end; ++q) {
+            const int jq = staged ? s_col[wv][q - e0] : ja[q];
+            const double aq = staged ? s_val[wv][q - e0] : val[q];
+            if (kDropZeros && aq == 0.0 && jq != r) continue;
+            j = jq;
+            a = aq;
+            ++q;
+            break;
+        }
+        scol[e] = j;
+        sval[e] = a;
+        if (j >= 0) {
             l1 = l1 + fabs(a);
             if (j == r) {
                 dj = a;
                 if (!seen) df = a;
                 seen = true;
             }
-        } else {
-            scol[e] = -1;
-            sval[e] = 0.0;
         }
     }
     if (r < n) {
@@ -107,10 +167,11 @@ __global__ __launch_bounds__(kBlock) void k_sell_fill(int n, const int *__restri
 // kKeep 1: the second half of each round uses ordinary loads, whose lines
 // stay in the last-level cache for the next kernel that streams the same
 // matrix; kKeep 2: every load is ordinary; kKeep 4: the column indices only.
-template <bool kNtTail, bool kWide = false, int kKeep = 0, class CT = int>
+template <bool kNtTail, int kWide = 0, int kKeep = 0, class CT = int>
 __device__ __forceinline__ double sell_row_dot(const CT *c, const double *v, int w, const double *x, int r) {
-    // kWide: rounds of 16 masked past the slice width (a 15-entry row in one round)
-    constexpr int U = kWide ? 16 : 8;
+    // kWide: rounds of that many entries masked past the slice width (a 15-entry
+    // row in one round of 16, a 7-entry row in one of 8)
+    constexpr int U = kWide ? kWide : 8;
     static_assert(kWide || std::is_same_v<CT, int>, "paired offsets: masked rounds only");
     constexpr int kKeepFrom = (kKeep == 2 || kKeep == 4) ? 0 : (kKeep == 1 ? U / 2 : U);
     double acc = 0.0;
@@ -139,7 +200,7 @@ __device__ __forceinline__ double sell_row_dot(const CT *c, const double *v, int
 }
 
 // y = A x (row sums from 0.0 in CSR order); optional deterministic (y, x).
-template <bool kDot, bool kWide = false, int kKeep = 0, class CT = int>
+template <bool kDot, int kWide = 0, int kKeep = 0, class CT = int>
 __global__ __launch_bounds__(kBlock) void k_spmv(int n, int nslices, const long long *__restrict__ sptr,
                                                  const CT *__restrict__ col,
                                                  const double *__restrict__ val,
@@ -170,7 +231,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv(int n, int nslices, const long 
 }
 
 // w = b - A x  (array_cp + dcsr_aAxpy(-1.0): row sum t from 0.0, then b - t)
-template <bool kWide = false, int kKeep = 0, class CT = int>
+template <int kWide = 0, int kKeep = 0, class CT = int>
 __global__ __launch_bounds__(kBlock) void k_residual(int n, int nslices, const long long *__restrict__ sptr,
                                                      const CT *__restrict__ col,
                                                      const double *__restrict__ val,
@@ -206,9 +267,9 @@ __device__ __forceinline__ double prolong_value(double xj, int g, double xcg, do
 // Jacobi (smoother.c:35-92): t = b - sum_{j!=i} a_ij x_j, d = last diagonal
 // entry; x_i <- (1-w) x_i + w t / d when |d| > SMALLREAL.
 // L1DIAG (smoother.c:324-381): t = b - sum_j a_ij x_j, d = sum_j |a_ij|; x_i += t/d.
-// Entries are consumed four at a time with all their loads issued first, so a
+// Entries are consumed U at a time with all their loads issued first, so a
 // row costs a few dependent memory round trips instead of one per entry.
-template <int kSmoother, bool kProlong, bool kDot, bool kWide = false, class CT = int>
+template <int kSmoother, bool kProlong, bool kDot, int U, class CT = int>
 __global__ __launch_bounds__(kBlock) void k_sweep(int n, int nslices, const long long *__restrict__ sptr,
                                                   const CT *__restrict__ col,
                                                   const double *__restrict__ val, double wgt,
@@ -233,27 +294,21 @@ __global__ __launch_bounds__(kBlock) void k_sweep(int n, int nslices, const long
         const double *v = val + base + lane;
         double t = (r < n) ? b[r] : 0.0;
         double d = 0.0;
-        // entries per round: loads first (matrix non-temporal), then the math in
-        // order.  With the prolongation folded in (the latency-bound small
-        // levels) rounds are 16 wide and masked past the slice width, so a
-        // 15-entry row takes one round; otherwise 8 wide plus a tail.
-        constexpr bool kMask = kProlong || kWide;
-        constexpr int U = kMask ? 16 : 8;
-        static_assert(kMask || std::is_same_v<CT, int>, "paired offsets: masked rounds only");
-        int k = 0;
-        for (; kMask ? (k < wd) : (k + U <= wd); k += U) {
+        // rounds of U entries masked past the slice width (U = 8 where rows are
+        // short): loads first (matrix non-temporal), then the math in order
+        for (int k = 0; k < wd; k += U) {
             int cc[U];
             double vv[U], xx[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const bool ok = !kMask || k + u < wd;
+                const bool ok = k + u < wd;
                 // the fine level's last sweep (kDot) precedes the PCG SpMV: the
                 // second half of each round uses ordinary loads, which stay in the
                 // last-level cache for that SpMV
-                const bool keep = kWide && kDot && u >= 8;
+                const bool keep = !kProlong && kDot && u >= U / 2;
                 vv[u] = ok ? (keep ? v[(k + u) * kSlice] : ld_nt(v + (k + u) * kSlice)) : 0.0;
             }
-            ld_cols<U, (kWide && kDot) ? 8 : U>(c, k, wd, r, cc);
+            ld_cols<U, (!kProlong && kDot) ? U / 2 : U>(c, k, wd, r, cc);
 #pragma unroll
             for (int u = 0; u < U; ++u) xx[u] = cc[u] >= 0 ? x[cc[u]] : 0.0;
             if (kProlong) {
@@ -277,24 +332,6 @@ __global__ __launch_bounds__(kBlock) void k_sweep(int n, int nslices, const long
                     if (cc[u] == r) d = vv[u];
                     else if (cc[u] >= 0) t = t - vv[u] * xx[u];
                 }
-            }
-        }
-        for (; k < wd; ++k) {
-            const int cj = c[k * kSlice];
-            const double a = v[k * kSlice];
-            double xj = cj >= 0 ? x[cj] : 0.0;
-            if (kProlong && cj >= 0) {
-                const int g = agg[cj];
-                xj = prolong_value(xj, g, g > HZ_UNPT ? xc[g] : 0.0, al);
-            }
-            if (kSmoother == HZ_SMOOTHER_L1DIAG) {
-                if (cj >= 0) {
-                    t = t - a * xj;
-                    d = d + fabs(a);
-                }
-            } else {
-                if (cj == r) d = a;
-                else if (cj >= 0) t = t - a * xj;
             }
         }
         if (r < n) {
@@ -633,16 +670,24 @@ inline int stream_grid(long n) {
 double g_alg_bytes = 0.0;
 
 
-void sell_from_csr(const DevCSR &A, DevSELL &S) {
+void sell_from_csr(const DevCSR &A, DevSELL &S, bool drop_zeros) {
     S.n = A.n;
     S.nnz = A.nnz;
     S.nslices = div_up(A.n, kSlice);
     const int ns = S.nslices;
     long long *wcount = arena().alloc_n<long long>((size_t)ns + 1);
-    S.sptr = arena().alloc_n<long long>((size_t)ns + 1);
+    // the counters of kept entries follow the offsets: one copy brings both back
+    constexpr int kParts = kKeptParts * kKeptStride;
+    S.sptr = arena().alloc_n<long long>((size_t)ns + 1 + kParts);
     hipStream_t st = stream();
+    if (drop_zeros) HZ_CHECK(hipMemsetAsync(S.sptr + ns + 1, 0, sizeof(long long) * kParts, st));
     if (ns > 0) {
-        k_slice_width<<<div_up(ns, kSlicesPerBlock), kBlock, 0, st>>>(A.n, A.ia, wcount, ns);
+        const int grid = div_up(ns, kSlicesPerBlock);
+        if (drop_zeros)
+            k_slice_width_nz<<<grid, kBlock, 0, st>>>(A.n, A.ia, A.ja, A.val, wcount, ns,
+                                                      reinterpret_cast<unsigned long long *>(S.sptr + ns + 1));
+        else
+            k_slice_width<<<grid, kBlock, 0, st>>>(A.n, A.ia, wcount, ns);
         HZ_LAUNCH_CHECK();
     }
     // exclusive scan of slice sizes (padded entries)
@@ -653,18 +698,28 @@ void sell_from_csr(const DevCSR &A, DevSELL &S) {
     void *tmp = arena().alloc(tmp_bytes);
     HZ_CHECK(rocprim::exclusive_scan(tmp, tmp_bytes, wcount, S.sptr, 0LL, (size_t)ns + 1,
                                      rocprim::plus<long long>(), st));
-    long long nent = 0;
-    HZ_CHECK(hipMemcpyAsync(&nent, S.sptr + ns, sizeof(long long), hipMemcpyDeviceToHost, st));
+    long long tail[1 + kParts] = {0};
+    HZ_CHECK(hipMemcpyAsync(tail, S.sptr + ns, sizeof(long long) * (drop_zeros ? 1 + kParts : 1),
+                            hipMemcpyDeviceToHost, st));
     HZ_CHECK(hipStreamSynchronize(st));
-    S.nent = nent;
-    S.col = arena().alloc_n<int>((size_t)nent + 1);
-    S.val = arena().alloc_n<double>((size_t)nent + 1);
+    S.nent = tail[0];
+    if (drop_zeros) {
+        S.nnz = 0;
+        for (int p = 0; p < kParts; p += kKeptStride) S.nnz += tail[1 + p];
+    }
+    S.col = arena().alloc_n<int>((size_t)S.nent + 1);
+    S.val = arena().alloc_n<double>((size_t)S.nent + 1);
     S.dl1 = arena().alloc_n<double>((size_t)A.n + 1);
     S.djac = arena().alloc_n<double>((size_t)A.n + 1);
     S.dfirst = arena().alloc_n<double>((size_t)A.n + 1);
     if (ns > 0) {
-        k_sell_fill<<<div_up(ns, kSlicesPerBlock), kBlock, 0, st>>>(A.n, A.ia, A.ja, A.val, S.sptr, S.col, S.val,
-                                                                  ns, S.dl1, S.djac, S.dfirst);
+        const int grid = div_up(ns, kSlicesPerBlock);
+        if (drop_zeros)
+            k_sell_fill<true><<<grid, kBlock, 0, st>>>(A.n, A.ia, A.ja, A.val, S.sptr, S.col, S.val, ns, S.dl1,
+                                                       S.djac, S.dfirst);
+        else
+            k_sell_fill<false><<<grid, kBlock, 0, st>>>(A.n, A.ia, A.ja, A.val, S.sptr, S.col, S.val, ns, S.dl1,
+                                                        S.djac, S.dfirst);
         HZ_LAUNCH_CHECK();
     }
 }
@@ -685,18 +740,21 @@ void spmv(const DevSELL &S, const double *x, double *y, double *dot_out, const R
     const int grid = div_up(S.nslices, kSlicesPerBlock);
     if (dot_out) {
         if (timer) timer->begin();
-        // the PCG's SpMV: rounds of 16, the second half of each with ordinary
+        // the PCG's SpMV: masked rounds, the second half of each with ordinary
         // loads that stay in the last-level cache for the cycle's residual
         // (ahead of an FP32 cycle: every column index, no value)
-        if (paired)
-            k_spmv<true, true, 1, unsigned int><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.pcol,
-                                                                                  S.val, x, y, ws.partials);
-        else if (cols_only)
-            k_spmv<true, true, 4><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, x, y,
-                                                                    ws.partials);
-        else
-            k_spmv<true, true, 1><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, x, y,
-                                                                    ws.partials);
+        by_round(S, [&](auto u) {
+            constexpr int U = decltype(u)::value;
+            if (paired)
+                k_spmv<true, U, 1, unsigned int><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.pcol, S.val,
+                                                                                 x, y, ws.partials);
+            else if (cols_only)
+                k_spmv<true, U, 4><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, x, y,
+                                                                   ws.partials);
+            else
+                k_spmv<true, U, 1><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, x, y,
+                                                                   ws.partials);
+        });
         if (timer) timer->end();
         HZ_LAUNCH_CHECK();
         k_final_sum<<<1, kFinBlock, 0, stream()>>>(ws.partials, grid, dot_out);
@@ -710,57 +768,54 @@ void spmv(const DevSELL &S, const double *x, double *y, double *dot_out, const R
 void residual(const DevSELL &S, const double *b, const double *x, double *w, LaunchTimer *timer) {
     if (S.n == 0) return;
     count_bytes(sell_bytes(S, S.pcol) + 24.0 * S.n);
-    // rounds of 16 masked loads: a 15-entry row in one round of loads
     if (timer) timer->begin();
     const int g = div_up(S.nslices, kSlicesPerBlock);
     // a matrix that fits the 256 MB last-level cache with room to spare is
     // loaded with ordinary loads: the same level's post-sweep, after the
     // coarser levels' work, still finds part of it there
     const bool resident = matrix_bytes(S.nnz, S.n) <= kCacheResidentBytes;
-    if (S.pcol && resident)
-        k_residual<true, 2, unsigned int><<<g, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.pcol, S.val, b, x, w);
-    else if (S.pcol)
-        k_residual<true, 0, unsigned int><<<g, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.pcol, S.val, b, x, w);
-    else if (resident)
-        k_residual<true, 2><<<g, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, b, x, w);
-    else
-        k_residual<true><<<g, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, b, x, w);
+    by_round(S, [&](auto u) {
+        constexpr int U = decltype(u)::value;
+        if (S.pcol && resident)
+            k_residual<U, 2, unsigned int><<<g, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.pcol, S.val, b, x, w);
+        else if (S.pcol)
+            k_residual<U, 0, unsigned int><<<g, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.pcol, S.val, b, x, w);
+        else if (resident)
+            k_residual<U, 2><<<g, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, b, x, w);
+        else
+            k_residual<U><<<g, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, b, x, w);
+    });
     if (timer) timer->end();
     HZ_LAUNCH_CHECK();
 }
 
 namespace {
+template <int kSm, bool kProlong, bool kDot>
+void launch_sweep_sm(const DevSELL &S, double w, const int *agg, const double *xc, double alpha,
+                     const double *alpha_dev, const double *b, const double *x, double *xout, double *partials) {
+    const int grid = div_up(S.nslices, kSlicesPerBlock);
+    const bool paired = !kProlong && S.pcol;
+    by_round(S, [&](auto u) {
+        constexpr int U = decltype(u)::value;
+        if (paired)
+            k_sweep<kSm, kProlong, kDot, U, unsigned int><<<grid, kBlock, 0, stream()>>>(
+                S.n, S.nslices, S.sptr, S.pcol, S.val, w, agg, xc, alpha, alpha_dev, b, x, xout, partials);
+        else
+            k_sweep<kSm, kProlong, kDot, U><<<grid, kBlock, 0, stream()>>>(
+                S.n, S.nslices, S.sptr, S.col, S.val, w, agg, xc, alpha, alpha_dev, b, x, xout, partials);
+    });
+    HZ_LAUNCH_CHECK();
+}
+
 template <bool kProlong, bool kDot>
 void launch_sweep(const DevSELL &S, int smoother, double w, const int *agg, const double *xc,
                   double alpha, const double *alpha_dev, const double *b, const double *x, double *xout,
                   double *partials) {
-    const int grid = div_up(S.nslices, kSlicesPerBlock);
-    const bool wide = !kProlong;   // rounds of 16 masked loads (the prolongation form has them anyway)
-    const bool paired = wide && S.pcol;
-    count_bytes(sell_bytes(S, paired) + 24.0 * S.n + (kProlong ? 4.0 * S.n : 0.0));
-    if (paired) {
-        if (smoother == HZ_SMOOTHER_L1DIAG)
-            k_sweep<HZ_SMOOTHER_L1DIAG, kProlong, kDot, true, unsigned int><<<grid, kBlock, 0, stream()>>>(
-                S.n, S.nslices, S.sptr, S.pcol, S.val, w, agg, xc, alpha, alpha_dev, b, x, xout, partials);
-        else
-            k_sweep<HZ_SMOOTHER_JACOBI, kProlong, kDot, true, unsigned int><<<grid, kBlock, 0, stream()>>>(
-                S.n, S.nslices, S.sptr, S.pcol, S.val, w, agg, xc, alpha, alpha_dev, b, x, xout, partials);
-    } else if (smoother == HZ_SMOOTHER_L1DIAG) {
-        if (wide)
-            k_sweep<HZ_SMOOTHER_L1DIAG, kProlong, kDot, true><<<grid, kBlock, 0, stream()>>>(
-                S.n, S.nslices, S.sptr, S.col, S.val, w, agg, xc, alpha, alpha_dev, b, x, xout, partials);
-        else
-            k_sweep<HZ_SMOOTHER_L1DIAG, kProlong, kDot><<<grid, kBlock, 0, stream()>>>(
-                S.n, S.nslices, S.sptr, S.col, S.val, w, agg, xc, alpha, alpha_dev, b, x, xout, partials);
-    } else {
-        if (wide)
-            k_sweep<HZ_SMOOTHER_JACOBI, kProlong, kDot, true><<<grid, kBlock, 0, stream()>>>(
-                S.n, S.nslices, S.sptr, S.col, S.val, w, agg, xc, alpha, alpha_dev, b, x, xout, partials);
-        else
-            k_sweep<HZ_SMOOTHER_JACOBI, kProlong, kDot><<<grid, kBlock, 0, stream()>>>(
-                S.n, S.nslices, S.sptr, S.col, S.val, w, agg, xc, alpha, alpha_dev, b, x, xout, partials);
-    }
-    HZ_LAUNCH_CHECK();
+    count_bytes(sell_bytes(S, !kProlong && S.pcol) + 24.0 * S.n + (kProlong ? 4.0 * S.n : 0.0));
+    if (smoother == HZ_SMOOTHER_L1DIAG)
+        launch_sweep_sm<HZ_SMOOTHER_L1DIAG, kProlong, kDot>(S, w, agg, xc, alpha, alpha_dev, b, x, xout, partials);
+    else
+        launch_sweep_sm<HZ_SMOOTHER_JACOBI, kProlong, kDot>(S, w, agg, xc, alpha, alpha_dev, b, x, xout, partials);
 }
 }  // namespace
 
