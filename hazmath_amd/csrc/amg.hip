@@ -895,31 +895,47 @@ static void itinfo(int prt, int stop, int iter, double rel, double absr, double 
 }
 
 namespace {
-PcgScalars *pinned_scalars() {
-    static PcgScalars *h = nullptr;
-    if (!h) HZ_CHECK(hipHostMalloc((void **)&h, sizeof(PcgScalars), hipHostMallocDefault));
+PcgMail *pinned_mail() {
+    static PcgMail *h = nullptr;
+    if (!h) {
+        HZ_CHECK(hipHostMalloc((void **)&h, sizeof(PcgMail), hipHostMallocDefault));
+        h->ticket = 0;
+    }
     return h;
 }
 
-hipEvent_t fetch_event() {
-    static hipEvent_t e = nullptr;
-    if (!e) HZ_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    return e;
+PcgMail *mail_on_device() {
+    static PcgMail *d = nullptr;
+    if (!d) HZ_CHECK(hipHostGetDevicePointer((void **)&d, pinned_mail(), 0));
+    return d;
 }
 
-// Queue a copy of the device scalars into pinned memory (non-blocking).
-void fetch_async(const Hierarchy &H) {
-    HZ_CHECK(hipMemcpyAsync(pinned_scalars(), H.sc, sizeof(PcgScalars), hipMemcpyDeviceToHost, stream()));
-    HZ_CHECK(hipEventRecord(fetch_event(), stream()));
+// Tickets only grow, so a letter of an earlier solve is never taken for this one.
+unsigned long long next_ticket() {
+    static unsigned long long t = 0;
+    return ++t;
 }
 
-void fetch_wait(PcgScalars &out) {
-    HZ_CHECK(hipEventSynchronize(fetch_event()));
-    out = *pinned_scalars();
+// Waits until the device has left the scalars under `ticket` (fields that
+// k_final_update writes).  A stream that ends or fails without it is an error.
+void mail_wait(unsigned long long ticket, PcgScalars &out) {
+    PcgMail *m = pinned_mail();
+    auto arrived = [&] { return __atomic_load_n(&m->ticket, __ATOMIC_ACQUIRE) == ticket; };
+    for (unsigned spin = 1; !arrived(); ++spin) {
+        if (spin % 4096 != 0) continue;
+        const hipError_t e = hipStreamQuery(stream());
+        if (e == hipErrorNotReady) {
+            (void)hipGetLastError();   // not an error of a later call
+            continue;
+        }
+        HZ_CHECK(e);
+        if (!arrived()) HZ_CHECK(hipErrorUnknown);
+    }
+    out = m->s;
 }
 
 void fetch(const Hierarchy &H, PcgScalars &out) {
-    PcgScalars *h = pinned_scalars();
+    PcgScalars *h = &pinned_mail()->s;
     HZ_CHECK(hipMemcpyAsync(h, H.sc, sizeof(PcgScalars), hipMemcpyDeviceToHost, stream()));
     HZ_CHECK(hipStreamSynchronize(stream()));
     out = *h;
@@ -950,6 +966,13 @@ PcgResult pcg_solve(Hierarchy &H, const DevSELL &A, const double *b, double *u, 
     auto precond_zr = [&](const double *rr_, double *zz_, bool first_done = false) {
         if (!amg_precond(H, rr_, zz_, sc_zr, first_done)) dot(m, zz_, rr_, sc_zr, H.ws);
     };
+    // partials of (A p, p) and (z, r) that the next vector kernel sums itself
+    const size_t maxgrid = (size_t)std::max(8192, div_up(A.nslices, 4) + 1);
+    int n_ap = 0, n_zr = 0;
+    ReduceWs ws_ap = H.ws;
+    ws_ap.dot_part = arena().alloc_n<double>(maxgrid);
+    ws_ap.npart = &n_ap;
+    double *zr_part = arena().alloc_n<double>(maxgrid);
     // the PCG update forms the preconditioner's first level-0 sweep when the
     // preconditioner is queued right behind it
     FirstSweep first;
@@ -1008,14 +1031,18 @@ PcgResult pcg_solve(Hierarchy &H, const DevSELL &A, const double *b, double *u, 
     // before the host has read that iteration's scalars (they do not touch u or
     // r); the rare restart / convergence paths below redo or drop that work.
     while (iter++ < MaxIt) {
-        spmv(A, p, t, &H.sc->temp2, H.ws, H.spmv_timer, H.cp.precision > 0 && H.nl > 1 && !A.pcol);
-        pcg_update(m, H.sc, p, t, u, r, alpha_hist, iter, H.ws, fuse_first ? &first : nullptr);
-        fetch_async(H);
+        spmv(A, p, t, &H.sc->temp2, ws_ap, H.spmv_timer, H.cp.precision > 0 && H.nl > 1 && !A.pcol);
+        const unsigned long long ticket = next_ticket();
+        pcg_update(m, H.sc, ws_ap.dot_part, n_ap, p, t, u, r, alpha_hist, iter, H.ws, mail_on_device(), ticket,
+                   fuse_first ? &first : nullptr);
         if (speculate) {
+            H.ws.dot_part = zr_part;
+            H.ws.npart = &n_zr;
             precond_zr(r, z, fuse_first);
-            pcg_direction(m, H.sc, z, p, beta_hist, iter);
+            H.ws.npart = nullptr;
+            pcg_direction(m, H.sc, zr_part, n_zr, z, p, beta_hist, iter);
         }
-        fetch_wait(hs);
+        mail_wait(ticket, hs);
         const double alpha = hs.alpha;
         bool redo = false;
         if (stop == HZ_STOP_REL_PRECRES) {
@@ -1088,11 +1115,11 @@ PcgResult pcg_solve(Hierarchy &H, const DevSELL &A, const double *b, double *u, 
         absres0 = absres;
         if (!speculate) {
             dot(m, z, r, sc_zr, H.ws);
-            pcg_direction(m, H.sc, z, p, beta_hist, iter);
+            pcg_direction(m, H.sc, nullptr, 0, z, p, beta_hist, iter);
         } else if (redo) {
             // r was recomputed (and p reset): redo z = B(r), (z, r) and p
             precond_zr(r, z);
-            pcg_direction(m, H.sc, z, p, beta_hist, iter);
+            pcg_direction(m, H.sc, nullptr, 0, z, p, beta_hist, iter);
         }
     }
     {

@@ -132,19 +132,26 @@ __device__ __forceinline__ double block_max(double v, double *sh) {
 }
 
 // Sum of partials[0..n) by one block in a fixed order (strided per thread,
-// then the block tree).
+// then the block tree).  A thread's loads are issued eight at a time: the sum
+// of 8,002 partials waits for memory once instead of eight times.
 template <int BLOCK>
-__device__ __forceinline__ double final_sum(const double *partials, int n, double *sh) {
+__device__ __forceinline__ double strided_sum(const double *partials, int n) {
+    constexpr int U = 8;
     double v = 0.0;
-    for (int i = threadIdx.x; i < n; i += BLOCK) v += partials[i];
-    return block_sum<BLOCK>(v, sh);
+    for (int i0 = threadIdx.x; i0 < n; i0 += U * BLOCK) {
+        double a[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) a[u] = i0 + u * BLOCK < n ? partials[i0 + u * BLOCK] : 0.0;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (i0 + u * BLOCK < n) v += a[u];
+    }
+    return v;
 }
 
 template <int BLOCK>
-__device__ __forceinline__ double final_max(const double *partials, int n, double *sh) {
-    double v = 0.0;
-    for (int i = threadIdx.x; i < n; i += BLOCK) v = fmax(v, partials[i]);
-    return block_max<BLOCK>(v, sh);
+__device__ __forceinline__ double final_sum(const double *partials, int n, double *sh) {
+    return block_sum<BLOCK>(strided_sum<BLOCK>(partials, n), sh);
 }
 
 // Matrix entries are streamed once per launch: loading them non-temporally

@@ -67,11 +67,30 @@ inline void count_bytes(double b) { g_alg_bytes += b; }
 // columns of nnz entries, int32 row pointers of n rows
 inline double matrix_bytes(long long nnz, long n, int vb = 8) { return (double)nnz * (vb + 4) + 4.0 * (n + 1); }
 
+// At most this many partials of a scalar are summed by every block of the
+// kernel that needs it (one load a thread) instead of by a launch between: on
+// levels of up to 65,536 rows, where that launch costs more than the sum (at
+// 16,129 rows 2.3 us and its gap, twice an iteration of 104 us).
+constexpr int kSelfSum = 256;
+
 struct ReduceWs {
     double *partials = nullptr;   // kMaxBlocks * kSlots
     unsigned int *tickets = nullptr;
+    // when npart is set, a dot's partials go to dot_part (room for the
+    // largest grid) and stay there if they are few enough: *npart is their count, or 0 when the
+    // total was formed as usual
+    double *dot_part = nullptr;
+    int *npart = nullptr;
+    double *dots() const { return npart ? dot_part : partials; }
     static constexpr int kMaxBlocks = 8192;
     static constexpr int kSlots = 4;
+};
+
+// The PCG's scalars as the device leaves them for the host in pinned memory;
+// the ticket is written last.
+struct PcgMail {
+    PcgScalars s;
+    unsigned long long ticket;
 };
 
 // HIP events around the launches of one kernel inside a solve (the stream is
@@ -110,6 +129,9 @@ struct LaunchTimer {
 // drop_zeros: stored off-diagonal zeros are left out (a product with one adds
 // nothing to a row's sum, so every finite result is the same).
 void sell_from_csr(const DevCSR &A, DevSELL &S, bool drop_zeros = false);
+// The total of a dot's partials (grid of them in ws.dots()) to *out, or left as
+// they are (ReduceWs::npart).
+void finish_dot(const ReduceWs &ws, int grid, double *out);
 // y = A x ; if dot_out: *dot_out = sum_i y_i * x_i (deterministic).  timer:
 // events around the SpMV kernel itself (not the partials' finalize).
 // cols_only: the PCG's SpMV ahead of an FP32 cycle, which shares only the
@@ -157,12 +179,17 @@ struct FirstSweep {
     const double *d = nullptr;
     double *x0 = nullptr;
 };
-void pcg_update(int n, PcgScalars *s, const double *p, const double *t, double *u, double *r,
-                double *alpha_hist, int iter, const ReduceWs &ws, const FirstSweep *first = nullptr);
+// (npart > 0: (A p, p) as that many partials; mail: the scalars also go there,
+// under `ticket`)
+void pcg_update(int n, PcgScalars *s, const double *dot_part, int npart, const double *p, const double *t, double *u,
+                double *r, double *alpha_hist, int iter, const ReduceWs &ws, PcgMail *mail, unsigned long long ticket,
+                const FirstSweep *first = nullptr);
 void dot(int n, const double *x, const double *y, double *out, const ReduceWs &ws);
 void norm2sq(int n, const double *x, double *out, const ReduceWs &ws);
 // beta = zr/temp1; temp1 = zr; p = z + beta p ; beta_hist[iter-1] = beta
-void pcg_direction(int n, PcgScalars *s, const double *z, double *p, double *beta_hist, int iter);
+// (npart > 0: (z, r) as that many partials)
+void pcg_direction(int n, PcgScalars *s, const double *dot_part, int npart, const double *z, double *p,
+                   double *beta_hist, int iter);
 // coarse scaling alpha = min((x,b)/(x^T A x), 2)
 void coarse_scaling_alpha(const DevSELL &S, const double *x, const double *b, PcgScalars *s,
                           double *alpha_out, const ReduceWs &ws);

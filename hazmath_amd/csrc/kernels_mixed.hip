@@ -20,7 +20,6 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kSlicesPerBlock = kBlock / kWave;
-constexpr int kFinBlock = 1024;
 constexpr int kStreamGrid = 2048;
 constexpr float kSmallRealF = 1e-20f;
 
@@ -530,13 +529,6 @@ __global__ __launch_bounds__(256) void k_gemv_m(int n, const double *__restrict_
     if (lane == 0) x[row] = (float)s;
 }
 
-__global__ __launch_bounds__(kFinBlock) void k_final_sum_m(const double *__restrict__ partials, int G,
-                                                           double *__restrict__ out) {
-    __shared__ double sh[kFinBlock / kWave];
-    const double t = final_sum<kFinBlock>(partials, G, sh);
-    if (threadIdx.x == 0) *out = t;
-}
-
 template <int kSm, bool kPro, bool kOut, class MT>
 void launch_sweep_m(const DevSELL &S, const MT *val, float w, const int *agg, const float *xc, const float *b,
                     const float *x, float *xout, double *out64, const double *r64, double *partials) {
@@ -665,7 +657,7 @@ void sweep_m(const DevSELL &S, const LowMatrix &M, int smoother, float w, const 
     if (S.n == 0) return;
     count_bytes(matrix_bytes(S.nnz, S.n, M.kind == kLowF32 ? 4 : 2) + 12.0 * S.n + (agg ? 4.0 * S.n : 0.0) +
                 (out64 ? 12.0 * S.n : 0.0));
-    double *partials = out64 ? ws.partials : nullptr;
+    double *partials = out64 ? ws.dots() : nullptr;
     if (M.kind == kLowF32) {
         const float *v = static_cast<const float *>(M.sell);
         if (smoother == HZ_SMOOTHER_L1DIAG)
@@ -679,10 +671,7 @@ void sweep_m(const DevSELL &S, const LowMatrix &M, int smoother, float w, const 
         else
             dispatch_sweep_m<HZ_SMOOTHER_JACOBI>(S, v, w, agg, xc, b, x, xout, out64, r64, partials);
     }
-    if (out64 && dot_out) {
-        k_final_sum_m<<<1, kFinBlock, 0, stream()>>>(ws.partials, div_up(S.nslices, kSlicesPerBlock), dot_out);
-        HZ_LAUNCH_CHECK();
-    }
+    if (out64 && dot_out) finish_dot(ws, div_up(S.nslices, kSlicesPerBlock), dot_out);
 }
 
 void residual_m(const DevSELL &S, const LowMatrix &M, const float *b, const float *x, float *w, const DevCSR *A) {
@@ -786,32 +775,26 @@ void cheby_apply_m(const DevSELL &S, const DevCSR &A, const LowMatrix &M, const 
             if (M.kind == kLowF32)
                 k_cheb_step_m<true, float, unsigned int><<<grid, kBlock, 0, stream()>>>(
                     S.n, S.nslices, S.sptr, dcol, static_cast<const float *>(M.sell), diag, (float)c1, (float)c2, b,
-                    x, nullptr, dwork, out64, r64, ws.partials);
+                    x, nullptr, dwork, out64, r64, ws.dots());
             else
                 k_cheb_step_m<true, unsigned short, unsigned int><<<grid, kBlock, 0, stream()>>>(
                     S.n, S.nslices, S.sptr, dcol, static_cast<const unsigned short *>(M.sell), diag, (float)c1,
-                    (float)c2, b, x, nullptr, dwork, out64, r64, ws.partials);
+                    (float)c2, b, x, nullptr, dwork, out64, r64, ws.dots());
             HZ_LAUNCH_CHECK();
-            if (dot_out) {
-                k_final_sum_m<<<1, kFinBlock, 0, stream()>>>(ws.partials, grid, dot_out);
-                HZ_LAUNCH_CHECK();
-            }
+            if (dot_out) finish_dot(ws, grid, dot_out);
             return;
         }
         if (last64) {
             if (M.kind == kLowF32)
                 k_cheb_step_m<true, float><<<grid, kBlock, 0, stream()>>>(
                     S.n, S.nslices, S.sptr, S.col, static_cast<const float *>(M.sell), diag, (float)c1, (float)c2, b,
-                    x, nullptr, dwork, out64, r64, ws.partials);
+                    x, nullptr, dwork, out64, r64, ws.dots());
             else
                 k_cheb_step_m<true, unsigned short><<<grid, kBlock, 0, stream()>>>(
                     S.n, S.nslices, S.sptr, S.col, static_cast<const unsigned short *>(M.sell), diag, (float)c1,
-                    (float)c2, b, x, nullptr, dwork, out64, r64, ws.partials);
+                    (float)c2, b, x, nullptr, dwork, out64, r64, ws.dots());
             HZ_LAUNCH_CHECK();
-            if (dot_out) {
-                k_final_sum_m<<<1, kFinBlock, 0, stream()>>>(ws.partials, grid, dot_out);
-                HZ_LAUNCH_CHECK();
-            }
+            if (dot_out) finish_dot(ws, grid, dot_out);
             return;
         }
         if (grp) {

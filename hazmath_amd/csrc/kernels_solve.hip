@@ -510,6 +510,43 @@ __global__ void k_copy(double *__restrict__ d, const double *__restrict__ s, lon
         d[i] = s[i];
 }
 
+static_assert(kSelfSum == kBlock, "one load a thread");
+
+// The partials' total in every thread, in k_final_sum's order for n <= kSelfSum.
+__device__ __forceinline__ double self_sum(const double *part, int n, double *sh) {
+    double v = (int)threadIdx.x < n ? 0.0 + part[threadIdx.x] : 0.0;
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+    if (threadIdx.x % kWave == 0) sh[threadIdx.x / kWave] = v;
+    __syncthreads();
+    double r = 0.0;
+#pragma unroll
+    for (int i = 0; i < kBlock / kWave; ++i) r += sh[i];
+    __syncthreads();
+    return r;
+}
+
+// Three sums and a maximum (the second) down to one value a wave in sh[q][wave],
+// with one barrier for all four.
+template <int BLOCK>
+__device__ __forceinline__ void block_sums4(double a, double b, double c, double d, double (*sh)[BLOCK / kWave]) {
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) {
+        a += __shfl_xor(a, off, kWave);
+        b = fmax(b, __shfl_xor(b, off, kWave));
+        c += __shfl_xor(c, off, kWave);
+        d += __shfl_xor(d, off, kWave);
+    }
+    if (threadIdx.x % kWave == 0) {
+        const int w = threadIdx.x / kWave;
+        sh[0][w] = a;
+        sh[1][w] = b;
+        sh[2][w] = c;
+        sh[3][w] = d;
+    }
+    __syncthreads();
+}
+
 // u += alpha p ; r -= alpha t ; then per-block partials of ||r||^2, ||u||_inf,
 // ||u||^2, ||p||^2 (finalized by k_final_update).  alpha = zr / temp2.
 // kFirst: also x0 = the preconditioner's first level-0 sweep from zero on the
@@ -517,8 +554,11 @@ __global__ void k_copy(double *__restrict__ d, const double *__restrict__ s, lon
 // with non-temporal loads, as in k_pcg_direction and k_prolong (a 1 GiB
 // stream reads at 6.6-6.8 TB/s that way against 4.4-4.8 TB/s with ordinary
 // loads).
+// npart > 0: (A p, p) comes as that many partials (at most kSelfSum), summed by
+// every block in k_final_sum's order; block 0 leaves it in temp2.
 template <bool kFirst>
-__global__ __launch_bounds__(kBlock) void k_pcg_update(int n, const PcgScalars *__restrict__ s,
+__global__ __launch_bounds__(kBlock) void k_pcg_update(int n, PcgScalars *__restrict__ s,
+                                                       const double *__restrict__ dot_part, int npart,
                                                        const double *__restrict__ p,
                                                        const double *__restrict__ t,
                                                        double *__restrict__ u,
@@ -526,8 +566,11 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(int n, const PcgScalars *
                                                        double *__restrict__ partials, int smoother,
                                                        double wgt, const double *__restrict__ d,
                                                        double *__restrict__ x0) {
-    __shared__ double sh[kBlock / kWave];
-    const double alpha = s->zr / s->temp2;
+    __shared__ double sh[4][kBlock / kWave];
+    const double zr = s->zr;
+    const double temp2 = npart > 0 ? self_sum(dot_part, npart, sh[0]) : s->temp2;
+    const double alpha = zr / temp2;
+    if (npart > 0 && blockIdx.x == 0 && threadIdx.x == 0) s->temp2 = temp2;
     const double malpha = -alpha;
     double rr = 0.0, ui = 0.0, uu = 0.0, pp = 0.0;
     for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
@@ -549,16 +592,14 @@ __global__ __launch_bounds__(kBlock) void k_pcg_update(int n, const PcgScalars *
         uu += ui_ * ui_;
         pp += pi * pi;
     }
-    const int G = gridDim.x;
-    double v;
-    v = block_sum<kBlock>(rr, sh);
-    if (threadIdx.x == 0) partials[0 * G + blockIdx.x] = v;
-    v = block_max<kBlock>(ui, sh);
-    if (threadIdx.x == 0) partials[1 * G + blockIdx.x] = v;
-    v = block_sum<kBlock>(uu, sh);
-    if (threadIdx.x == 0) partials[2 * G + blockIdx.x] = v;
-    v = block_sum<kBlock>(pp, sh);
-    if (threadIdx.x == 0) partials[3 * G + blockIdx.x] = v;
+    block_sums4<kBlock>(rr, ui, uu, pp, sh);
+    if (threadIdx.x < 4) {
+        double v = 0.0;
+#pragma unroll
+        for (int i = 0; i < kBlock / kWave; ++i)
+            v = threadIdx.x == 1 ? fmax(v, sh[1][i]) : v + sh[threadIdx.x][i];
+        partials[threadIdx.x * gridDim.x + blockIdx.x] = v;
+    }
 }
 
 constexpr int kFinBlock = 1024;
@@ -572,23 +613,53 @@ __global__ __launch_bounds__(kFinBlock) void k_final_sum(const double *__restric
     if (threadIdx.x == 0) *out = t;
 }
 
+// The totals of k_pcg_update's norms.  mail: the host's copy of the scalars in
+// pinned memory, followed by a ticket the host waits for, so an iteration
+// needs neither a copy nor an event on the stream (those and the gap behind
+// them took 10 of the 430 us of a 128^3 iteration).
 __global__ __launch_bounds__(kFinBlock) void k_final_update(PcgScalars *__restrict__ s,
                                                             const double *__restrict__ partials, int G,
-                                                            double *__restrict__ alpha_hist, int iter) {
-    __shared__ double sh[kFinBlock / kWave];
-    const double a0 = final_sum<kFinBlock>(partials + 0 * G, G, sh);
-    const double a1 = final_max<kFinBlock>(partials + 1 * G, G, sh);
-    const double a2 = final_sum<kFinBlock>(partials + 2 * G, G, sh);
-    const double a3 = final_sum<kFinBlock>(partials + 3 * G, G, sh);
-    if (threadIdx.x == 0) {
-        const double alpha = s->zr / s->temp2;
-        s->rr = a0;
-        s->uinf = a1;
-        s->uu = a2;
-        s->pp = a3;
-        s->alpha = alpha;
-        s->temp1 = s->zr;
-        if (alpha_hist) alpha_hist[iter - 1] = alpha;
+                                                            double *__restrict__ alpha_hist, int iter,
+                                                            PcgMail *mail, unsigned long long ticket) {
+    __shared__ double sh[4][kFinBlock / kWave];
+    constexpr int U = 2;   // the update's grid is at most 2048 blocks: a thread's loads in one round
+    static_assert(U * kFinBlock >= kStreamGrid, "one round");
+    double a[4][U];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int i = threadIdx.x + u * kFinBlock;
+            a[q][u] = i < G ? partials[q * G + i] : 0.0;
+        }
+    const double zr = s->zr, temp2 = s->temp2;
+    block_sums4<kFinBlock>(0.0 + a[0][0] + a[0][1], fmax(fmax(0.0, a[1][0]), a[1][1]), 0.0 + a[2][0] + a[2][1],
+                           0.0 + a[3][0] + a[3][1], sh);
+    if (threadIdx.x < kWave) {
+        double v = 0.0;
+        if (threadIdx.x < 4)
+            for (int i = 0; i < kFinBlock / kWave; ++i)
+                v = threadIdx.x == 1 ? fmax(v, sh[1][i]) : v + sh[threadIdx.x][i];
+        const double rr = __shfl(v, 0, kWave), uinf = __shfl(v, 1, kWave), uu = __shfl(v, 2, kWave),
+                     pp = __shfl(v, 3, kWave);
+        if (threadIdx.x == 0) {
+            const double alpha = zr / temp2;
+            s->rr = rr;
+            s->uinf = uinf;
+            s->uu = uu;
+            s->pp = pp;
+            s->alpha = alpha;
+            s->temp1 = zr;
+            if (alpha_hist) alpha_hist[iter - 1] = alpha;
+            if (mail) {
+                mail->s.rr = rr;
+                mail->s.uinf = uinf;
+                mail->s.uu = uu;
+                mail->s.pp = pp;
+                mail->s.alpha = alpha;
+                __hip_atomic_store(&mail->ticket, ticket, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        }
     }
 }
 
@@ -602,14 +673,21 @@ __global__ __launch_bounds__(kBlock) void k_dot(int n, const double *__restrict_
     if (threadIdx.x == 0) partials[blockIdx.x] = v;
 }
 
-// beta = zr / temp1 ; p = 1.0*z + beta*p (array_axpby, array.c:423-433)
-__global__ void k_pcg_direction(int n, PcgScalars *__restrict__ s, const double *__restrict__ z,
-                                double *__restrict__ p, double *__restrict__ beta_hist, int iter) {
-    const double beta = s->zr / s->temp1;
+// beta = zr / temp1 ; p = 1.0*z + beta*p (array_axpby, array.c:423-433).
+// npart > 0: (z, r) comes as partials, as (A p, p) does to k_pcg_update.
+__global__ __launch_bounds__(kBlock) void k_pcg_direction(int n, PcgScalars *__restrict__ s,
+                                                          const double *__restrict__ dot_part, int npart,
+                                                          const double *__restrict__ z, double *__restrict__ p,
+                                                          double *__restrict__ beta_hist, int iter) {
+    __shared__ double sh[kBlock / kWave];
+    const double temp1 = s->temp1;
+    const double zr = npart > 0 ? self_sum(dot_part, npart, sh) : s->zr;
+    const double beta = zr / temp1;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
         p[i] = 1.0 * ld_nt(z + i) + beta * ld_nt(p + i);
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         s->beta = beta;
+        if (npart > 0) s->zr = zr;
         if (beta_hist) beta_hist[iter - 1] = beta;
     }
 }
@@ -669,6 +747,13 @@ inline int stream_grid(long n) {
 
 double g_alg_bytes = 0.0;
 
+void finish_dot(const ReduceWs &ws, int grid, double *out) {
+    const bool left = ws.npart && grid <= kSelfSum;
+    if (ws.npart) *ws.npart = left ? grid : 0;
+    if (left) return;
+    k_final_sum<<<1, kFinBlock, 0, stream()>>>(ws.dots(), grid, out);
+    HZ_LAUNCH_CHECK();
+}
 
 void sell_from_csr(const DevCSR &A, DevSELL &S, bool drop_zeros) {
     S.n = A.n;
@@ -747,17 +832,17 @@ void spmv(const DevSELL &S, const double *x, double *y, double *dot_out, const R
             constexpr int U = decltype(u)::value;
             if (paired)
                 k_spmv<true, U, 1, unsigned int><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.pcol, S.val,
-                                                                                 x, y, ws.partials);
+                                                                                 x, y, ws.dots());
             else if (cols_only)
                 k_spmv<true, U, 4><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, x, y,
-                                                                   ws.partials);
+                                                                   ws.dots());
             else
                 k_spmv<true, U, 1><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, x, y,
-                                                                   ws.partials);
+                                                                   ws.dots());
         });
         if (timer) timer->end();
         HZ_LAUNCH_CHECK();
-        k_final_sum<<<1, kFinBlock, 0, stream()>>>(ws.partials, grid, dot_out);
+        finish_dot(ws, grid, dot_out);
     } else {
         k_spmv<false><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, x, y,
                                                      nullptr);
@@ -829,10 +914,9 @@ void smooth_sweep_dot(const DevSELL &S, int smoother, double w, const double *b,
                       double *xout, double *dot_out, const ReduceWs &ws, LaunchTimer *timer) {
     if (S.n == 0) return;
     if (timer) timer->begin();
-    launch_sweep<false, true>(S, smoother, w, nullptr, nullptr, 1.0, nullptr, b, x, xout, ws.partials);
+    launch_sweep<false, true>(S, smoother, w, nullptr, nullptr, 1.0, nullptr, b, x, xout, ws.dots());
     if (timer) timer->end();
-    k_final_sum<<<1, kFinBlock, 0, stream()>>>(ws.partials, div_up(S.nslices, kSlicesPerBlock), dot_out);
-    HZ_LAUNCH_CHECK();
+    finish_dot(ws, div_up(S.nslices, kSlicesPerBlock), dot_out);
 }
 
 void smoother_diag(const DevSELL &S, int smoother, double *d) {
@@ -883,9 +967,8 @@ void up_fused(const DevSELL &S, int smoother, double w, const int *agg, const do
               double *dot_out, const ReduceWs &ws) {
     if (S.n == 0) return;
     if (dot_out) {
-        launch_sweep<true, true>(S, smoother, w, agg, xc, alpha, alpha_dev, b, x, xout, ws.partials);
-        k_final_sum<<<1, kFinBlock, 0, stream()>>>(ws.partials, div_up(S.nslices, kSlicesPerBlock), dot_out);
-        HZ_LAUNCH_CHECK();
+        launch_sweep<true, true>(S, smoother, w, agg, xc, alpha, alpha_dev, b, x, xout, ws.dots());
+        finish_dot(ws, div_up(S.nslices, kSlicesPerBlock), dot_out);
     } else {
         launch_sweep<true, false>(S, smoother, w, agg, xc, alpha, alpha_dev, b, x, xout, nullptr);
     }
@@ -913,36 +996,38 @@ void copy(double *dst, const double *src, long n) {
     HZ_LAUNCH_CHECK();
 }
 
-void pcg_update(int n, PcgScalars *s, const double *p, const double *t, double *u, double *r,
-                double *alpha_hist, int iter, const ReduceWs &ws, const FirstSweep *first) {
+void pcg_update(int n, PcgScalars *s, const double *dot_part, int npart, const double *p, const double *t, double *u,
+                double *r, double *alpha_hist, int iter, const ReduceWs &ws, PcgMail *mail, unsigned long long ticket,
+                const FirstSweep *first) {
     const int G = stream_grid(n);
     if (first) {
         count_bytes(64.0 * n);
-        k_pcg_update<true><<<G, kBlock, 0, stream()>>>(n, s, p, t, u, r, ws.partials, first->smoother, first->w,
-                                                       first->d, first->x0);
+        k_pcg_update<true><<<G, kBlock, 0, stream()>>>(n, s, dot_part, npart, p, t, u, r, ws.partials,
+                                                       first->smoother, first->w, first->d, first->x0);
     } else {
         count_bytes(48.0 * n);
-        k_pcg_update<false><<<G, kBlock, 0, stream()>>>(n, s, p, t, u, r, ws.partials, 0, 1.0, nullptr, nullptr);
+        k_pcg_update<false><<<G, kBlock, 0, stream()>>>(n, s, dot_part, npart, p, t, u, r, ws.partials, 0, 1.0,
+                                                        nullptr, nullptr);
     }
     HZ_LAUNCH_CHECK();
-    k_final_update<<<1, kFinBlock, 0, stream()>>>(s, ws.partials, G, alpha_hist, iter);
+    k_final_update<<<1, kFinBlock, 0, stream()>>>(s, ws.partials, G, alpha_hist, iter, mail, ticket);
     HZ_LAUNCH_CHECK();
 }
 
 void dot(int n, const double *x, const double *y, double *out, const ReduceWs &ws) {
     const int G = stream_grid(n);
     count_bytes(x == y ? 8.0 * n : 16.0 * n);
-    k_dot<<<G, kBlock, 0, stream()>>>(n, x, y, ws.partials);
+    k_dot<<<G, kBlock, 0, stream()>>>(n, x, y, ws.dots());
     HZ_LAUNCH_CHECK();
-    k_final_sum<<<1, kFinBlock, 0, stream()>>>(ws.partials, G, out);
-    HZ_LAUNCH_CHECK();
+    finish_dot(ws, G, out);
 }
 
 void norm2sq(int n, const double *x, double *out, const ReduceWs &ws) { dot(n, x, x, out, ws); }
 
-void pcg_direction(int n, PcgScalars *s, const double *z, double *p, double *beta_hist, int iter) {
+void pcg_direction(int n, PcgScalars *s, const double *dot_part, int npart, const double *z, double *p,
+                   double *beta_hist, int iter) {
     count_bytes(24.0 * n);
-    k_pcg_direction<<<stream_grid(n), kBlock, 0, stream()>>>(n, s, z, p, beta_hist, iter);
+    k_pcg_direction<<<stream_grid(n), kBlock, 0, stream()>>>(n, s, dot_part, npart, z, p, beta_hist, iter);
     HZ_LAUNCH_CHECK();
 }
 
