@@ -342,6 +342,23 @@ int amg_setup(Hierarchy &H, const DevCSR &A0, AMG_param *param, bool) {
     return HZ_SUCCESS;
 }
 
+namespace {
+// Levels up to this many rows are latency-bound: they use the fused kernels
+// (HZ_FUSE_DOWN_MAX overrides the default).  PCG ms by limit, 128^3 Poisson /
+// 76^3 anisotropic (438,976 rows) / 128^3 FP32 cycle: 300,000 rows 13.76 /
+// 16.35 / 24.41; 600,000 13.76 / 18.09 / 24.37; every level 14.42 / 18.07 /
+// 24.79.  Above it a level's kernels are bandwidth-bound, and a finest level
+// shares its matrix with the PCG's product through the last-level cache.
+int fused_down_max_rows() {
+    static int v = -1;
+    if (v < 0) {
+        const char *e = std::getenv("HZ_FUSE_DOWN_MAX");
+        v = e ? std::atoi(e) : 300000;
+    }
+    return v;
+}
+}  // namespace
+
 void amg_prepare_cycle(Hierarchy &H, const AMG_param *param) {
     // precond_amg rebuilds its parameters from param_amg_init + param_prec_to_amg
     // (precond.c:173-174, parameters.c:649-675): tol is the default 1e-6.
@@ -413,6 +430,18 @@ void amg_prepare_cycle(Hierarchy &H, const AMG_param *param) {
             }
         }
     }
+    // latency-bound levels of a Jacobi / L1 cycle: the layout of kernels_fused.hip
+    if (cp.smoother == HZ_SMOOTHER_L1DIAG || cp.smoother == HZ_SMOOTHER_JACOBI) {
+        std::vector<Level *> small;
+        std::vector<int> kinds;
+        for (int l = 0; l < H.nl - 1; ++l) {
+            Level &L = H.lv[l];
+            if (L.sa || L.A.n > fused_down_max_rows()) continue;
+            small.push_back(&L);
+            kinds.push_back(cp.precision == 0 ? 0 : L.low.kind);
+        }
+        fused_prepare(small, kinds, cp.smoother);
+    }
     // the FP64 Jacobi / L1 cycle and the PCG's product read 16-bit column
     // offsets on levels of 65,536 rows or more where every offset fits: one
     // conversion a level, one wait for all of them
@@ -481,18 +510,6 @@ void presmooth(Hierarchy &H, int l, CycleState &cs) {
     }
 }
 
-// Levels up to this many rows are latency-bound: they use the fused
-// one-thread-per-coarse-row restriction and the prolongation folded into the
-// sweep (HZ_FUSE_DOWN_MAX overrides the default).
-int fused_down_max_rows() {
-    static int v = -1;
-    if (v < 0) {
-        const char *e = std::getenv("HZ_FUSE_DOWN_MAX");
-        v = e ? std::atoi(e) : 300000;
-    }
-    return v;
-}
-
 // Prolongation x_l += alpha P x_{l+1} followed by the post-smoothing sweeps;
 // the prolongation is folded into the first sweep.  dot_out: when non-null
 // and the fused sweep is the last one, it also yields sum_i x_i b_i.
@@ -516,6 +533,9 @@ void prolong_postsmooth(Hierarchy &H, int l, double alpha, const double *alpha_d
             smooth_sweep_dot(L.S, cp.smoother, cp.jacobi_w, L.b, L.x, L.xt, dot_out, H.ws);
         else
             smooth_sweep(L.S, cp.smoother, cp.jacobi_w, L.b, L.x, L.xt);
+    } else if (L.F.on) {
+        fused_up(L, cp.smoother, cp.jacobi_w, C.x, alpha, alpha_dev, L.b, L.x, L.xt, want_dot ? dot_out : nullptr,
+                 H.ws);
     } else if (L.A.n <= fused_down_max_rows()) {
         // latency-bound level: one kernel
         up_fused(L.S, cp.smoother, cp.jacobi_w, L.agg, C.x, alpha, alpha_dev, L.b, L.x, L.xt,
@@ -558,6 +578,8 @@ forward:
         if (L.sa) {
             residual(L.S, L.b, L.x, L.w);
             csr_mxv(L.R, L.w, C.b);    // dcsr_mxv(R), mgcycle.c:302
+        } else if (L.F.on) {
+            fused_down(L, L.b, L.x, C.b, cp.smoother, cp.jacobi_w, fuse ? C.dsm : nullptr, fuse ? C.x : nullptr);
         } else if (L.A.n <= fused_down_max_rows()) {
             down_fused(L.nagg, L.rptr, L.rmem, L.A, L.b, L.x, C.b, cp.smoother, cp.jacobi_w,
                        fuse ? C.dsm : nullptr, fuse ? C.x : nullptr);
@@ -667,6 +689,13 @@ bool prolong_postsmooth_m(Hierarchy &H, int l, bool final, double *z, const doub
         const bool last = final && s == cp.postsmooth - 1;
         const int *agg = nullptr;
         const float *xc = nullptr;
+        if (s == 0 && !L.sa && L.F.on) {
+            fused_up(L, cp.smoother, cp.jacobi_w, C.xf, L.bf, L.xf, L.xtf, last ? z : nullptr, r,
+                     last ? dot_out : nullptr, H.ws);
+            if (last) return true;
+            std::swap(L.xf, L.xtf);
+            continue;
+        }
         if (s == 0 && !L.sa) {
             if (L.A.n <= fused_down_max_rows()) {
                 agg = L.agg;
@@ -707,6 +736,9 @@ forward:
                 csr_mxv_m(L.R, L.Rf, L.wf, C.bf, C.cdiagf, cheb_first_c2(C.cheb), C.xf, C.cworkf);
             else
                 csr_mxv_m(L.R, L.Rf, L.wf, C.bf);
+        } else if (L.F.on) {
+            fused_down(L, L.bf, L.xf, C.bf, cp.smoother, cp.jacobi_w, fuse ? C.dsmf : nullptr,
+                       fuse ? C.xf : nullptr);
         } else if (L.A.n <= fused_down_max_rows()) {
             down_fused_m(L.nagg, L.rptr, L.rmem, L.A, L.low, L.bf, L.xf, C.bf, cp.smoother, w,
                          fuse ? C.dsmf : nullptr, fuse ? C.xf : nullptr);

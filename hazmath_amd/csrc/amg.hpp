@@ -7,6 +7,22 @@
 
 namespace hz {
 
+// A small level's matrix in the order of its restriction (kernels_fused.hip).
+struct FusedLevel {
+    bool on = false;
+    int kind = 0;             // values: 0 FP64, kLowF32, kLowBF16
+    int C = 0, K = 0;         // coarse rows and slices of a workgroup
+    int nblk = 0;             // workgroups
+    int wmax = 0, amax = 0;   // longest row of A and of A P
+    int *width = nullptr, *awidth = nullptr;   // per slice, or null: wmax / amax everywhere
+    int *prow = nullptr, *pagg = nullptr;      // per position: row (-1: none) and its aggregate
+    int *col = nullptr;       // A by position
+    void *val = nullptr;
+    int *acol = nullptr;      // A P by position
+    void *aval = nullptr;
+    void *wpos = nullptr;     // residual by position, from fused_down to fused_up
+};
+
 struct Level {
     DevCSR A;                 // CSR (setup input; coarsest: sorted transpose for coarse_solver 32)
     DevSELL S;                // SELL-64 copy used by every solve kernel
@@ -24,6 +40,7 @@ struct Level {
     GsLevel gs;               // colouring and colour-sliced matrix (GS family)
     double *Ainv = nullptr;   // coarsest, coarse_solver 32
     double *cgwork = nullptr; // coarsest, coarse_solver 0
+    FusedLevel F;             // latency-bound levels of a Jacobi / L1 cycle
     // FP32 cycle (CycleParams::precision > 0)
     LowMatrix low;            // values in FP32 or BF16 (non-coarsest levels)
     float *dsmf = nullptr;    // smoother diagonal rounded to FP32
@@ -86,6 +103,23 @@ bool amg_precond(Hierarchy &H, const double *r, double *z, double *zr_out, bool 
 // sweep (FP32 cycle, one level, Chebyshev or Gauss-Seidel-type smoothers, no
 // pre-smoothing).
 bool amg_precond_first_sweep(Hierarchy &H, double *z, FirstSweep &out);
+
+// ---- kernels_fused.hip ----
+// Builds F of the given levels (kinds: FusedLevel::kind); a level whose
+// aggregates or rows do not suit the layout keeps F.on == false.
+void fused_prepare(std::vector<Level *> &levels, const std::vector<int> &kinds, int smoother);
+// bc = R (b - A x), xc (optional) = the coarse level's first sweep from zero
+void fused_down(const Level &L, const double *b, const double *x, double *bc, int smoother, double w,
+                const double *dc, double *xc);
+void fused_down(const Level &L, const float *b, const float *x, float *bc, int smoother, double w, const float *dc,
+                float *xc);
+// xout = sweep(x + alpha P xc) after a fused_down on the same x and b, with
+// (xout, b) to dot_out; in the FP32 cycle
+// optionally to out64 in FP64 instead, with (out64, r64) to dot_out
+void fused_up(const Level &L, int smoother, double w, const double *xc, double alpha, const double *alpha_dev,
+              const double *b, const double *x, double *xout, double *dot_out, const ReduceWs &ws);
+void fused_up(const Level &L, int smoother, double w, const float *xc, const float *b, const float *x, float *xout,
+              double *out64, const double *r64, double *dot_out, const ReduceWs &ws);
 
 struct PcgResult {
     int iter = 0;

@@ -162,6 +162,13 @@ __device__ __forceinline__ T ld_nt(const T *p) {
     return __builtin_nontemporal_load(p);
 }
 
+// bf16 stored as the upper half of the FP32 bit pattern
+__device__ __forceinline__ unsigned short f2bf(float f) {
+    const unsigned int u = __float_as_uint(f);
+    const unsigned int r = u + 0x7FFFu + ((u >> 16) & 1u);   // round to nearest even
+    return (unsigned short)(r >> 16);
+}
+
 // 16-bit column offsets from the row, two entries of a row to a 32-bit word:
 // entry 2p of the row in the low half of word p, 2p+1 in the high half, words
 // of a SELL slice lane-major as its entries are, padding kColPad16.  Slice s's

@@ -21,7 +21,7 @@ struct DevSELL {
     long long nnz = 0;         // entries without the padding (algorithmic bytes count these)
     long long nent = 0;        // padded entries
     long long *sptr = nullptr; // nslices+1 offsets
-    int *len = nullptr;        // row lengths
+    int *len = nullptr;        // entries of each row
     int *col = nullptr;
     double *val = nullptr;
     double *dl1 = nullptr;     // row l1 norms (L1DIAG diagonal), formed by sell_from_csr

@@ -28,17 +28,10 @@ inline int grid_for(long n) {
     return (int)std::max(1L, std::min<long>(g, kStreamGrid));
 }
 
-// bf16 stored as the upper half of the FP32 bit pattern
 // matrix values are streamed once per launch: non-temporal loads
 __device__ __forceinline__ float ldv(const float *p) { return ld_nt(p); }
 __device__ __forceinline__ float ldv(const unsigned short *p) {
     return __uint_as_float(((unsigned int)ld_nt(p)) << 16);
-}
-
-__device__ __forceinline__ unsigned short f2bf(float f) {
-    const unsigned int u = __float_as_uint(f);
-    const unsigned int r = u + 0x7FFFu + ((u >> 16) & 1u);   // round to nearest even
-    return (unsigned short)(r >> 16);
 }
 
 __global__ void k_vals_f32(long long n, const double *__restrict__ v, float *__restrict__ o) {

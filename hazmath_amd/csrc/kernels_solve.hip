@@ -102,7 +102,8 @@ __global__ __launch_bounds__(kBlock) void k_sell_fill(int n, const int *__restri
                                                       const double *__restrict__ val,
                                                       const long long *__restrict__ sptr, int *__restrict__ scol,
                                                       double *__restrict__ sval, int nslices, double *__restrict__ dl1,
-                                                      double *__restrict__ djac, double *__restrict__ dfirst) {
+                                                      double *__restrict__ djac, double *__restrict__ dfirst,
+                                                      int *__restrict__ rowlen) {
     __shared__ int s_col[kSlicesPerBlock][kSellStage];
     __shared__ double s_val[kSlicesPerBlock][kSellStage];
     const int wv = threadIdx.x / kWave;
@@ -129,6 +130,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_fill(int n, const int *__restri
     int q = (r < n) ? ia[r] : 0;
     double l1 = 0.0, dj = 0.0, df = 0.0;
     bool seen = false;
+    int len = 0;
     for (int k = 0; k < w; ++k) {
         const long long e = base + (long long)k * kSlice + lane;
         int j = -1;
@@ -145,6 +147,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_fill(int n, const int *__restri
         scol[e] = j;
         sval[e] = a;
         if (j >= 0) {
+            ++len;
             l1 = l1 + fabs(a);
             if (j == r) {
                 dj = a;
@@ -157,6 +160,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_fill(int n, const int *__restri
         dl1[r] = l1;
         djac[r] = dj;
         dfirst[r] = df;
+        rowlen[r] = len;
     }
 }
 
@@ -797,14 +801,15 @@ void sell_from_csr(const DevCSR &A, DevSELL &S, bool drop_zeros) {
     S.dl1 = arena().alloc_n<double>((size_t)A.n + 1);
     S.djac = arena().alloc_n<double>((size_t)A.n + 1);
     S.dfirst = arena().alloc_n<double>((size_t)A.n + 1);
+    S.len = arena().alloc_n<int>((size_t)A.n + 1);
     if (ns > 0) {
         const int grid = div_up(ns, kSlicesPerBlock);
         if (drop_zeros)
             k_sell_fill<true><<<grid, kBlock, 0, st>>>(A.n, A.ia, A.ja, A.val, S.sptr, S.col, S.val, ns, S.dl1,
-                                                       S.djac, S.dfirst);
+                                                       S.djac, S.dfirst, S.len);
         else
             k_sell_fill<false><<<grid, kBlock, 0, st>>>(A.n, A.ia, A.ja, A.val, S.sptr, S.col, S.val, ns, S.dl1,
-                                                        S.djac, S.dfirst);
+                                                        S.djac, S.dfirst, S.len);
         HZ_LAUNCH_CHECK();
     }
 }

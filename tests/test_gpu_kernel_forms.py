@@ -51,3 +51,110 @@ def test_solve_with_stored_zeros(lib, orc, libc, m, per_row, smoother):
     # two iterates below 1e-10 of a system of condition below 2e3 (2-D Laplacian, h = 1/45)
     tol = 1e-10 if smoother == capi.SMOOTHER_L1DIAG else 2e-7
     assert np.linalg.norm(xg - xo) / np.linalg.norm(xo) < tol
+
+
+def _dirichlet_rows(m):
+    """2-D Laplacian with every 7th unknown turned into an identity row (rows outside every aggregate)."""
+    import scipy.sparse as sp
+    ia, ja, va = problems.poisson2d_p1(m)
+    n = ia.size - 1
+    M = sp.csr_matrix((va, ja, ia), shape=(n, n))
+    keep = np.arange(n) % 7 != 3
+    D = sp.diags(keep.astype(float))
+    M = (D @ M @ D + sp.diags(1.0 - keep)).tocsr()
+    M.eliminate_zeros()
+    M.sort_indices()
+    return M.indptr.astype(np.int32), M.indices.astype(np.int32), M.data
+
+
+def _long_row(m, entries):
+    """2-D Laplacian with `entries` weak couplings of row 0 added (symmetric, diagonally dominant)."""
+    import scipy.sparse as sp
+    ia, ja, va = problems.poisson2d_p1(m)
+    n = ia.size - 1
+    M = sp.csr_matrix((va, ja, ia), shape=(n, n)).tolil()
+    for k in range(1, entries + 1):
+        j = (k * 13) % (n - 1) + 1
+        M[0, j] -= 0.01
+        M[j, 0] -= 0.01
+        M[0, 0] += 0.01
+        M[j, j] += 0.01
+    M = M.tocsr()
+    M.sort_indices()
+    return M.indptr.astype(np.int32), M.indices.astype(np.int32), M.data
+
+
+def _two_diagonals(m):
+    """2-D Laplacian whose rows store their diagonal as two entries, 3 and 1."""
+    ia, ja, va = problems.poisson2d_p1(m)
+    n = ia.size - 1
+    row = np.repeat(np.arange(n), np.diff(ia))
+    va = va.copy()
+    va[ja == row] = 3.0
+    r, c, v = np.concatenate([row, np.arange(n)]), np.concatenate([ja, np.arange(n)]), np.concatenate([va, np.ones(n)])
+    order = np.argsort(r, kind="stable")
+    ia2 = np.concatenate([[0], np.cumsum(np.bincount(r, minlength=n))]).astype(np.int32)
+    return ia2, c[order].astype(np.int32), v[order]
+
+
+FUSED = {
+    "p2d_hec": (lambda: problems.poisson2d_p1(80), capi.HEC),         # aggregates of uneven size, last workgroup part full
+    "p2d_vmb": (lambda: problems.poisson2d_p1(61), capi.VMB),         # larger aggregates
+    "kuhn_hem": (lambda: problems.poisson3d_kuhn(22), capi.HEM),      # pairs, zeros left out
+    "aniso_hec": (lambda: problems.aniso3d_kuhn(24, 0.7, 0.05), capi.HEC),   # rows of over 16 entries below
+    "large_hem": (lambda: problems.aniso3d_kuhn(46, 0.7, 0.05), capi.HEM),   # 91,125 rows: widths by slice
+    "dirichlet": (lambda: _dirichlet_rows(50), capi.HEC),             # rows in no aggregate: the list-walking kernels
+    "row64": (lambda: _long_row(40, 59), capi.HEC),                   # the longest row that the merge takes
+    "two_diagonals": (lambda: _two_diagonals(40), capi.HEC),          # Jacobi: the list-walking kernels
+    "row200": (lambda: _long_row(40, 195), capi.HEC),                 # longer: the list-walking kernels
+}
+
+
+@pytest.mark.parametrize("case", list(FUSED))
+@pytest.mark.parametrize("smoother", [capi.SMOOTHER_L1DIAG, capi.SMOOTHER_JACOBI])
+def test_fused_cycle_kernels_vs_oracle(lib, orc, libc, case, smoother):
+    """One preconditioner application (both fused kernels on every level that takes them) against the oracle's cycle:
+    FP64 within 1e-12 relative (two summation orders of at most 200 terms over at most 10 levels, whose coarsest
+    solve amplifies by its condition number, below 1e3); the FP32 and BF16 cycles within their bounds of the FP64
+    one (2e-5: 10 levels of 2^-24 roundings; 5e-2: 2^-9 in the values)."""
+    import oracle
+    make, agg = FUSED[case]
+    ia, ja, va = make()
+    n = ia.size - 1
+    A = capi.HostCSR(ia, ja, va)
+    kw = dict(aggregation=agg, smoother=smoother, coarse_dof=60, theta=0.04)
+    opts = capi.hz_options()
+    lib.hz_get_options(C.byref(opts))
+    old = opts.vcycle_precision, opts.jacobi_weight
+    opts.jacobi_weight = w = 2.0 / 3.0 if smoother == capi.SMOOTHER_JACOBI else 1.0
+    orc.orc_set_jacobi_weight.argtypes = [C.c_double]
+    r = problems.uniform_rhs(n, seed=9)
+    z = {}
+    try:
+        orc.orc_set_jacobi_weight(w)
+        _, amgo = oracle.params(**kw)
+        libc.srand(1)
+        h = orc.orc_precond_create(A.ptr(), C.byref(amgo))
+        z["oracle"] = np.zeros(n)
+        orc.orc_precond_apply(h, capi.dptr(r), capi.dptr(z["oracle"]))
+        orc.orc_precond_free(h)
+        for precision in (0, 1, 2):
+            opts.vcycle_precision = precision
+            lib.hz_set_options(C.byref(opts))
+            _, amg = capi.solver_params(lib, **kw)
+            libc.srand(1)
+            pc = lib.create_precond_amg(A.ptr(), C.byref(amg))
+            assert pc
+            z[precision] = np.zeros(n)
+            lib.apply_precond(capi.dptr(r), capi.dptr(z[precision]), pc)
+            lib.hz_precond_free(pc)
+    finally:
+        orc.orc_set_jacobi_weight(1.0)
+        opts.vcycle_precision, opts.jacobi_weight = old
+        lib.hz_set_options(C.byref(opts))
+
+    def off(a, b):
+        return np.linalg.norm(z[a] - z[b]) / np.linalg.norm(z[b])
+    assert off(0, "oracle") < 1e-12
+    assert off(1, 0) < 2e-5
+    assert off(2, 0) < 5e-2
