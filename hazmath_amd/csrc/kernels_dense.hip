@@ -321,6 +321,7 @@ __global__ __launch_bounds__(256) void k_gemv(int n, const double *__restrict__ 
 // ---------------------------------------------------------------------------
 constexpr int kCgBlock = 1024;
 
+template <int kThreads>
 __device__ double cg_block_sum(double v, double *sh) {
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
@@ -330,10 +331,11 @@ __device__ double cg_block_sum(double v, double *sh) {
     __syncthreads();
     double r = 0.0;
 #pragma unroll
-    for (int i = 0; i < kCgBlock / kWave; ++i) r += sh[i];
+    for (int i = 0; i < kThreads / kWave; ++i) r += sh[i];
     return r;   // every thread gets the same value
 }
 
+template <int kThreads>
 __device__ double cg_block_max(double v, double *sh) {
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) v = fmax(v, __shfl_xor(v, off, kWave));
@@ -343,14 +345,15 @@ __device__ double cg_block_max(double v, double *sh) {
     __syncthreads();
     double r = 0.0;
 #pragma unroll
-    for (int i = 0; i < kCgBlock / kWave; ++i) r = fmax(r, sh[i]);
+    for (int i = 0; i < kThreads / kWave; ++i) r = fmax(r, sh[i]);
     return r;
 }
 
+template <int kThreads>
 __device__ void cg_matvec(int n, int nslices, const long long *sptr, const int *col, const double *val,
                           const double *x, double *y, double alpha_mode, const double *b) {
     // alpha_mode 0: y = A x ; 1: y = b - A x
-    for (int s = threadIdx.x / kWave; s < nslices; s += kCgBlock / kWave) {
+    for (int s = threadIdx.x / kWave; s < nslices; s += kThreads / kWave) {
         const int lane = threadIdx.x % kWave;
         const int r = s * kSlice + lane;
         const long long base = sptr[s];
@@ -373,25 +376,25 @@ __device__ int coarse_cg_body(int n, int nslices, const long long *__restrict__ 
     const int tid = threadIdx.x;
     const double maxdiff = tol * 1e-4;
     int iter = 0, stag = 1, more_step = 1;
-    cg_matvec(n, nslices, sptr, col, val, u, r, 1.0, b);
+    cg_matvec<kCgBlock>(n, nslices, sptr, col, val, u, r, 1.0, b);
     __syncthreads();
     double acc = 0.0;
     for (int i = tid; i < n; i += kCgBlock) acc += r[i] * r[i];
-    double absres0 = sqrt(cg_block_sum(acc, sh));
+    double absres0 = sqrt(cg_block_sum<kCgBlock>(acc, sh));
     const double normr0 = absres0 > kSmallReal ? absres0 : kSmallReal;
     double relres = absres0 / normr0, absres = absres0;
     if (relres < tol || absres0 < 1e-3 * tol) return 0;
     for (int i = tid; i < n; i += kCgBlock) p[i] = r[i];
     acc = 0.0;
     for (int i = tid; i < n; i += kCgBlock) acc += r[i] * r[i];
-    double temp1 = cg_block_sum(acc, sh);
+    double temp1 = cg_block_sum<kCgBlock>(acc, sh);
     while (iter++ < maxit) {
         __syncthreads();
-        cg_matvec(n, nslices, sptr, col, val, p, t, 0.0, nullptr);
+        cg_matvec<kCgBlock>(n, nslices, sptr, col, val, p, t, 0.0, nullptr);
         __syncthreads();
         acc = 0.0;
         for (int i = tid; i < n; i += kCgBlock) acc += t[i] * p[i];
-        const double temp2 = cg_block_sum(acc, sh);
+        const double temp2 = cg_block_sum<kCgBlock>(acc, sh);
         const double alpha = temp1 / temp2;
         double rr = 0.0, ui = 0.0, uu = 0.0, pp = 0.0;
         for (int i = tid; i < n; i += kCgBlock) {
@@ -404,19 +407,19 @@ __device__ int coarse_cg_body(int n, int nslices, const long long *__restrict__ 
             uu += ui_ * ui_;
             pp += p[i] * p[i];
         }
-        absres = sqrt(cg_block_sum(rr, sh));
+        absres = sqrt(cg_block_sum<kCgBlock>(rr, sh));
         relres = absres / normr0;
-        const double infnormu = cg_block_max(ui, sh);
+        const double infnormu = cg_block_max<kCgBlock>(ui, sh);
         if (infnormu <= kSmallReal) return HZ_ERROR_SOLVER_SOLSTAG;   // Check I
-        const double normu = sqrt(cg_block_sum(uu, sh));
-        const double reldiff = fabs(alpha) * sqrt(cg_block_sum(pp, sh)) / normu;
+        const double normu = sqrt(cg_block_sum<kCgBlock>(uu, sh));
+        const double reldiff = fabs(alpha) * sqrt(cg_block_sum<kCgBlock>(pp, sh)) / normu;
         if ((stag <= 20) & (reldiff < maxdiff)) {                  // Check II
             __syncthreads();
-            cg_matvec(n, nslices, sptr, col, val, u, r, 1.0, b);
+            cg_matvec<kCgBlock>(n, nslices, sptr, col, val, u, r, 1.0, b);
             __syncthreads();
             acc = 0.0;
             for (int i = tid; i < n; i += kCgBlock) acc += r[i] * r[i];
-            absres = sqrt(cg_block_sum(acc, sh));
+            absres = sqrt(cg_block_sum<kCgBlock>(acc, sh));
             relres = absres / normr0;
             if (relres < tol) return iter;
             if (stag >= 20) return HZ_ERROR_SOLVER_STAG;
@@ -425,11 +428,11 @@ __device__ int coarse_cg_body(int n, int nslices, const long long *__restrict__ 
         }
         if (relres < tol) {                                        // Check III
             __syncthreads();
-            cg_matvec(n, nslices, sptr, col, val, u, r, 1.0, b);
+            cg_matvec<kCgBlock>(n, nslices, sptr, col, val, u, r, 1.0, b);
             __syncthreads();
             acc = 0.0;
             for (int i = tid; i < n; i += kCgBlock) acc += r[i] * r[i];
-            absres = sqrt(cg_block_sum(acc, sh));
+            absres = sqrt(cg_block_sum<kCgBlock>(acc, sh));
             relres = absres / normr0;
             if (relres < tol) return iter;
             if (more_step >= 20) return HZ_ERROR_SOLVER_TOLSMALL;
@@ -440,7 +443,7 @@ __device__ int coarse_cg_body(int n, int nslices, const long long *__restrict__ 
         __syncthreads();
         acc = 0.0;
         for (int i = tid; i < n; i += kCgBlock) acc += r[i] * r[i];
-        const double zr = cg_block_sum(acc, sh);
+        const double zr = cg_block_sum<kCgBlock>(acc, sh);
         const double beta = zr / temp1;
         temp1 = zr;
         for (int i = tid; i < n; i += kCgBlock) p[i] = 1.0 * r[i] + beta * p[i];
@@ -449,23 +452,204 @@ __device__ int coarse_cg_body(int n, int nslices, const long long *__restrict__ 
 }
 
 
+// Wavefront sum of non-negative or signed values / maximum of non-negative
+// ones through the lanes' data paths (row shifts, then the two row
+// broadcasts), the result in every lane.  Six dependent steps of a few cycles
+// each; through LDS permutes they are most of a short reduction.
+template <int kCtrl, int kRowMask>
+__device__ __forceinline__ double dpp_move(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), kCtrl, kRowMask, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), kCtrl, kRowMask, 0xf, false);
+    return __hiloint2double(hi, lo);   // 0.0 where no lane sends
+}
+__device__ __forceinline__ double last_lane(double v) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), kWave - 1);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), kWave - 1);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_sum(double v) {
+    v += dpp_move<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8
+    v += dpp_move<0x112, 0xf>(v);
+    v += dpp_move<0x114, 0xf>(v);
+    v += dpp_move<0x118, 0xf>(v);
+    v += dpp_move<0x142, 0xa>(v);   // row_bcast 15
+    v += dpp_move<0x143, 0xc>(v);   // row_bcast 31
+    return last_lane(v);
+}
+__device__ __forceinline__ double wave_max(double v) {
+    v = fmax(v, dpp_move<0x111, 0xf>(v));
+    v = fmax(v, dpp_move<0x112, 0xf>(v));
+    v = fmax(v, dpp_move<0x114, 0xf>(v));
+    v = fmax(v, dpp_move<0x118, 0xf>(v));
+    v = fmax(v, dpp_move<0x142, 0xa>(v));
+    v = fmax(v, dpp_move<0x143, 0xc>(v));
+    return last_lane(v);
+}
+
+// coarse_cg_body for n <= kThreads: a thread owns a row, its u, r and p in
+// registers, up to kCgRowRegs of its entries too (longer rows read the rest
+// from memory), p in LDS for the products; three barriers an iteration.  The
+// solve is one chain of short dependent steps, so what counts is their latency:
+// 690 -> 76 us for the 192-row coarsest level of a 10,000-row 2-D hierarchy
+// (vectors and matrix through memory, 1,024 threads, eleven barriers an
+// iteration before).  The stopping rules are coarse_cg_body's; squares decide
+// first whether a root has to be taken to compare it.
+constexpr int kCgRowRegs = 16;
+constexpr int kCgSmallRows = 1024;
+template <int kThreads>
+__device__ int coarse_cg_small(int n, const long long *__restrict__ sptr, const int *__restrict__ col,
+                               const double *__restrict__ val, const double *__restrict__ b, double *__restrict__ u,
+                               double tol, int maxit) {
+    constexpr int kWaves = kThreads / kWave;
+    __shared__ double s_v[kThreads];            // the vector being multiplied
+    __shared__ double s_red[2][3][kWaves];      // partials of two reductions
+    const int tid = threadIdx.x, wv = tid / kWave;
+    const bool own = tid < n;
+    // the row's entries; padding multiplies the row's own value by zero
+    int cc[kCgRowRegs];
+    double vv[kCgRowRegs];
+    const long long base = own ? sptr[tid / kSlice] : 0;
+    const int wd = own ? (int)((sptr[tid / kSlice + 1] - base) / kSlice) : 0;
+    const int *c_row = col + base + tid % kSlice;
+    const double *v_row = val + base + tid % kSlice;
+#pragma unroll
+    for (int k = 0; k < kCgRowRegs; ++k) {
+        const int c = k < wd ? c_row[k * kSlice] : -1;
+        cc[k] = c >= 0 ? c : tid;
+        vv[k] = c >= 0 ? v_row[k * kSlice] : 0.0;
+    }
+    auto times = [&]() {   // the row's product with s_v, entries in stored order
+        double acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < kCgRowRegs; ++k) acc = acc + vv[k] * s_v[cc[k]];
+        for (int k = kCgRowRegs; k < wd; ++k) {
+            const int c = c_row[k * kSlice];
+            if (c >= 0) acc = acc + v_row[k * kSlice] * s_v[c];
+        }
+        return acc;
+    };
+    auto sum = [&](double v) {   // every thread gets the same total
+        const double w = wave_sum(v);
+        if (tid % kWave == 0) s_red[0][0][wv] = w;
+        __syncthreads();
+        double t = 0.0;
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) t += s_red[0][0][i];
+        return t;
+    };
+    const double bi = own ? b[tid] : 0.0;
+    double ui = own ? u[tid] : 0.0, ri = 0.0, pi = 0.0;
+    auto true_residual = [&]() {   // r = b - A u and its squared norm
+        __syncthreads();
+        s_v[tid] = ui;
+        __syncthreads();
+        ri = own ? bi - times() : 0.0;
+        const double t = sum(ri * ri);
+        __syncthreads();           // s_v and the partials are free again
+        return t;
+    };
+    const double maxdiff = tol * 1e-4;
+    int iter = 0, stag = 1, more_step = 1, result = HZ_ERROR_SOLVER_MAXIT;
+    double temp1 = true_residual();
+    const double absres0 = sqrt(temp1);
+    const double normr0 = absres0 > kSmallReal ? absres0 : kSmallReal;
+    if (absres0 / normr0 < tol || absres0 < 1e-3 * tol) return 0;
+    pi = ri;
+    s_v[tid] = pi;
+    __syncthreads();
+    while (iter++ < maxit) {
+        const double ti = own ? times() : 0.0;
+        const double alpha = temp1 / sum(ti * pi);
+        ui = ui + alpha * pi;
+        ri = ri + (-alpha) * ti;
+        const double w0 = wave_sum(ri * ri), w1 = wave_sum(ui * ui), w2 = wave_sum(pi * pi);
+        if (tid % kWave == 0) {
+            s_red[1][0][wv] = w0;
+            s_red[1][1][wv] = w1;
+            s_red[1][2][wv] = w2;
+        }
+        __syncthreads();
+        double rr = 0.0, uu = 0.0, pp = 0.0;
+#pragma unroll
+        for (int i = 0; i < kWaves; ++i) {
+            rr += s_red[1][0][i];
+            uu += s_red[1][1][i];
+            pp += s_red[1][2][i];
+        }
+        // ||u||_inf is not small while ||u||^2 is over n SMALLREAL^2
+        if (!(uu > 2.0 * n * kSmallReal * kSmallReal)) {           // Check I
+            const double w = wave_max(fabs(ui));
+            if (tid % kWave == 0) s_red[0][1][wv] = w;
+            __syncthreads();
+            double uinf = 0.0;
+            for (int i = 0; i < kWaves; ++i) uinf = fmax(uinf, s_red[0][1][i]);
+            if (uinf <= kSmallReal) {
+                result = HZ_ERROR_SOLVER_SOLSTAG;
+                break;
+            }
+        }
+        // reldiff = |alpha| ||p|| / ||u|| and relres = ||r|| / normr0 are taken
+        // only where their squares are not clearly above the limits
+        if (!(alpha * alpha * pp > 4.0 * maxdiff * maxdiff * uu)) {   // Check II
+            const double reldiff = fabs(alpha) * sqrt(pp) / sqrt(uu);
+            if ((stag <= 20) & (reldiff < maxdiff)) {
+                rr = true_residual();
+                if (sqrt(rr) / normr0 < tol) {
+                    result = iter;
+                    break;
+                }
+                if (stag >= 20) {
+                    result = HZ_ERROR_SOLVER_STAG;
+                    break;
+                }
+                pi = 0.0;
+                ++stag;
+            }
+        }
+        if (!(rr > 4.0 * tol * tol * normr0 * normr0) && sqrt(rr) / normr0 < tol) {   // Check III
+            rr = true_residual();
+            if (sqrt(rr) / normr0 < tol) {
+                result = iter;
+                break;
+            }
+            if (more_step >= 20) {
+                result = HZ_ERROR_SOLVER_TOLSMALL;
+                break;
+            }
+            pi = 0.0;
+            ++more_step;
+        }
+        const double beta = rr / temp1;
+        temp1 = rr;
+        pi = 1.0 * ri + beta * pi;
+        s_v[tid] = pi;
+        __syncthreads();
+    }
+    if (own) u[tid] = ui;
+    __syncthreads();
+    return result;
+}
+
 // Block-wide vector helpers of the coarse GMRES: element i always belongs to
-// thread i mod kCgBlock, so consecutive element-wise steps need no barrier.
+// thread i mod kThreads, so consecutive element-wise steps need no barrier.
+template <int kThreads>
 __device__ double blk_dot(int n, const double *x, const double *y, double *sh) {
     double acc = 0.0;
-    for (int i = threadIdx.x; i < n; i += kCgBlock) acc += x[i] * y[i];
-    return cg_block_sum(acc, sh);
+    for (int i = threadIdx.x; i < n; i += kThreads) acc += x[i] * y[i];
+    return cg_block_sum<kThreads>(acc, sh);
 }
+template <int kThreads>
 __device__ void blk_axpy(int n, double a, const double *x, double *y) {   // array_axpy (array.c:357-373)
-    for (int i = threadIdx.x; i < n; i += kCgBlock) {
+    for (int i = threadIdx.x; i < n; i += kThreads) {
         if (a == 1.0) y[i] += x[i];
         else if (a == -1.0) y[i] -= x[i];
         else y[i] += a * x[i];
     }
 }
+template <int kThreads>
 __device__ void blk_ax(int n, double a, double *x) {   // array_ax (array.c:332-341)
     if (a != 1.0)
-        for (int i = threadIdx.x; i < n; i += kCgBlock) x[i] *= a;
+        for (int i = threadIdx.x; i < n; i += kThreads) x[i] *= a;
 }
 
 // dcsr_pvgmres (krylov.c:4612-4931) without preconditioner, stop type 1, from
@@ -475,6 +659,7 @@ __device__ void blk_ax(int n, double a, double *x) {   // array_ax (array.c:332-
 // The Hessenberg matrix and the rotations live in LDS and are updated by
 // thread 0; every branch depends only on block-wide sums or LDS values read
 // after a barrier, so all threads take it together.  work: (restart + 3) n.
+template <int kThreads>
 __device__ int coarse_gmres_body(int n, int nslices, const long long *__restrict__ sptr, const int *__restrict__ col,
                                  const double *__restrict__ val, const double *__restrict__ b, double *__restrict__ x,
                                  double tol, int MaxIt, double *__restrict__ work, double *sh, double *hh, double *cs,
@@ -488,16 +673,17 @@ __device__ int coarse_gmres_body(int n, int nslices, const long long *__restrict
     int iter = 0, i = 0, Restart = R;
     double cr = 1.0, r_norm, r_norm_old, absres0, absres, relres;
     __syncthreads();
-    cg_matvec(n, nslices, sptr, col, val, x, Pk(0), 1.0, b);
+    cg_matvec<kThreads>(n, nslices, sptr, col, val, x, Pk(0), 1.0, b);
     __syncthreads();
-    r_norm = sqrt(blk_dot(n, Pk(0), Pk(0), sh));
+    r_norm = sqrt(blk_dot<kThreads>(n, Pk(0), Pk(0), sh));
     absres0 = r_norm > kSmallReal ? r_norm : kSmallReal;
     relres = r_norm / absres0;
     if (relres < tol || absres0 < 1e-3 * tol) return 0;
     while (iter < MaxIt) {
         r_norm_old = r_norm;
+        __syncthreads();   // the last cycle's readers of rs are done
         if (tid == 0) rs[0] = r_norm;
-        blk_ax(n, 1.0 / r_norm, Pk(0));
+        blk_ax<kThreads>(n, 1.0 / r_norm, Pk(0));
         if (cr > cr_max || iter == 0) Restart = restart_max;
         else if (cr < cr_min) {
         } else if (Restart - d > restart_min) Restart -= d;
@@ -507,16 +693,16 @@ __device__ int coarse_gmres_body(int n, int nslices, const long long *__restrict
             ++i;
             ++iter;
             __syncthreads();
-            cg_matvec(n, nslices, sptr, col, val, Pk(i - 1), Pk(i), 0.0, nullptr);
+            cg_matvec<kThreads>(n, nslices, sptr, col, val, Pk(i - 1), Pk(i), 0.0, nullptr);
             __syncthreads();
             for (int j = 0; j < i; ++j) {
-                const double h = blk_dot(n, Pk(j), Pk(i), sh);
+                const double h = blk_dot<kThreads>(n, Pk(j), Pk(i), sh);
                 if (tid == 0) hh[j * R + i - 1] = h;
-                blk_axpy(n, -h, Pk(j), Pk(i));
+                blk_axpy<kThreads>(n, -h, Pk(j), Pk(i));
             }
-            double t = sqrt(blk_dot(n, Pk(i), Pk(i), sh));
+            double t = sqrt(blk_dot<kThreads>(n, Pk(i), Pk(i), sh));
             if (tid == 0) hh[i * R + i - 1] = t;
-            if (t != 0.0) blk_ax(n, 1.0 / t, Pk(i));
+            if (t != 0.0) blk_ax<kThreads>(n, 1.0 / t, Pk(i));
             __syncthreads();
             if (tid == 0) {
                 for (int j = 1; j < i; ++j) {
@@ -551,19 +737,19 @@ __device__ int coarse_gmres_body(int n, int nslices, const long long *__restrict
             }
         }
         __syncthreads();
-        for (int e = tid; e < n; e += kCgBlock) w[e] = Pk(i - 1)[e];
-        blk_ax(n, rs[i - 1], w);
-        for (int j = i - 2; j >= 0; --j) blk_axpy(n, rs[j], Pk(j), w);
-        blk_axpy(n, 1.0, w, x);
+        for (int e = tid; e < n; e += kThreads) w[e] = Pk(i - 1)[e];
+        blk_ax<kThreads>(n, rs[i - 1], w);
+        for (int j = i - 2; j >= 0; --j) blk_axpy<kThreads>(n, rs[j], Pk(j), w);
+        blk_axpy<kThreads>(n, 1.0, w, x);
         if (relres < tol) {
             __syncthreads();
-            cg_matvec(n, nslices, sptr, col, val, x, r, 1.0, b);
+            cg_matvec<kThreads>(n, nslices, sptr, col, val, x, r, 1.0, b);
             __syncthreads();
-            r_norm = sqrt(blk_dot(n, r, r, sh));
+            r_norm = sqrt(blk_dot<kThreads>(n, r, r, sh));
             absres = r_norm;
             relres = absres / absres0;
             if (relres < tol) break;
-            for (int e = tid; e < n; e += kCgBlock) Pk(0)[e] = r[e];
+            for (int e = tid; e < n; e += kThreads) Pk(0)[e] = r[e];
             i = 0;
         }
         // the cycle's residual vector, the next cycle's first basis vector
@@ -574,11 +760,11 @@ __device__ int coarse_gmres_body(int n, int nslices, const long long *__restrict
                 rs[j] = cs[j - 1] * rs[j];
             }
         __syncthreads();
-        if (i) blk_axpy(n, rs[i] - 1.0, Pk(i), Pk(i));
-        for (int j = i - 1; j > 0; --j) blk_axpy(n, rs[j], Pk(j), Pk(i));
+        if (i) blk_axpy<kThreads>(n, rs[i] - 1.0, Pk(i), Pk(i));
+        for (int j = i - 1; j > 0; --j) blk_axpy<kThreads>(n, rs[j], Pk(j), Pk(i));
         if (i) {
-            blk_axpy(n, rs[0] - 1.0, Pk(0), Pk(0));
-            blk_axpy(n, 1.0, Pk(i), Pk(0));
+            blk_axpy<kThreads>(n, rs[0] - 1.0, Pk(0), Pk(0));
+            blk_axpy<kThreads>(n, 1.0, Pk(i), Pk(0));
         }
         cr = r_norm / r_norm_old;
     }
@@ -588,20 +774,24 @@ __device__ int coarse_gmres_body(int n, int nslices, const long long *__restrict
 // coarse_itsolver (mgcycle.c:34-53): CG from x, and GMRES(30) from CG's last
 // iterate when CG fails.  status (optional): [0] the final result code, [1]
 // CG's; u_cg (optional): CG's last iterate.
-__global__ __launch_bounds__(kCgBlock) void k_coarse_itsolver(int n, int nslices, const long long *__restrict__ sptr,
+// kSmall: n <= kThreads.
+template <int kThreads, bool kSmall>
+__global__ __launch_bounds__(kThreads) void k_coarse_itsolver(int n, int nslices, const long long *__restrict__ sptr,
                                                               const int *__restrict__ col,
                                                               const double *__restrict__ val,
                                                               const double *__restrict__ b, double *__restrict__ u,
                                                               double tol, int maxit, double *__restrict__ work,
                                                               int *__restrict__ status, double *__restrict__ u_cg) {
-    __shared__ double sh[kCgBlock / kWave];
+    __shared__ double sh[kThreads / kWave];
     __shared__ double hh[(kCoarseGmresRestart + 1) * kCoarseGmresRestart];
     __shared__ double cs[kCoarseGmresRestart + 1], sn[kCoarseGmresRestart + 1], rs[kCoarseGmresRestart + 1];
-    const int st_cg = coarse_cg_body(n, nslices, sptr, col, val, b, u, tol, maxit, work, sh);
+    int st_cg;
+    if constexpr (kSmall) st_cg = coarse_cg_small<kThreads>(n, sptr, col, val, b, u, tol, maxit);
+    else st_cg = coarse_cg_body(n, nslices, sptr, col, val, b, u, tol, maxit, work, sh);
     if (u_cg)
-        for (int i = threadIdx.x; i < n; i += kCgBlock) u_cg[i] = u[i];
+        for (int i = threadIdx.x; i < n; i += kThreads) u_cg[i] = u[i];
     int st = st_cg;
-    if (st < 0) st = coarse_gmres_body(n, nslices, sptr, col, val, b, u, tol, maxit, work, sh, hh, cs, sn, rs);
+    if (st < 0) st = coarse_gmres_body<kThreads>(n, nslices, sptr, col, val, b, u, tol, maxit, work, sh, hh, cs, sn, rs);
     if (status && threadIdx.x == 0) {
         status[0] = st;
         status[1] = st_cg;
@@ -722,8 +912,18 @@ void coarse_dense_solve(int n, const double *Ainv, const double *b, double *x) {
 void coarse_cg(const DevSELL &S, const double *b, double *x, double tol, int maxit, double *work, int *status,
                double *x_cg) {
     if (S.n == 0) return;
-    k_coarse_itsolver<<<1, kCgBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, b, x, tol, maxit, work,
-                                                    status, x_cg);
+    // the fewest wavefronts that give every row a thread: their barriers are
+    // in the solve's chain
+    auto go = [&](auto threads, auto small) {
+        constexpr int T = decltype(threads)::value;
+        k_coarse_itsolver<T, decltype(small)::value><<<1, T, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, b, x,
+                                                                            tol, maxit, work, status, x_cg);
+    };
+    if (S.n <= 64) go(std::integral_constant<int, 64>{}, std::true_type{});
+    else if (S.n <= 256) go(std::integral_constant<int, 256>{}, std::true_type{});
+    else if (S.n <= 512) go(std::integral_constant<int, 512>{}, std::true_type{});
+    else if (S.n <= kCgSmallRows) go(std::integral_constant<int, 1024>{}, std::true_type{});
+    else go(std::integral_constant<int, kCgBlock>{}, std::false_type{});
     HZ_LAUNCH_CHECK();
 }
 

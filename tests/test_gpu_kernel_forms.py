@@ -158,3 +158,46 @@ def test_fused_cycle_kernels_vs_oracle(lib, orc, libc, case, smoother):
     assert off(0, "oracle") < 1e-12
     assert off(1, 0) < 2e-5
     assert off(2, 0) < 5e-2
+
+
+# thread counts of the one-row-a-thread CG are 64, 256, 512 and 1,024; 1,025 rows run the general form; 20
+# off-diagonal entries a row read past the 16 held in registers
+@pytest.mark.parametrize("n", [1, 5, 63, 64, 65, 255, 256, 257, 512, 513, 1024, 1025])
+@pytest.mark.parametrize("per_row", [4, 20])
+def test_coarse_cg_sizes_vs_oracle(lib, orc, n, per_row):
+    """The coarsest level's CG against the oracle's: iterations within one; solutions of systems of condition below
+    10 at relative residuals of 1e-8 differ by less than 2e-7; and on a nonsymmetric matrix of the same size CG
+    fails and GMRES takes over, as the oracle's does."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(n + per_row)
+    k = min(per_row // 2, max(0, n - 1))
+    i = np.repeat(np.arange(n), k)
+    j = rng.integers(0, n, i.size)
+    off = sp.csr_matrix((rng.uniform(-1.0, 0.0, i.size), (i, j)), shape=(n, n))
+    off = off + off.T
+    off.setdiag(0.0)
+    off.eliminate_zeros()
+    A = (off + sp.diags(1.0 + 1.5 * np.abs(off).sum(axis=1).A1)).tocsr()
+    A.sort_indices()
+    b = problems.uniform_rhs(n, seed=2)
+    Ah = capi.HostCSR(A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data.astype(np.float64))
+    x, xcg, xo = np.zeros(n), np.zeros(n), np.zeros(n)
+    st_cg = capi.INT()
+    st = lib.hz_coarse_itsolver(Ah.ptr(), capi.dptr(b), capi.dptr(x), 1e-8, C.byref(st_cg), capi.dptr(xcg))
+    so = orc.orc_coarse_itsolver(Ah.ptr(), capi.dptr(b), capi.dptr(xo), 1e-8)
+    assert st == st_cg.value > 0 and abs(st - so) <= 1
+    assert np.array_equal(x, xcg)
+    assert np.linalg.norm(x - xo) <= 2e-7 * np.linalg.norm(xo)
+
+
+@pytest.mark.parametrize("m", [7, 16, 20, 32])
+def test_coarse_gmres_after_small_cg_vs_oracle(lib, orc, m):
+    from test_gpu_semantics import _coarse_gpu, _convdiff
+    A = _convdiff(m, 6.0, 4.0)
+    n = A.shape[0]
+    b = problems.uniform_rhs(n, seed=3)
+    st, st_cg, x, xcg, Ah = _coarse_gpu(lib, A, b)
+    xo = xcg.copy()
+    so = orc.orc_pvgmres(Ah.ptr(), capi.dptr(b), capi.dptr(xo), 1e-8, 20 * n, 30)
+    assert st_cg < 0 < st and abs(st - so) <= 2
+    assert np.linalg.norm(x - xo) <= 1e-6 * np.linalg.norm(xo)
