@@ -482,14 +482,15 @@ void presmooth(Hierarchy &H, int l, CycleState &cs) {
     const CycleParams &cp = H.cp;
     int sweeps = cp.smoother == HZ_SMOOTHER_CHEBY ? cheb_steps_at(cp, l, cp.presmooth) : cp.presmooth;
     if (cp.smoother == HZ_SMOOTHER_CHEBY || is_gs_family(cp.smoother)) {
-        // Chebyshev from zero: its first step reads no x (nor the matrix)
-        const bool cheb_from_zero = cp.smoother == HZ_SMOOTHER_CHEBY && cs.zero[l] && sweeps > 0;
-        if (cs.zero[l] && !cheb_from_zero) fill(L.x, 0.0, L.A.n);
+        // from zero, Chebyshev's first step reads no x (nor the matrix) and
+        // Gauss-Seidel takes its starting values as zeros
+        const bool from_zero = cs.zero[l];
+        if (from_zero && cp.smoother == HZ_SMOOTHER_CHEBY && sweeps <= 0) fill(L.x, 0.0, L.A.n);
         cs.zero[l] = false;
         cs.first_done[l] = false;
         if (cp.smoother == HZ_SMOOTHER_CHEBY)
-            cheby_apply(L.S, L.cheb, sweeps, L.b, L.x, L.xt, L.cwork, &L.A, cheb_from_zero);
-        else gs_smooth(L.gs, cp.smoother, false, sweeps, cp.relax, L.b, L.x);
+            cheby_apply(L.S, L.cheb, sweeps, L.b, L.x, L.xt, L.cwork, &L.A, from_zero && sweeps > 0);
+        else gs_smooth(L.gs, cp.smoother, false, sweeps, cp.relax, L.b, L.x, from_zero);
         return;
     }
     if (cs.zero[l]) {

@@ -1401,7 +1401,7 @@ INT hz_gs_smooth(dCSRmat *A, const REAL *b, REAL *x, INT smoother, INT post, INT
         gs_prepare(dA, G);
         gs_smooth(G, (int)smoother, post != 0, (int)nsweeps, relax, db, dx);
         HZ_CHECK(memcpy_sync(x, dx, sizeof(double) * A->row, hipMemcpyDeviceToHost));
-        if (order && A->row > 0) HZ_CHECK(memcpy_sync(order, G.rows, sizeof(int) * A->row, hipMemcpyDeviceToHost));
+        if (order && A->row > 0) HZ_CHECK(memcpy_sync(order, G.order, sizeof(int) * A->row, hipMemcpyDeviceToHost));
         if (cptr)
             for (int c = 0; c <= G.ncolors; ++c) cptr[c] = G.cptr.empty() ? 0 : G.cptr[c];
         if (ncolors) *ncolors = G.ncolors;

@@ -12,13 +12,30 @@
 // colour), not in the natural order the reference sweeps in: results follow
 // the reference's by convergence behaviour, not bit for bit.
 //
-// Layout: per colour, the rows (ascending) are cut into slices of 64; a slice
-// stores its rows' off-diagonal entries column-major (entry k of lane t at
-// sptr[s] + 64 k + t, CSR order inside the row, zero-padded to the slice
-// width), and the diagonal a_ii separately.  One launch per colour; a wave
-// handles one slice.
+// Layout: the rows are listed colour by colour (ascending inside one), each
+// colour padded to slices of 64 positions; a slice stores its rows'
+// off-diagonal entries column-major as positions (entry k of lane t at
+// 64 (W slice + k) + t, CSR order inside the row, W the longest row, padding a
+// zero entry on the lane's own position) and the diagonal a_ii separately, so
+// that nothing has to be loaded to find a slice's data.  Stored zeros are left
+// out.  A wave handles one slice; one launch per colour, or on levels whose x
+// fits LDS one workgroup for the whole smoothing call.
+//
+// What bounds a sweep on all but the largest levels is the chain of a colour
+// visit: a launch or a barrier, the entries' loads, the gathers, the division
+// (SGS visits 21 colours a call, twice a level and cycle).  Entries go in
+// rounds of 8 or 16 masked loads (rows of 6 entries took six dependent pairs of
+// loads when only whole rounds of eight were batched), and the one-workgroup
+// form loads a wave's next two slices ahead.  Measured on the 64^3 Poisson
+// hierarchy (SGS, 11 colours): a colour's launch 7.5 -> 4.1 us, the one-workgroup
+// call on 7,811 / 3,902 / 1,950 rows 165 / 90 / 65 -> 62 / 40 / 29 us, PCG
+// 42.5 -> 26.2 ms; the preparation (rows sorted and placed on the GPU, no
+// transpose where the pattern is symmetric) 9 -> 5 ms over eight levels.
 #include <algorithm>
+#include <type_traits>
 #include <vector>
+
+#include <rocprim/device/device_radix_sort.hpp>
 
 #include "hz_internal.h"
 
@@ -29,8 +46,15 @@ namespace {
 constexpr int kBlock = 256;
 static_assert(kSlice == 64, "one wave per slice");
 constexpr int kGsMaxPass = 8;               // passes per single-workgroup launch
-constexpr int kGsLdsRows = 8192;            // levels up to this size keep x in LDS (64 KiB)
+// Levels of up to this many positions keep x in LDS (144 of the CU's 160 KiB)
+// and run as one workgroup.  At the upper end, 15,627 rows of 10 entries, 21
+// colour visits take 105 us (the random LDS gathers of eight waves bound it)
+// against 21 launches of 4.1 us and a permutation of 5; with one pass and
+// shorter rows (10,000 rows of 5, 10 visits) 24 us against 46.
+constexpr int kGsLdsPos = 18432;
+constexpr int kGsMaxPhase = 1024;           // colour visits per single-workgroup launch
 constexpr int kSlicesPerBlock = kBlock / kSlice;
+constexpr int kHistBins = 256;
 
 int grid_rows(long n) { return (int)std::max(1L, std::min<long>((n + kBlock - 1) / kBlock, 16384)); }
 
@@ -47,8 +71,45 @@ __device__ __forceinline__ bool beats(int j, unsigned pj, int i, unsigned pi) {
     return pj > pi || (pj == pi && j > i);
 }
 
+// Whether some uncoloured neighbour in one list beats row i, a round of eight
+// columns' loads at a time.
+__device__ __forceinline__ bool jp_beaten(int i, unsigned pi, const int *__restrict__ p, const int *__restrict__ q,
+                                          const int *__restrict__ color) {
+    const int k1 = p[i + 1];
+    for (int k = p[i]; k < k1; k += 8) {
+        int j[8], c[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) j[u] = k + u < k1 ? q[k + u] : i;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) c[u] = color[j[u]];
+        bool lost = false;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) lost = lost || (j[u] != i && c[u] < 0 && beats(j[u], jp_priority(j[u]), i, pi));
+        if (lost) return true;
+    }
+    return false;
+}
+
+__device__ __forceinline__ unsigned long long jp_used(int i, int base, const int *__restrict__ p,
+                                                      const int *__restrict__ q, const int *__restrict__ color) {
+    unsigned long long used = 0ull;
+    const int k1 = p[i + 1];
+    for (int k = p[i]; k < k1; k += 8) {
+        int j[8], c[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) j[u] = k + u < k1 ? q[k + u] : i;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) c[u] = j[u] != i ? color[j[u]] - base : -1;
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (c[u] >= 0 && c[u] < 64) used |= 1ull << c[u];
+    }
+    return used;
+}
+
 // One Jones-Plassmann round over the pattern of A (ia/ja) and of A^T
-// (ta/tj).  color_in[i] = -1 while row i is uncoloured.
+// (ta/tj; null when the pattern is symmetric).  color_in[i] = -1 while row i is
+// uncoloured.
 __global__ void k_jp_round(int n, const int *__restrict__ ia, const int *__restrict__ ja,
                            const int *__restrict__ ta, const int *__restrict__ tj, const int *__restrict__ color_in,
                            int *__restrict__ color_out, int *__restrict__ left) {
@@ -57,111 +118,148 @@ __global__ void k_jp_round(int n, const int *__restrict__ ia, const int *__restr
         int c = color_in[i];
         if (c < 0) {
             const unsigned pi = jp_priority(i);
-            bool wins = true;
-            for (int pass = 0; pass < 2 && wins; ++pass) {
-                const int *p = pass ? ta : ia;
-                const int *q = pass ? tj : ja;
-                for (int k = p[i]; k < p[i + 1]; ++k) {
-                    const int j = q[k];
-                    if (j != i && color_in[j] < 0 && beats(j, jp_priority(j), i, pi)) {
-                        wins = false;
-                        break;
-                    }
-                }
-            }
-            if (wins) {
+            if (jp_beaten(i, pi, ia, ja, color_in) || (ta && jp_beaten(i, pi, ta, tj, color_in))) {
+                ++local;
+            } else {
                 // smallest colour free among the coloured neighbours, 64 at a time
                 for (int base = 0;; base += 64) {
-                    unsigned long long used = 0ull;
-                    for (int pass = 0; pass < 2; ++pass) {
-                        const int *p = pass ? ta : ia;
-                        const int *q = pass ? tj : ja;
-                        for (int k = p[i]; k < p[i + 1]; ++k) {
-                            const int j = q[k];
-                            const int cj = j != i ? color_in[j] - base : -1;
-                            if (cj >= 0 && cj < 64) used |= 1ull << cj;
-                        }
-                    }
+                    unsigned long long used = jp_used(i, base, ia, ja, color_in);
+                    if (ta) used |= jp_used(i, base, ta, tj, color_in);
                     if (~used) {
                         c = base + __ffsll((long long)~used) - 1;
                         break;
                     }
                 }
-            } else {
-                ++local;
             }
         }
         color_out[i] = c;
     }
-    if (local && left) atomicAdd(left, local);
-}
-
-// Off-diagonal entries a sweep reads: stored zeros are left out (a product with
-// one changes no sum); the colouring sees the whole pattern.
-__global__ void k_offdiag_count(int n, const int *__restrict__ ia, const int *__restrict__ ja,
-                                const double *__restrict__ a, int *__restrict__ cnt) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        int c = 0;
-        for (int k = ia[i]; k < ia[i + 1]; ++k) c += ja[k] != i && a[k] != 0.0;
-        cnt[i] = c;
+    if (left) {
+#pragma unroll
+        for (int off = kWave / 2; off > 0; off >>= 1) local += __shfl_xor(local, off, kWave);
+        if (threadIdx.x % kWave == 0 && local) atomicAdd(left, local);
     }
 }
 
-// Slice fill: one thread per (slice, lane).  Columns are stored as list
-// positions (pos_of[j]): the sweeps work on vectors permuted to the
-// colour-major order, where the rows a colour's slice reads lie close
-// together, as they do in the natural order.
-__global__ void k_gs_fill(int nslices, const int *__restrict__ spos, const int *__restrict__ scnt,
-                          const long long *__restrict__ sptr, const int *__restrict__ rows,
-                          const int *__restrict__ pos_of, const int *__restrict__ ia, const int *__restrict__ ja,
-                          const double *__restrict__ a, int *__restrict__ col, double *__restrict__ val,
-                          double *__restrict__ diag) {
-    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int s = (int)(gid / kSlice), lane = (int)(gid % kSlice);
+// *bad is set when some entry (i, j) has no (j, i)
+__global__ void k_gs_symmetric(int n, const int *__restrict__ ia, const int *__restrict__ ja, int *__restrict__ bad) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+        for (int k = ia[i]; k < ia[i + 1]; ++k) {
+            const int j = ja[k];
+            if (j == i) continue;
+            bool found = false;
+            const int q1 = ia[j + 1];
+            for (int q = ia[j]; q < q1 && !found; q += 8) {
+                int c[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) c[u] = q + u < q1 ? ja[q + u] : -1;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) found = found || c[u] == i;
+            }
+            if (!found) {
+                *bad = 1;
+                return;
+            }
+        }
+}
+
+// rows per colour and info[0] = the largest colour; keys and idx for the sort
+__global__ __launch_bounds__(kBlock) void k_color_hist(int n, const int *__restrict__ color, int *__restrict__ cnt,
+                                                       int *__restrict__ info, unsigned int *__restrict__ keys,
+                                                       int *__restrict__ idx) {
+    __shared__ int h[kHistBins];
+    for (int t = threadIdx.x; t < kHistBins; t += kBlock) h[t] = 0;
+    __syncthreads();
+    int most = 0;
+    for (int i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+        const int c = color[i];
+        keys[i] = (unsigned int)c;
+        idx[i] = i;
+        most = max(most, c);
+        if (c < kHistBins) atomicAdd(&h[c], 1);
+        else atomicAdd(&cnt[c], 1);
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < kHistBins; t += kBlock)
+        if (h[t]) atomicAdd(&cnt[t], h[t]);
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) most = max(most, __shfl_xor(most, off, kWave));
+    if (threadIdx.x % kWave == 0) atomicMax(info, most);
+}
+
+// One wave per slice: the rows at its positions, their positions, and the
+// widest row's off-diagonal entries that a sweep reads (stored zeros are left
+// out; the colouring sees the whole pattern).  cptr: first sorted row of each
+// colour, sl0: first slice.
+__global__ __launch_bounds__(kBlock) void k_gs_place(int nslices, int nc, const int *__restrict__ cptr,
+                                                     const int *__restrict__ sl0, const int *__restrict__ sorted,
+                                                     const int *__restrict__ ia, const int *__restrict__ ja,
+                                                     const double *__restrict__ a, int *__restrict__ rows,
+                                                     int *__restrict__ pos_of, int *__restrict__ width,
+                                                     int *__restrict__ info) {
+    const int s = blockIdx.x * kSlicesPerBlock + threadIdx.x / kSlice;
+    const int lane = threadIdx.x % kSlice;
     if (s >= nslices) return;
-    const long long base = sptr[s];
-    const int width = (int)((sptr[s + 1] - base) / kSlice);
-    const int pos0 = spos[s];
-    const int me = pos0 + (lane < scnt[s] ? lane : 0);
-    const int i = rows[me];
+    int lo = 0, hi = nc - 1;   // the last colour whose first slice is not after s
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) / 2;
+        if (sl0[mid] <= s) lo = mid;
+        else hi = mid - 1;
+    }
+    const int q = cptr[lo] + (s - sl0[lo]) * kSlice + lane;
+    const int i = q < cptr[lo + 1] ? sorted[q] : -1;
+    rows[s * kSlice + lane] = i;
+    int w = 0;
+    if (i >= 0) {
+        pos_of[i] = s * kSlice + lane;
+        for (int k = ia[i]; k < ia[i + 1]; ++k) w += ja[k] != i && a[k] != 0.0;
+    }
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) w = max(w, __shfl_xor(w, off, kWave));
+    if (lane == 0) {
+        width[s] = w;
+        if (w > info[1]) atomicMax(info + 1, w);
+    }
+}
+
+// Slice fill: one thread per position.  Columns are stored as positions
+// (pos_of[j]): the sweeps work on vectors in that order, where the rows a
+// colour's slice reads lie close together, as they do in the natural order.
+__global__ void k_gs_fill(int nslices, int W, const int *__restrict__ rows, const int *__restrict__ pos_of,
+                          const int *__restrict__ ia, const int *__restrict__ ja, const double *__restrict__ a,
+                          int *__restrict__ col, double *__restrict__ val, double *__restrict__ diag) {
+    const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p >= (long)nslices * kSlice) return;
+    const long long base = p / kSlice * W * kSlice + p % kSlice;
+    const int i = rows[p];
     int k2 = 0;
-    if (lane < scnt[s]) {
-        double d = 0.0;
+    double d = 0.0;
+    if (i >= 0)
         for (int k = ia[i]; k < ia[i + 1]; ++k) {
             const int j = ja[k];
             if (j == i) {
                 d = a[k];
             } else if (a[k] != 0.0) {
-                col[base + (long long)k2 * kSlice + lane] = pos_of[j];
-                val[base + (long long)k2 * kSlice + lane] = a[k];
+                col[base + (long long)k2 * kSlice] = pos_of[j];
+                val[base + (long long)k2 * kSlice] = a[k];
                 ++k2;
             }
         }
-        diag[me] = d;
-    }
-    for (; k2 < width; ++k2) {   // padding: a zero entry on a valid position
-        col[base + (long long)k2 * kSlice + lane] = me;
-        val[base + (long long)k2 * kSlice + lane] = 0.0;
+    diag[p] = d;   // 0.0 at an empty position, whose value then stays
+    for (; k2 < W; ++k2) {
+        col[base + (long long)k2 * kSlice] = (int)p;
+        val[base + (long long)k2 * kSlice] = 0.0;
     }
 }
 
-__global__ void k_pos_of(int n, const int *__restrict__ rows, int *__restrict__ pos_of) {
-    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) pos_of[rows[p]] = p;
-}
-
-// xp[p] = x[rows[p]], bp[p] = b[rows[p]]
-__global__ void k_perm_in(int n, const int *__restrict__ rows, const double *__restrict__ x,
+// xp[p] = x[rows[p]] (0 where x is zero: x null), bp[p] = b[rows[p]]
+__global__ void k_perm_in(int npos, const int *__restrict__ rows, const double *__restrict__ x,
                           const double *__restrict__ b, double *__restrict__ xp, double *__restrict__ bp) {
-    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
+    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < npos; p += gridDim.x * blockDim.x) {
         const int i = rows[p];
-        xp[p] = x[i];
-        bp[p] = b[i];
+        xp[p] = x && i >= 0 ? x[i] : 0.0;
+        bp[p] = i >= 0 ? b[i] : 0.0;
     }
-}
-
-__global__ void k_perm_out(int n, const int *__restrict__ rows, const double *__restrict__ xp,
-                           double *__restrict__ x) {
-    for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) x[rows[p]] = xp[p];
 }
 
 // The update of one row from t = b_i - sum_{j != i} a_ij x_j (CSR order):
@@ -176,92 +274,170 @@ __device__ __forceinline__ double gs_update(int mode, double t, double d, double
     return w * (t / d) + (1 - w) * xo;
 }
 
-// t - sum_k val[k] x[col[k]] over one lane's slice entries, subtracted in
-// entry order; the loads of 8 entries are issued before their products so
-// that the gathers overlap (the order of the subtractions is unchanged).
-template <class XT>
-__device__ __forceinline__ double slice_row_sub(double t, const int *__restrict__ cp, const double *__restrict__ vp,
-                                                int width, const XT *x) {
-    int k = 0;
-    for (; k + 8 <= width; k += 8) {
-        int c[8];
-        double v[8], xv[8];
+// A slice's first U entries in a lane's registers (zero past its width).
+template <int U>
+struct GsEntries {
+    int c[U];
+    double v[U];
+};
+template <bool kNt, int U>
+__device__ __forceinline__ void gs_load(GsEntries<U> &e, const int *__restrict__ cp, const double *__restrict__ vp,
+                                        int k, int width, int self) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            c[u] = ld_nt(cp + (long long)(k + u) * kSlice);
-            v[u] = ld_nt(vp + (long long)(k + u) * kSlice);
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) xv[u] = x[c[u]];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) t -= v[u] * xv[u];
+    for (int u = 0; u < U; ++u) {
+        const bool ok = k + u < width;
+        const int *c = cp + (long long)(k + u) * kSlice;
+        const double *v = vp + (long long)(k + u) * kSlice;
+        e.c[u] = ok ? (kNt ? ld_nt(c) : *c) : self;
+        e.v[u] = ok ? (kNt ? ld_nt(v) : *v) : 0.0;
     }
-    for (; k < width; ++k) t -= ld_nt(vp + (long long)k * kSlice) * x[ld_nt(cp + (long long)k * kSlice)];
+}
+// t - sum of products, subtracted in entry order
+template <int U, class XT>
+__device__ __forceinline__ double gs_subtract(double t, const GsEntries<U> &e, const XT *x) {
+    double xv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) xv[u] = x[e.c[u]];
+#pragma unroll
+    for (int u = 0; u < U; ++u) t -= e.v[u] * xv[u];
     return t;
 }
 
-// One colour on the permuted vectors; a wave per slice.
-template <int kMode>
-__global__ void __launch_bounds__(kBlock) k_gs_color(int s0, int ns, const int *__restrict__ spos,
-                                                     const int *__restrict__ scnt, const long long *__restrict__ sptr,
-                                                     const int *__restrict__ col, const double *__restrict__ val,
-                                                     const double *__restrict__ diag, const double *__restrict__ bp,
-                                                     double *__restrict__ xp, double w) {
+// One colour (slices s0 .. s0 + ns - 1); a wave per slice.  xout (optional):
+// the new values in the rows' own order as well (the colour's last visit).
+// kNt: the entries stream past the caches (levels whose matrix does not stay
+// there from one colour visit to the next).
+template <int kMode, int U, bool kNt>
+__global__ void __launch_bounds__(kBlock) k_gs_color(int s0, int ns, int W, const int *__restrict__ width,
+                                                     const int *__restrict__ rows, const int *__restrict__ col,
+                                                     const double *__restrict__ val, const double *__restrict__ diag,
+                                                     const double *__restrict__ bp, double *__restrict__ xp, double w,
+                                                     double *__restrict__ xout) {
     const int sl = blockIdx.x * kSlicesPerBlock + threadIdx.x / kSlice;
     const int lane = threadIdx.x % kSlice;
     if (sl >= ns) return;
-    const int s = s0 + sl;
-    // slice header loads issued together
-    const int cnt = scnt[s], p0 = spos[s];
-    const long long base = sptr[s], end = sptr[s + 1];
-    if (lane >= cnt) return;
-    const int width = (int)((end - base) / kSlice);
-    const int pos = p0 + lane;
-    const double bi = bp[pos], d = diag[pos];
-    const double t = slice_row_sub(bi, col + base + lane, val + base + lane, width, xp);
-    xp[pos] = gs_update(kMode, t, d, xp[pos], w);
+    const int s = s0 + sl, p = s * kSlice + lane;
+    const int wd = width ? width[s] : W;
+    const int *cp = col + (long long)s * W * kSlice + lane;
+    const double *vp = val + (long long)s * W * kSlice + lane;
+    const double bi = bp[p], d = diag[p], xo = xp[p];
+    const int row = xout ? rows[p] : -1;
+    double t = bi;
+    for (int k = 0; k < wd; k += U) {
+        GsEntries<U> e;
+        gs_load<kNt>(e, cp, vp, k, wd, p);
+        t = gs_subtract(t, e, xp);
+    }
+    const double xn = gs_update(kMode, t, d, xo, w);
+    xp[p] = xn;
+    if (row >= 0) xout[row] = xn;
 }
 
-// Whole smoothing call of a small level in one workgroup, x held in LDS
-// (permuted): the passes in turn, the colours of a pass in turn, a barrier
-// after each colour.  Same arithmetic as k_gs_color.
+// Whole smoothing call of a small level in one workgroup, x held in LDS: the
+// passes in turn, the colours of a pass in turn, a barrier after each colour.
+// Same arithmetic as k_gs_color.  The slices a wave visits are known ahead, so
+// the entries of its next kGsAhead slices are on their way while one is
+// computed, and the barrier waits for LDS only, not for those loads.
+constexpr int kGsAhead = 2;
 struct GsProgram {
     int npass;
     int forward[kGsMaxPass], mode[kGsMaxPass], skip[kGsMaxPass];
     double w[kGsMaxPass];
 };
 
-__global__ void __launch_bounds__(1024) k_gs_lds(int n, int ncolors, const int *__restrict__ sl0,
-                                                 const int *__restrict__ spos, const int *__restrict__ scnt,
-                                                 const long long *__restrict__ sptr, const int *__restrict__ rows,
-                                                 const int *__restrict__ col, const double *__restrict__ val,
-                                                 const double *__restrict__ diag, const double *__restrict__ b,
-                                                 double *__restrict__ x, GsProgram prog) {
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// kMixed: the passes differ in mode or weight (looked up per colour visit).
+template <int U, int kThreads, bool kMixed>
+__global__ void __launch_bounds__(kThreads) k_gs_lds(int npos, int ncolors, int W, int steps,
+                                                     const int *__restrict__ sl0, const int *__restrict__ rows,
+                                                     const int *__restrict__ col, const double *__restrict__ val,
+                                                     const double *__restrict__ diag, double *__restrict__ bp,
+                                                     const double *__restrict__ b, const double *__restrict__ x,
+                                                     double *__restrict__ xout, GsProgram prog) {
     extern __shared__ double xs[];
-    for (int p = threadIdx.x; p < n; p += blockDim.x) xs[p] = x[rows[p]];
-    __syncthreads();
-    const int wave = threadIdx.x / kSlice, nwaves = blockDim.x / kSlice;
-    const int lane = threadIdx.x % kSlice;
+    __shared__ int ph_s0[kGsMaxPhase], ph_s1[kGsMaxPhase];
+    __shared__ unsigned char ph_pass[kMixed ? kGsMaxPhase : 1];
+    int nph = 0;
     for (int ps = 0; ps < prog.npass; ++ps) {
         const int count = ncolors - prog.skip[ps];
-        const int mode = prog.mode[ps];
-        const double w = prog.w[ps];
-        for (int q = 0; q < count; ++q) {
+        for (int q = threadIdx.x; q < count; q += kThreads) {
             const int c = prog.forward[ps] ? q + prog.skip[ps] : ncolors - 1 - prog.skip[ps] - q;
-            for (int s = sl0[c] + wave; s < sl0[c + 1]; s += nwaves) {
-                const int cnt = scnt[s], p0 = spos[s];
-                const long long base = sptr[s], end = sptr[s + 1];
-                if (lane >= cnt) continue;
-                const int width = (int)((end - base) / kSlice);
-                const int pos = p0 + lane;
-                const double bi = b[rows[pos]], d = diag[pos];
-                const double t = slice_row_sub(bi, col + base + lane, val + base + lane, width, xs);
-                xs[pos] = gs_update(mode, t, d, xs[pos], w);
-            }
-            __syncthreads();
+            ph_s0[nph + q] = sl0[c];
+            ph_s1[nph + q] = sl0[c + 1];
+            if (kMixed) ph_pass[nph + q] = (unsigned char)ps;
         }
+        nph += count;
     }
-    for (int p = threadIdx.x; p < n; p += blockDim.x) x[rows[p]] = xs[p];
+    for (int p = threadIdx.x; p < npos; p += kThreads) {
+        const int i = rows[p];
+        xs[p] = x && i >= 0 ? x[i] : 0.0;
+        bp[p] = i >= 0 ? b[i] : 0.0;
+    }
+    __syncthreads();
+    constexpr int kWaves = kThreads / kSlice;
+    const int wave = threadIdx.x / kSlice, lane = threadIdx.x % kSlice;
+    struct Slice {
+        bool on;
+        int p, pass;
+        double bi, d;
+        GsEntries<U> e;
+    };
+    const int total = nph * steps;   // a colour takes `steps` slices a wave at most
+    const int mode0 = prog.mode[0];
+    const double w0 = prog.w[0];
+    // the visit that is loaded next: colour visit ph, its step j
+    int ph = 0, j = 0;
+    auto load = [&](Slice &S) {
+        const bool more = ph < nph;
+        const int s = __builtin_amdgcn_readfirstlane(more ? ph_s0[ph] + wave + kWaves * j : 0);
+        const int s1 = __builtin_amdgcn_readfirstlane(more ? ph_s1[ph] : 0);
+        S.on = s < s1;
+        if (kMixed) S.pass = more ? ph_pass[ph] : 0;
+        if (++j == steps) {
+            j = 0;
+            ++ph;
+        }
+        if (!S.on) return;
+        S.p = s * kSlice + lane;
+        S.bi = bp[S.p];
+        S.d = diag[S.p];
+        gs_load<false>(S.e, col + (long long)s * W * kSlice + lane, val + (long long)s * W * kSlice + lane, 0, W, S.p);
+    };
+    int done = 0;   // steps of the current visit
+    auto compute = [&](Slice &S) {
+        if (S.on) {
+            double t = gs_subtract(S.bi, S.e, xs);
+            const long long base = (long long)(S.p / kSlice) * W * kSlice + lane;
+            for (int k = U; k < W; k += U) {
+                GsEntries<U> e;
+                gs_load<false>(e, col + base, val + base, k, W, S.p);
+                t = gs_subtract(t, e, xs);
+            }
+            const int mode = kMixed ? prog.mode[S.pass] : mode0;
+            const double w = kMixed ? prog.w[S.pass] : w0;
+            xs[S.p] = gs_update(mode, t, S.d, xs[S.p], w);
+        }
+        if (++done == steps) {   // the same in every wave
+            done = 0;
+            lds_barrier();
+        }
+    };
+    Slice S[kGsAhead];
+#pragma unroll
+    for (int q = 0; q < kGsAhead; ++q) load(S[q]);
+    for (int idx = 0; idx < total; idx += kGsAhead)
+#pragma unroll
+        for (int q = 0; q < kGsAhead; ++q)
+            if (idx + q < total) {   // the same in every wave
+                compute(S[q]);
+                load(S[q]);
+            }
+    __syncthreads();
+    for (int p = threadIdx.x; p < npos; p += kThreads) {
+        const int i = rows[p];
+        if (i >= 0) xout[i] = xs[p];
+    }
 }
 
 }  // namespace
@@ -276,12 +452,17 @@ void gs_prepare(const DevCSR &A, GsLevel &G) {
     const int n = A.n;
     if (n == 0) return;
     hipStream_t st = stream();
-    // colouring on the pattern of A + A^T
-    DevCSR AT;
-    csr_transpose_gpu(A, AT);
+    // colouring on the pattern of A + A^T: A's own where that is symmetric
     int *c0 = arena().alloc_n<int>((size_t)n + 1);
     int *c1 = arena().alloc_n<int>((size_t)n + 1);
     int *left = arena().alloc_n<int>(1);
+    int h = 0;
+    HZ_CHECK(hipMemsetAsync(left, 0, sizeof(int), st));
+    k_gs_symmetric<<<grid_rows(n), kBlock, 0, st>>>(n, A.ia, A.ja, left);
+    HZ_LAUNCH_CHECK();
+    HZ_CHECK(memcpy_sync(&h, left, sizeof(int), hipMemcpyDeviceToHost));
+    DevCSR AT;
+    if (h) csr_transpose_gpu(A, AT);
     HZ_CHECK(hipMemsetAsync(c0, 0xff, sizeof(int) * n, st));
     // Rounds after the last one change nothing, so the count of uncoloured
     // rows is read back only every kCheck rounds.  Every round colours at
@@ -299,64 +480,68 @@ void gs_prepare(const DevCSR &A, GsLevel &G) {
         HZ_CHECK(memcpy_sync(&hl, left, sizeof(int), hipMemcpyDeviceToHost));
         if (hl == 0) break;
     }
-    std::vector<int> color(n), offd(n);
-    k_offdiag_count<<<grid_rows(n), kBlock, 0, st>>>(n, A.ia, A.ja, A.val, c1);
+    // rows by colour: a stable sort keeps them ascending inside a colour
+    int *info = arena().alloc_n<int>((size_t)n + 3);   // largest colour, widest row, then rows per colour
+    int *cnt = info + 2;
+    unsigned int *keys = arena().alloc_n<unsigned int>((size_t)n), *keys_out = arena().alloc_n<unsigned int>((size_t)n);
+    int *idx = arena().alloc_n<int>((size_t)n), *sorted = arena().alloc_n<int>((size_t)n);
+    HZ_CHECK(hipMemsetAsync(info, 0, sizeof(int) * ((size_t)n + 3), st));
+    k_color_hist<<<std::min(256, div_up(n, kBlock)), kBlock, 0, st>>>(n, c0, cnt, info, keys, idx);
     HZ_LAUNCH_CHECK();
-    HZ_CHECK(memcpy_sync(color.data(), c0, sizeof(int) * n, hipMemcpyDeviceToHost));
-    HZ_CHECK(memcpy_sync(offd.data(), c1, sizeof(int) * n, hipMemcpyDeviceToHost));
-    int nc = 0;
-    for (int v : color) nc = std::max(nc, v + 1);
+    const int first = std::min(n + 3, 258);
+    std::vector<int> hi(first);
+    HZ_CHECK(memcpy_sync(hi.data(), info, sizeof(int) * first, hipMemcpyDeviceToHost));
+    const int nc = hi[0] + 1;
+    if (nc + 2 > first) {
+        hi.resize((size_t)nc + 2);
+        HZ_CHECK(memcpy_sync(hi.data(), info, sizeof(int) * hi.size(), hipMemcpyDeviceToHost));
+    }
+    int bits = 1;
+    while ((1u << bits) < (unsigned)nc && bits < 32) ++bits;
+    size_t tmp_bytes = 0;
+    HZ_CHECK(rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys, keys_out, idx, sorted, (size_t)n, 0, bits, st));
+    void *tmp = arena().alloc(tmp_bytes);
+    HZ_CHECK(rocprim::radix_sort_pairs(tmp, tmp_bytes, keys, keys_out, idx, sorted, (size_t)n, 0, bits, st));
+    G.n = n;
     G.ncolors = nc;
     G.cptr.assign(nc + 1, 0);
-    for (int v : color) G.cptr[v + 1]++;
-    for (int c = 0; c < nc; ++c) G.cptr[c + 1] += G.cptr[c];
-    std::vector<int> rows(n), fillp(G.cptr.begin(), G.cptr.end() - 1);
-    for (int i = 0; i < n; ++i) rows[fillp[color[i]]++] = i;
-    // slices of each colour (diagonal entries are stored apart)
     G.sl0.assign(nc + 1, 0);
-    std::vector<int> spos, scnt;
-    std::vector<long long> sptr(1, 0);
+    G.most_slices = 0;
     for (int c = 0; c < nc; ++c) {
-        G.sl0[c] = (int)spos.size();
-        for (int p = G.cptr[c]; p < G.cptr[c + 1]; p += kSlice) {
-            const int cnt = std::min(kSlice, G.cptr[c + 1] - p);
-            int width = 0;
-            for (int t = 0; t < cnt; ++t) width = std::max(width, offd[rows[p + t]]);
-            spos.push_back(p);
-            scnt.push_back(cnt);
-            sptr.push_back(sptr.back() + (long long)width * kSlice);
-        }
+        const int ns = div_up(hi[2 + c], kSlice);
+        G.cptr[c + 1] = G.cptr[c] + hi[2 + c];
+        G.sl0[c + 1] = G.sl0[c] + ns;
+        G.most_slices = std::max(G.most_slices, ns);
     }
-    const int ns = (int)spos.size();
-    G.sl0[nc] = ns;
+    const int ns = G.sl0[nc];
     G.nslices = ns;
-    G.n = n;
-    G.rows = arena().alloc_n<int>((size_t)n + 1);
-    G.spos = arena().alloc_n<int>((size_t)ns + 1);
-    G.scnt = arena().alloc_n<int>((size_t)ns + 1);
-    G.sptr = arena().alloc_n<long long>((size_t)ns + 1);
-    G.diag = arena().alloc_n<double>((size_t)n + 1);
-    G.col = arena().alloc_n<int>((size_t)sptr.back() + 1);
-    G.val = arena().alloc_n<double>((size_t)sptr.back() + 1);
-    HZ_CHECK(memcpy_sync(G.rows, rows.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-    HZ_CHECK(memcpy_sync(G.spos, spos.data(), sizeof(int) * ns, hipMemcpyHostToDevice));
-    HZ_CHECK(memcpy_sync(G.scnt, scnt.data(), sizeof(int) * ns, hipMemcpyHostToDevice));
-    HZ_CHECK(memcpy_sync(G.sptr, sptr.data(), sizeof(long long) * (ns + 1), hipMemcpyHostToDevice));
+    G.npos = ns * kSlice;
+    G.order = sorted;
+    std::vector<int> tables(G.cptr);
+    tables.insert(tables.end(), G.sl0.begin(), G.sl0.end());
+    int *dtab = arena().alloc_n<int>(tables.size());
+    HZ_CHECK(hipMemcpyAsync(dtab, tables.data(), sizeof(int) * tables.size(), hipMemcpyHostToDevice, st));
+    G.dsl0 = dtab + nc + 1;
+    G.rows = arena().alloc_n<int>((size_t)G.npos);
+    int *width = arena().alloc_n<int>((size_t)ns);
     int *pos_of = c1;   // scratch: the colouring buffers are free now
-    k_pos_of<<<grid_rows(n), kBlock, 0, st>>>(n, G.rows, pos_of);
+    k_gs_place<<<div_up(ns, kSlicesPerBlock), kBlock, 0, st>>>(ns, nc, dtab, G.dsl0, sorted, A.ia, A.ja, A.val, G.rows,
+                                                                pos_of, width, info);
     HZ_LAUNCH_CHECK();
-    const long threads = (long)ns * kSlice;
-    k_gs_fill<<<div_up(threads, kBlock), kBlock, 0, st>>>(ns, G.spos, G.scnt, G.sptr, G.rows, pos_of, A.ia, A.ja,
-                                                          A.val, G.col, G.val, G.diag);
+    HZ_CHECK(memcpy_sync(&G.W, info + 1, sizeof(int), hipMemcpyDeviceToHost));
+    const size_t room = (size_t)G.npos * std::max(1, G.W);
+    G.diag = arena().alloc_n<double>((size_t)G.npos);
+    G.col = arena().alloc_n<int>(room);
+    G.val = arena().alloc_n<double>(room);
+    G.xp = arena().alloc_n<double>((size_t)G.npos);
+    G.bp = arena().alloc_n<double>((size_t)G.npos);
+    k_gs_fill<<<div_up(G.npos, kBlock), kBlock, 0, st>>>(ns, G.W, G.rows, pos_of, A.ia, A.ja, A.val, G.col, G.val,
+                                                         G.diag);
     HZ_LAUNCH_CHECK();
-    G.dsl0 = arena().alloc_n<int>((size_t)nc + 1);
-    HZ_CHECK(memcpy_sync(G.dsl0, G.sl0.data(), sizeof(int) * (nc + 1), hipMemcpyHostToDevice));
-    G.in_lds = n <= kGsLdsRows;
-    if (!G.in_lds) {
-        G.xp = arena().alloc_n<double>((size_t)n + 1);
-        G.bp = arena().alloc_n<double>((size_t)n + 1);
-    }
-    HZ_CHECK(hipStreamSynchronize(st));
+    // one workgroup where x and the rest fit LDS; else per-slice widths where
+    // the padding to the longest row is worth the load that skips it
+    G.in_lds = G.npos <= kGsLdsPos;
+    G.width = n > 65536 ? width : nullptr;
 }
 
 namespace {
@@ -417,29 +602,60 @@ std::vector<Pass> gs_program(int smoother, bool post, int L, double relax) {
     return prog;
 }
 
-void color_launch(const GsLevel &G, int c, int mode, double w) {
+void color_launch(const GsLevel &G, int c, int mode, double w, double *xout) {
     const int s0 = G.sl0[c], ns = G.sl0[c + 1] - G.sl0[c];
     if (ns == 0) return;
     const int grid = div_up(ns, kSlicesPerBlock);
-    hipStream_t st = stream();
-    if (mode == 0)
-        k_gs_color<0><<<grid, kBlock, 0, st>>>(s0, ns, G.spos, G.scnt, G.sptr, G.col, G.val, G.diag, G.bp, G.xp, w);
-    else if (mode == 1)
-        k_gs_color<1><<<grid, kBlock, 0, st>>>(s0, ns, G.spos, G.scnt, G.sptr, G.col, G.val, G.diag, G.bp, G.xp, w);
-    else
-        k_gs_color<2><<<grid, kBlock, 0, st>>>(s0, ns, G.spos, G.scnt, G.sptr, G.col, G.val, G.diag, G.bp, G.xp, w);
+    auto go = [&](auto m, auto u) {
+        constexpr int M = decltype(m)::value, U = decltype(u)::value;
+        if (G.width)
+            k_gs_color<M, U, true><<<grid, kBlock, 0, stream()>>>(s0, ns, G.W, G.width, G.rows, G.col, G.val, G.diag,
+                                                                  G.bp, G.xp, w, xout);
+        else
+            k_gs_color<M, U, false><<<grid, kBlock, 0, stream()>>>(s0, ns, G.W, G.width, G.rows, G.col, G.val, G.diag,
+                                                                   G.bp, G.xp, w, xout);
+    };
+    auto by_mode = [&](auto u) {
+        if (mode == 0) go(std::integral_constant<int, 0>{}, u);
+        else if (mode == 1) go(std::integral_constant<int, 1>{}, u);
+        else go(std::integral_constant<int, 2>{}, u);
+    };
+    if (G.W <= 8) by_mode(std::integral_constant<int, 8>{});
+    else by_mode(std::integral_constant<int, 16>{});
+}
+
+// The one-workgroup form: 16 waves with eight entries in flight for short
+// rows, 8 waves with sixteen for longer ones (registers).
+template <int U, int kThreads, bool kMixed>
+void lds_launch(const GsLevel &G, const double *b, const double *x, double *xout, const GsProgram &gp) {
+    static const bool ready = [] {
+        HZ_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gs_lds<U, kThreads, kMixed>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, kGsLdsPos * (int)sizeof(double)));
+        return true;
+    }();
+    (void)ready;
+    const int steps = std::max(1, div_up(G.most_slices, kThreads / kSlice));
+    k_gs_lds<U, kThreads, kMixed><<<1, kThreads, sizeof(double) * G.npos, stream()>>>(
+        G.npos, G.ncolors, G.W, steps, G.dsl0, G.rows, G.col, G.val, G.diag, G.bp, b, x, xout, gp);
+    HZ_LAUNCH_CHECK();
 }
 
 }  // namespace
 
-void gs_smooth(const GsLevel &G, int smoother, bool post, int nsweeps, double relax, const double *b, double *x) {
+void gs_smooth(const GsLevel &G, int smoother, bool post, int nsweeps, double relax, const double *b, double *x,
+               bool x_zero) {
     const std::vector<Pass> prog = gs_program(smoother, post, nsweeps, relax);
-    if (prog.empty() || G.n == 0) return;
+    if (G.n == 0) return;
+    if (prog.empty()) {
+        if (x_zero) fill(x, 0.0, G.n);
+        return;
+    }
     hipStream_t st = stream();
-    if (G.in_lds) {
-        for (size_t p0 = 0; p0 < prog.size(); p0 += kGsMaxPass) {
+    if (G.in_lds && G.ncolors <= kGsMaxPhase) {
+        const size_t per = std::max<size_t>(1, std::min<size_t>(kGsMaxPass, kGsMaxPhase / G.ncolors));
+        for (size_t p0 = 0; p0 < prog.size(); p0 += per) {
             GsProgram gp{};
-            gp.npass = (int)std::min<size_t>(kGsMaxPass, prog.size() - p0);
+            gp.npass = (int)std::min<size_t>(per, prog.size() - p0);
             for (int k = 0; k < gp.npass; ++k) {
                 const Pass &P = prog[p0 + k];
                 gp.forward[k] = P.forward;
@@ -447,18 +663,32 @@ void gs_smooth(const GsLevel &G, int smoother, bool post, int nsweeps, double re
                 gp.skip[k] = (P.skip && G.ncolors > 0) ? 1 : 0;
                 gp.w[k] = P.w;
             }
-            k_gs_lds<<<1, 1024, sizeof(double) * G.n, st>>>(G.n, G.ncolors, G.dsl0, G.spos, G.scnt, G.sptr, G.rows,
-                                                            G.col, G.val, G.diag, b, x, gp);
-            HZ_LAUNCH_CHECK();
+            const double *xin = x_zero && p0 == 0 ? nullptr : x;
+            bool mixed = false;
+            for (int k = 1; k < gp.npass; ++k) mixed = mixed || gp.mode[k] != gp.mode[0] || gp.w[k] != gp.w[0];
+            if (mixed) {
+                if (G.W <= 8) lds_launch<8, 1024, true>(G, b, xin, x, gp);
+                else lds_launch<16, 512, true>(G, b, xin, x, gp);
+            } else {
+                if (G.W <= 8) lds_launch<8, 1024, false>(G, b, xin, x, gp);
+                else lds_launch<16, 512, false>(G, b, xin, x, gp);
+            }
         }
         return;
     }
-    k_perm_in<<<grid_rows(G.n), kBlock, 0, st>>>(G.n, G.rows, x, b, G.xp, G.bp);
-    for (const Pass &P : prog) {
-        for (int q = P.skip ? 1 : 0; q < G.ncolors; ++q)
-            color_launch(G, P.forward ? q : G.ncolors - 1 - q, P.mode, P.w);
+    k_perm_in<<<grid_rows(G.npos), kBlock, 0, st>>>(G.npos, G.rows, x_zero ? nullptr : x, b, G.xp, G.bp);
+    HZ_LAUNCH_CHECK();
+    // a colour's last visit writes its rows of x as well
+    std::vector<int> last(G.ncolors, -1);
+    for (int k = 0; k < (int)prog.size(); ++k)
+        for (int q = prog[k].skip ? 1 : 0; q < G.ncolors; ++q) last[prog[k].forward ? q : G.ncolors - 1 - q] = k;
+    for (int k = 0; k < (int)prog.size(); ++k) {
+        const Pass &P = prog[k];
+        for (int q = P.skip ? 1 : 0; q < G.ncolors; ++q) {
+            const int c = P.forward ? q : G.ncolors - 1 - q;
+            color_launch(G, c, P.mode, P.w, last[c] == k ? x : nullptr);
+        }
     }
-    k_perm_out<<<grid_rows(G.n), kBlock, 0, st>>>(G.n, G.rows, G.xp, x);
     HZ_LAUNCH_CHECK();
 }
 

@@ -201,3 +201,38 @@ def test_coarse_gmres_after_small_cg_vs_oracle(lib, orc, m):
     so = orc.orc_pvgmres(Ah.ptr(), capi.dptr(b), capi.dptr(xo), 1e-8, 20 * n, 30)
     assert st_cg < 0 < st and abs(st - so) <= 2
     assert np.linalg.norm(x - xo) <= 1e-6 * np.linalg.norm(xo)
+
+
+# positions (64 per slice, colours padded): one workgroup up to 18,432, colour launches above; rows of up to 8, up to
+# 16 and over 16 off-diagonal entries; a nonsymmetric pattern; more than 65,536 rows: widths by slice
+@pytest.mark.parametrize("rows,per_row,symmetric", [(1, 0, True), (70, 6, True), (3000, 6, True), (3000, 14, True),
+                                                    (3000, 30, True), (3000, 8, False), (21000, 6, True),
+                                                    (21000, 20, False), (70001, 6, True)])
+@pytest.mark.parametrize("smoother", [capi.SMOOTHER_GS, capi.SMOOTHER_SGS, capi.SMOOTHER_SGSOR])
+def test_gauss_seidel_forms_bitexact(lib, orc, rows, per_row, symmetric, smoother):
+    """Smoothing calls (two sweeps, before and after the coarse correction) in the library's colour order, bit for bit
+    as the oracle sweeps the rows in that order, on every form that the level's size and rows choose."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(rows + per_row)
+    i = np.repeat(np.arange(rows), per_row // 2 if symmetric else per_row)
+    j = (i + rng.integers(1, max(2, min(rows, 300)), i.size)) % rows
+    off = sp.csr_matrix((rng.uniform(-1.0, 1.0, i.size), (i, j)), shape=(rows, rows))
+    if symmetric:
+        off = off + off.T
+    off.setdiag(0.0)
+    off.eliminate_zeros()
+    A = (off + sp.diags(1.0 + np.asarray(np.abs(off).sum(axis=1)).ravel())).tocsr()
+    A.sort_indices()
+    M = capi.HostCSR(A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data.astype(np.float64))
+    b, x0 = rng.standard_normal(rows), rng.standard_normal(rows)
+    for post in (0, 1):
+        order, cptr = np.zeros(rows, np.int32), np.zeros(rows + 2, np.int32)
+        nc = capi.INT()
+        xg = x0.copy()
+        assert lib.hz_gs_smooth(M.ptr(), capi.dptr(b), capi.dptr(xg), smoother, post, 2, 0.8, capi.dptr(order, capi.INT),
+                                capi.dptr(cptr, capi.INT), C.byref(nc)) == 0
+        xo = x0.copy()
+        orc.orc_gs_smooth_ordered(M.ptr(), capi.dptr(b), capi.dptr(xo), smoother, post, 2, 0.8,
+                                  capi.dptr(order, capi.INT), capi.dptr(cptr, capi.INT), nc.value)
+        assert np.array_equal(np.sort(order), np.arange(rows))
+        assert np.array_equal(xg, xo)
