@@ -242,7 +242,7 @@ int amg_setup(Hierarchy &H, const DevCSR &A0, AMG_param *param, bool) {
                 aggregate_features(L.A, L.agg, nagg, rp, rm, lvl, feat);
                 MlpWork w = mlp_work(nagg);
                 float *out = arena().alloc_n<float>((size_t)nagg * HZ_MLP_OUTPUTS + 1);
-                mlp_inputs(feat, nullptr, nagg, w);
+                mlp_inputs(feat, nagg, w);
                 mlp_forward(H.mlp_theta, w, nagg);
                 mlp_outputs(nagg, w, out);
                 float *om = arena().alloc_n<float>((size_t)nagg + 1);

@@ -983,7 +983,7 @@ INT hz_mlp_forward(const float *theta, const float *x, INT B, float *y) {
         const float *dx = upload(x, (size_t)B * HZ_MLP_INPUTS);
         MlpWork w = mlp_work(B);
         float *dy = arena().alloc_n<float>((size_t)B * HZ_MLP_OUTPUTS);
-        mlp_inputs(dx, nullptr, B, w);
+        mlp_inputs(dx, B, w);
         mlp_forward(dth, w, B);
         mlp_outputs(B, w, dy);
         HZ_CHECK(memcpy_sync(y, dy, sizeof(float) * B * HZ_MLP_OUTPUTS, hipMemcpyDeviceToHost));
@@ -1013,14 +1013,9 @@ INT hz_mlp_loss_grad(const float *theta, const float *x, const float *t, INT B, 
         const float *dth = upload(theta, HZ_MLP_PARAMS);
         const float *dx = upload(x, (size_t)B * HZ_MLP_INPUTS);
         const float *dt = upload(t, (size_t)B * HZ_MLP_OUTPUTS);
-        MlpWork w = mlp_work(B);
         float *dg = arena().alloc_n<float>(HZ_MLP_PARAMS);
         float *dl = arena().alloc_n<float>(1);
-        HZ_CHECK(hipMemsetAsync(dg, 0, sizeof(float) * HZ_MLP_PARAMS, stream()));
-        mlp_inputs(dx, nullptr, B, w);
-        mlp_targets(dt, nullptr, B, w);
-        mlp_forward(dth, w, B);
-        mlp_backward(dth, w, B, dg, dl);
+        mlp_loss_grad(dth, dx, dt, nullptr, B, mlp_grad_work(), dg, dl);
         HZ_CHECK(memcpy_sync(grad, dg, sizeof(float) * HZ_MLP_PARAMS, hipMemcpyDeviceToHost));
         HZ_CHECK(memcpy_sync(loss, dl, sizeof(float), hipMemcpyDeviceToHost));
         return HZ_SUCCESS;
@@ -1039,7 +1034,7 @@ INT hz_mlp_train(float *theta, const float *x, const float *t, INT B, INT epochs
         const float *dx = upload(x, (size_t)B * HZ_MLP_INPUTS);
         const float *dt = upload(t, (size_t)B * HZ_MLP_OUTPUTS);
         const int bs = std::min<int>(batch, B);
-        MlpWork w = mlp_work(std::max<int>(bs, B));
+        const MlpGradWork w = mlp_grad_work();
         float *dg = arena().alloc_n<float>(HZ_MLP_PARAMS);
         float *dm = arena().alloc_n<float>(HZ_MLP_PARAMS);
         float *dv = arena().alloc_n<float>(HZ_MLP_PARAMS);
@@ -1048,10 +1043,7 @@ INT hz_mlp_train(float *theta, const float *x, const float *t, INT B, INT epochs
         HZ_CHECK(hipMemsetAsync(dm, 0, sizeof(float) * HZ_MLP_PARAMS, stream()));
         HZ_CHECK(hipMemsetAsync(dv, 0, sizeof(float) * HZ_MLP_PARAMS, stream()));
         auto full_loss = [&]() {
-            mlp_inputs(dx, nullptr, B, w);
-            mlp_targets(dt, nullptr, B, w);
-            mlp_forward(dth, w, B);
-            mlp_backward(dth, w, B, dg, dl);
+            mlp_loss_grad(dth, dx, dt, nullptr, B, w, dg, dl);
             float l = 0.0f;
             HZ_CHECK(memcpy_sync(&l, dl, sizeof(float), hipMemcpyDeviceToHost));
             return l;
@@ -1072,10 +1064,7 @@ INT hz_mlp_train(float *theta, const float *x, const float *t, INT B, INT epochs
             HZ_CHECK(hipMemcpyAsync(didx, perm.data(), sizeof(int) * B, hipMemcpyHostToDevice, stream()));
             for (int o = 0; o < B; o += bs) {
                 const int nb = std::min(bs, B - o);
-                mlp_inputs(dx, didx + o, nb, w);
-                mlp_targets(dt, didx + o, nb, w);
-                mlp_forward(dth, w, nb);
-                mlp_backward(dth, w, nb, dg, dl);
+                mlp_loss_grad(dth, dx, dt, didx + o, nb, w, dg, dl);
                 mlp_adam(dth, dg, dm, dv, lr, ++step);
             }
             HZ_CHECK(hipStreamSynchronize(stream()));   // perm is reused next epoch

@@ -300,21 +300,24 @@ void aggregate_features(const DevCSR &A, const int *agg, int nagg, const int *rp
                         float *feat);
 
 // ---- kernels_mlp.hip: the per-aggregate parameter network -----------------
-constexpr int kMlpWgradBlocks = 256;
 struct MlpWork {
     int cap = 0;   // rows (multiple of 64)
-    float *X = nullptr, *Z1 = nullptr, *H1 = nullptr, *Z2 = nullptr, *H2 = nullptr, *Y = nullptr;
-    float *T = nullptr, *dY = nullptr, *dH = nullptr, *dZ = nullptr, *part = nullptr;
-    double *lpart = nullptr;
+    float *X = nullptr, *H1 = nullptr, *H2 = nullptr, *Y = nullptr;
 };
 MlpWork mlp_work(int capacity);
-// X = rows idx[0..B) (or 0..B) of x [.][12], padded
-void mlp_inputs(const float *x, const int *idx, int B, const MlpWork &w);
-void mlp_targets(const float *t, const int *idx, int B, const MlpWork &w);
+// X = rows 0..B of x [.][12], padded
+void mlp_inputs(const float *x, int B, const MlpWork &w);
 void mlp_forward(const float *theta, const MlpWork &w, int B);
 void mlp_outputs(int B, const MlpWork &w, float *y);   // y [B][2]
-// gradient of the loss w.r.t. theta (after mlp_forward with the same inputs) and the loss
-void mlp_backward(const float *theta, const MlpWork &w, int B, float *grad, float *loss);
+constexpr int kMlpGradBlocks = 256;   // one workgroup a CU
+struct MlpGradWork {
+    float *part = nullptr;
+    double *lpart = nullptr;
+};
+MlpGradWork mlp_grad_work();
+// loss and its gradient w.r.t. theta on rows idx[0..B) (idx null: 0..B) of x [.][12] and t [.][2]
+void mlp_loss_grad(const float *theta, const float *x, const float *t, const int *idx, int B, const MlpGradWork &w,
+                   float *grad, float *loss);
 void mlp_adam(float *theta, const float *grad, float *m, float *v, float lr, int step);
 // Forward pass with device x, y and theta through the static scratch array,
 // queued on st; no device memory is allocated.  B <= HZ_MLP_NOALLOC_MAX_ROWS.

@@ -39,26 +39,18 @@ constexpr int kRows = 64;   // batch rows per tile
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float gelu(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
-__device__ __forceinline__ float gelu_grad(float z) {
-    const float cdf = 0.5f * (1.0f + erff(z * 0.70710678118654752f));
-    const float pdf = 0.39894228040143268f * expf(-0.5f * z * z);
-    return cdf + z * pdf;
-}
 
-enum Epi { kEpiNone = 0, kEpiGelu = 1, kEpiGeluGrad = 2 };
+enum Epi { kEpiNone = 0, kEpiGelu = 1 };
 
-// C[M x N] = A[M x K] * op(B) (+ bias), K <= 64, N <= 64; op(B) = B [K x N] or
-// B^T with B stored [N x K].  One workgroup (4 wavefronts) per 64-row tile;
-// wavefront w owns rows 16w..16w+15 and all N columns as 16x16 MFMA blocks.
-// Epilogues: kEpiGelu stores Z = acc + bias and C = gelu(Z); kEpiGeluGrad
-// stores C = acc * gelu'(Zin).
+// C[M x N] = A[M x K] B + bias, K <= 64, N <= 64 (the forward pass).  One
+// workgroup (4 wavefronts) per 64-row tile; wavefront w owns rows 16w..16w+15
+// and all N columns as 16x16 MFMA blocks.  Epilogue kEpiGelu: C = gelu(C).
 // MFMA f32 16x16x4 lanes: A[lane % 16][k + lane / 16], B[k + lane / 16][lane % 16],
 // accumulator element r = D[4 (lane / 16) + r][lane % 16].
-template <bool kTransB, int kEpi>
+template <int kEpi>
 __global__ __launch_bounds__(256) void k_mlp_gemm(int M, int N, int K, const float *__restrict__ A,
                                                   const float *__restrict__ B, const float *__restrict__ bias,
-                                                  float *__restrict__ C, float *__restrict__ Z,
-                                                  const float *__restrict__ Zin) {
+                                                  float *__restrict__ C) {
     __shared__ float As[kRows][65];
     __shared__ float Bs[64][65];
     const int r0 = blockIdx.x * kRows;
@@ -69,9 +61,7 @@ __global__ __launch_bounds__(256) void k_mlp_gemm(int M, int N, int K, const flo
     }
     for (int e = tid; e < 64 * 64; e += 256) {
         const int k = e / 64, c = e % 64;
-        float v = 0.0f;
-        if (k < K && c < N) v = kTransB ? B[(size_t)c * K + k] : B[(size_t)k * N + c];
-        Bs[k][c] = v;
+        Bs[k][c] = k < K && c < N ? B[(size_t)k * N + c] : 0.0f;
     }
     __syncthreads();
     const int w = tid / kWave, lane = tid % kWave;
@@ -91,107 +81,246 @@ __global__ __launch_bounds__(256) void k_mlp_gemm(int M, int N, int K, const flo
             const int row = r0 + 16 * w + 4 * (lane / 16) + r;
             const int col = 16 * j + lane % 16;
             if (row >= M || col >= N) continue;
-            const size_t o = (size_t)row * N + col;
-            float v = acc[j][r];
-            if (kEpi == kEpiGeluGrad) {
-                C[o] = v * gelu_grad(Zin[o]);
-            } else {
-                if (bias) v += bias[col];
-                if (kEpi == kEpiGelu) {
-                    if (Z) Z[o] = v;   // kept for the backward pass; null in a forward-only pass
-                    C[o] = gelu(v);
-                } else {
-                    C[o] = v;
-                }
-            }
+            const float v = acc[j][r] + bias[col];
+            C[(size_t)row * N + col] = kEpi == kEpiGelu ? gelu(v) : v;
         }
 }
 
-// Weight gradient partials: part[g] = sum over the rows of this workgroup's
-// tiles of A^T D, A [M x KA], D [M x ND], KA, ND <= 64; plus column sums of D
-// (bias gradient) in part[g][KA*ND ...].  The output tile (KA x ND) is split
-// over the 4 wavefronts by 16-row bands of KA.
-__global__ __launch_bounds__(256) void k_mlp_wgrad(int M, int KA, int ND, const float *__restrict__ A,
-                                                   const float *__restrict__ D, float *__restrict__ part) {
-    __shared__ float As[kRows][65];
-    __shared__ float Ds[kRows][65];
-    const int tid = threadIdx.x;
-    const int w = tid / kWave, lane = tid % kWave;
-    const int nb = (ND + 15) / 16;
-    f4 acc[4];
-    for (int j = 0; j < 4; ++j) acc[j] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-    float csum = 0.0f;   // column sums: thread t < ND owns column t
-    const int ntiles = (M + kRows - 1) / kRows;
-    for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
-        const int r0 = t * kRows;
-        __syncthreads();
-        for (int e = tid; e < kRows * 64; e += 256) {
-            const int r = e / 64, c = e % 64;
-            const bool ok = r0 + r < M;
-            As[r][c] = (ok && c < KA) ? A[(size_t)(r0 + r) * KA + c] : 0.0f;
-            Ds[r][c] = (ok && c < ND) ? D[(size_t)(r0 + r) * ND + c] : 0.0f;
-        }
-        __syncthreads();
-        if (16 * w < KA) {
-            // C[i][j] += sum_b A[b][i] D[b][j]: MFMA A operand = A^T (rows i), K = batch rows
-            for (int ks = 0; ks < kRows; ks += 4) {
-                const float a = As[ks + lane / 16][16 * w + lane % 16];
-                for (int j = 0; j < nb; ++j) {
-                    const float b = Ds[ks + lane / 16][16 * j + lane % 16];
-                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc[j], 0, 0, 0);
-                }
-            }
-        }
-        if (tid < ND)
-            for (int r = 0; r < kRows; ++r) csum += Ds[r][tid];
+// Loss and gradient partials of the network in one pass over the batch.
+//
+// Layer by layer this read and wrote eight 64-column activations a row (2 KB of
+// traffic for 56 bytes of input) in eleven launches, and the sums over partials
+// ran on 17 blocks and one thread.  The whole network is 25 KB, so a workgroup
+// keeps it in LDS and takes its 64-row tiles through forward and backward
+// there: only inputs and targets are read, and a workgroup's 6,288 gradient
+// sums, held in MFMA accumulators over its tiles, are written once.  96 KB of
+// LDS: one workgroup a CU, eight wavefronts to cover each other's LDS reads
+// and erf chains (four took 104 us).  84,400 rows: 877 -> 82 us of kernels.
+//
+// Wavefront wave = w + 4 half owns rows 16w..16w+15 and the column half `half`
+// of a tile's activations and of gW2; gW1 (columns 16w..) and the outputs go to
+// half 0, gW3 (rows 16w..) to half 1.  G1, G2 first hold gelu'(Z) and then dZ.
+// Rows past the batch have dY = 0 and add nothing.  MFMA lanes as in k_mlp_gemm.
+constexpr int kGradThreads = 512;
+struct GradTile {
+    float W1[kIn][kHid + 1], W2[kHid][kHid + 1], W3[kHid][kOut + 1];
+    float b1[kHid], b2[kHid], b3[kOut];
+    float X[kRows][kIn + 1], D[kRows][kOut + 1];
+    float H1[kRows][kHid + 1], H2[kRows][kHid + 1], G1[kRows][kHid + 1], G2[kRows][kHid + 1];
+};
+
+// gelu(z) and its derivative from one erf: 0.5 z (1 + e) and 0.5 (1 + e) + z pdf
+__device__ __forceinline__ void gelu_both(float z, float &h, float &g) {
+    const float cdf = 0.5f * (1.0f + erff(z * 0.70710678118654752f));
+    h = z * cdf;
+    g = cdf + z * (0.39894228040143268f * expf(-0.5f * z * z));
+}
+
+__global__ __launch_bounds__(kGradThreads) void k_mlp_grad(int B, const float *__restrict__ theta, const float *__restrict__ x,
+                                                  const float *__restrict__ t, const int *__restrict__ idx,
+                                                  float *__restrict__ part, double *__restrict__ lpart) {
+    extern __shared__ double s_tile[];
+    GradTile &S = *reinterpret_cast<GradTile *>(s_tile);
+    __shared__ double sh[kGradThreads / kWave];
+    const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave;
+    const int w = wave % 4, half = wave / 4, j0 = 2 * half;
+    const int lm = lane % 16, lk = lane / 16;
+    for (int e = tid; e < kIn * kHid; e += kGradThreads) S.W1[e / kHid][e % kHid] = theta[kOffW1 + e];
+    for (int e = tid; e < kHid * kHid; e += kGradThreads) S.W2[e / kHid][e % kHid] = theta[kOffW2 + e];
+    for (int e = tid; e < kHid * kOut; e += kGradThreads) S.W3[e / kOut][e % kOut] = theta[kOffW3 + e];
+    if (tid < kHid) {
+        S.b1[tid] = theta[kOffB1 + tid];
+        S.b2[tid] = theta[kOffB2 + tid];
     }
-    float *out = part + (size_t)blockIdx.x * (KA * ND + ND);
-    if (16 * w < KA)
-        for (int j = 0; j < nb; ++j)
+    if (tid < kOut) S.b3[tid] = theta[kOffB3 + tid];
+    const f4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f4 gW1 = zero, gW3 = zero, gW2[2] = {zero, zero};
+    // bias gradients: thread's column tid % 64 (tid % 16), rows of its part
+    float gb1 = 0.0f, gb2 = 0.0f, gb3 = 0.0f;
+    double loss = 0.0;
+    const float scale = 1.0f / (2.0f * (float)B);
+    const int ntiles = (B + kRows - 1) / kRows;
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int r0 = tile * kRows;
+        __syncthreads();   // weights are there; the last tile's readers of X and G1 are done
+        for (int e = tid; e < kRows * kIn; e += kGradThreads) {
+            const int r = e / kIn, c = e % kIn;
+            float v = 0.0f;
+            if (r0 + r < B && c < HZ_MLP_INPUTS) v = x[(size_t)(idx ? idx[r0 + r] : r0 + r) * HZ_MLP_INPUTS + c];
+            S.X[r][c] = v;
+        }
+        float tv[4] = {0.0f, 0.0f, 0.0f, 0.0f};   // targets of this lane's outputs
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = r0 + 16 * w + 4 * lk + r;
+            if (row < B && lm < HZ_MLP_OUTPUTS) tv[r] = t[(size_t)(idx ? idx[row] : row) * HZ_MLP_OUTPUTS + lm];
+        }
+        __syncthreads();
+        f4 acc[2];
+        // layer 1
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[j] = zero;
+#pragma unroll
+        for (int ks = 0; ks < kIn; ks += 4) {
+            const float a = S.X[16 * w + lm][ks + lk];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, S.W1[ks + lk][16 * (j0 + j) + lm], acc[j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const int i = 16 * w + 4 * (lane / 16) + r;
-                const int c = 16 * j + lane % 16;
-                if (i < KA && c < ND) out[i * ND + c] = acc[j][r];
+                const int row = 16 * w + 4 * lk + r, col = 16 * (j0 + j) + lm;
+                gelu_both(acc[j][r] + S.b1[col], S.H1[row][col], S.G1[row][col]);
             }
-    if (tid < ND) out[KA * ND + tid] = csum;
-}
-
-// grad[o + e] = sum over partials g (in order) of part[g][e]
-__global__ void k_mlp_reduce(int G, int len, const float *__restrict__ part, float *__restrict__ out) {
-    for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < len; e += gridDim.x * blockDim.x) {
-        float s = 0.0f;
-        for (int g = 0; g < G; ++g) s += part[(size_t)g * len + e];
-        out[e] = s;
-    }
-}
-
-// dY = 2 (Y - T) w / (2 * nvalid) on the two outputs, 0 elsewhere; per-block loss partials
-__global__ __launch_bounds__(256) void k_mlp_dloss(int M, int nvalid, const float *__restrict__ Y,
-                                                   const float *__restrict__ T, float *__restrict__ dY,
-                                                   double *__restrict__ lpart) {
-    __shared__ double sh[256 / kWave];
-    double l = 0.0;
-    const float scale = 1.0f / (2.0f * (float)nvalid);
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < M * kOut; i += gridDim.x * blockDim.x) {
-        const int row = i / kOut, o = i % kOut;
-        float g = 0.0f;
-        if (row < nvalid && o < HZ_MLP_OUTPUTS) {
-            const float d = Y[i] - T[row * HZ_MLP_OUTPUTS + o];
-            g = 2.0f * d * scale;
-            l += (double)d * (double)d;
+        __syncthreads();
+        // layer 2
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[j] = zero;
+#pragma unroll 4
+        for (int ks = 0; ks < kHid; ks += 4) {
+            const float a = S.H1[16 * w + lm][ks + lk];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, S.W2[ks + lk][16 * (j0 + j) + lm], acc[j], 0, 0, 0);
         }
-        dY[i] = g;
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * w + 4 * lk + r, col = 16 * (j0 + j) + lm;
+                gelu_both(acc[j][r] + S.b2[col], S.H2[row][col], S.G2[row][col]);
+            }
+        __syncthreads();
+        // layer 3, dY = 2 (Y - T) / (2 B)
+        if (half == 0) {
+            acc[0] = zero;
+#pragma unroll 4
+            for (int ks = 0; ks < kHid; ks += 4)
+                acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(S.H2[16 * w + lm][ks + lk], S.W3[ks + lk][lm], acc[0], 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = 16 * w + 4 * lk + r;
+                float g = 0.0f;
+                if (r0 + row < B && lm < HZ_MLP_OUTPUTS) {
+                    const float d = acc[0][r] + S.b3[lm] - tv[r];
+                    g = 2.0f * d * scale;
+                    loss += (double)d * (double)d;
+                }
+                S.D[row][lm] = g;
+            }
+        }
+        __syncthreads();
+        // gW3 += H2^T dY;  dZ2 = (dY W3^T) gelu'(Z2), own rows of G2
+        if (half == 1)
+#pragma unroll 4
+            for (int ks = 0; ks < kRows; ks += 4)
+                gW3 = __builtin_amdgcn_mfma_f32_16x16x4f32(S.H2[ks + lk][16 * w + lm], S.D[ks + lk][lm], gW3, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[j] = zero;
+#pragma unroll
+        for (int ks = 0; ks < kOut; ks += 4) {
+            const float a = S.D[16 * w + lm][ks + lk];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, S.W3[16 * (j0 + j) + lm][ks + lk], acc[j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S.G2[16 * w + 4 * lk + r][16 * (j0 + j) + lm] *= acc[j][r];
+        if (tid < 4 * kOut)
+            for (int r = 0; r < kRows / 4; ++r) gb3 += S.D[tid / kOut * (kRows / 4) + r][tid % kOut];
+        __syncthreads();
+        // gW2 += H1^T dZ2;  dZ1 = (dZ2 W2^T) gelu'(Z1), own rows of G1
+#pragma unroll 4
+        for (int ks = 0; ks < kRows; ks += 4) {
+            const float a = S.H1[ks + lk][16 * w + lm];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                gW2[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, S.G2[ks + lk][16 * (j0 + j) + lm], gW2[j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[j] = zero;
+#pragma unroll 4
+        for (int ks = 0; ks < kHid; ks += 4) {
+            const float a = S.G2[16 * w + lm][ks + lk];
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, S.W2[16 * (j0 + j) + lm][ks + lk], acc[j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S.G1[16 * w + 4 * lk + r][16 * (j0 + j) + lm] *= acc[j][r];
+#pragma unroll 4
+        for (int r = 0; r < kRows / 8; ++r) gb2 += S.G2[wave * (kRows / 8) + r][lane];
+        __syncthreads();
+        // gW1 += X^T dZ1
+        if (half == 0)
+#pragma unroll 4
+            for (int ks = 0; ks < kRows; ks += 4)
+                gW1 = __builtin_amdgcn_mfma_f32_16x16x4f32(S.X[ks + lk][lm], S.G1[ks + lk][16 * w + lm], gW1, 0, 0, 0);
+#pragma unroll 4
+        for (int r = 0; r < kRows / 8; ++r) gb1 += S.G1[wave * (kRows / 8) + r][lane];
     }
-    const double bs = block_sum<256>(l, sh);
-    if (threadIdx.x == 0) lpart[blockIdx.x] = bs;
+    float *out = part + (size_t)blockIdx.x * kParams;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (half == 0) out[kOffW1 + (4 * lk + r) * kHid + 16 * w + lm] = gW1[r];
+        else out[kOffW3 + (16 * w + 4 * lk + r) * kOut + lm] = gW3[r];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) out[kOffW2 + (16 * w + 4 * lk + r) * kHid + 16 * (j0 + j) + lm] = gW2[j][r];
+    }
+    // the bias sums' parts meet in LDS
+    __syncthreads();
+    S.H1[wave][lane] = gb1;
+    S.H2[wave][lane] = gb2;
+    if (tid < 4 * kOut) S.D[tid / kOut][tid % kOut] = gb3;
+    __syncthreads();
+    if (tid < kHid) {
+        float v1 = 0.0f, v2 = 0.0f;
+        for (int q = 0; q < kGradThreads / kWave; ++q) {
+            v1 += S.H1[q][tid];
+            v2 += S.H2[q][tid];
+        }
+        out[kOffB1 + tid] = v1;
+        out[kOffB2 + tid] = v2;
+    }
+    if (tid < kOut) out[kOffB3 + tid] = S.D[0][tid] + S.D[1][tid] + S.D[2][tid] + S.D[3][tid];
+    const double bs = block_sum<kGradThreads>(loss, sh);
+    if (tid == 0) lpart[blockIdx.x] = bs;
 }
 
-__global__ void k_mlp_loss_final(int G, int nvalid, const double *__restrict__ lpart, float *__restrict__ loss) {
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int g = 0; g < G; ++g) s += lpart[g];
-        *loss = (float)(s / (2.0 * nvalid));
+// grad[e] = sum over the G partials, a wavefront per quarter of them and 64
+// entries a workgroup; the last workgroup forms the loss.
+__global__ __launch_bounds__(256) void k_mlp_reduce(int G, int nvalid, const float *__restrict__ part,
+                                                    const double *__restrict__ lpart, float *__restrict__ out,
+                                                    float *__restrict__ loss) {
+    __shared__ float s[4][kWave];
+    __shared__ double sh[256 / kWave];
+    const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    if (blockIdx.x == gridDim.x - 1) {
+        const double tot = final_sum<256>(lpart, G, sh);
+        if (threadIdx.x == 0) *loss = (float)(tot / (2.0 * nvalid));
+        return;
     }
+    const int e = blockIdx.x * kWave + lane;
+    const int per = (G + 3) / 4, g1 = min(G, (w + 1) * per);
+    float v = 0.0f;
+    constexpr int U = 16;
+    if (e < kParams)
+        for (int g = w * per; g < g1; g += U) {
+            float a[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) a[u] = g + u < g1 ? part[(size_t)(g + u) * kParams + e] : 0.0f;
+#pragma unroll
+            for (int u = 0; u < U; ++u) v += a[u];
+        }
+    s[w][lane] = v;
+    __syncthreads();
+    if (w == 0 && e < kParams) out[e] = s[0][lane] + s[1][lane] + s[2][lane] + s[3][lane];
 }
 
 __global__ void k_mlp_adam(int n, float *__restrict__ th, const float *__restrict__ g, float *__restrict__ m,
@@ -207,21 +336,12 @@ __global__ void k_mlp_adam(int n, float *__restrict__ th, const float *__restric
 }
 
 // padded input rows: x[b][0..11], zeros in 12..15 and in padded rows
-__global__ void k_mlp_pad_inputs(int B, int M, const float *__restrict__ x, const int *__restrict__ idx,
-                                 float *__restrict__ X) {
+__global__ void k_mlp_pad_inputs(int B, int M, const float *__restrict__ x, float *__restrict__ X) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < M * kIn; i += gridDim.x * blockDim.x) {
         const int row = i / kIn, c = i % kIn;
         float v = 0.0f;
-        if (row < B && c < HZ_MLP_INPUTS) v = x[(size_t)(idx ? idx[row] : row) * HZ_MLP_INPUTS + c];
+        if (row < B && c < HZ_MLP_INPUTS) v = x[(size_t)row * HZ_MLP_INPUTS + c];
         X[i] = v;
-    }
-}
-
-__global__ void k_mlp_gather_targets(int B, const float *__restrict__ t, const int *__restrict__ idx,
-                                     float *__restrict__ T) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < B * HZ_MLP_OUTPUTS; i += gridDim.x * blockDim.x) {
-        const int row = i / HZ_MLP_OUTPUTS, o = i % HZ_MLP_OUTPUTS;
-        T[i] = t[(size_t)(idx ? idx[row] : row) * HZ_MLP_OUTPUTS + o];
     }
 }
 
@@ -239,17 +359,9 @@ MlpWork mlp_work(int capacity) {
     w.cap = (capacity + kRows - 1) / kRows * kRows;
     const size_t M = (size_t)w.cap;
     w.X = arena().alloc_n<float>(M * kIn);
-    w.Z1 = arena().alloc_n<float>(M * kHid);
     w.H1 = arena().alloc_n<float>(M * kHid);
-    w.Z2 = arena().alloc_n<float>(M * kHid);
     w.H2 = arena().alloc_n<float>(M * kHid);
     w.Y = arena().alloc_n<float>(M * kOut);
-    w.T = arena().alloc_n<float>(M * HZ_MLP_OUTPUTS + 1);
-    w.dY = arena().alloc_n<float>(M * kOut);
-    w.dH = arena().alloc_n<float>(M * kHid);
-    w.dZ = arena().alloc_n<float>(M * kHid);
-    w.part = arena().alloc_n<float>((size_t)kMlpWgradBlocks * (kHid * kHid + kHid));
-    w.lpart = arena().alloc_n<double>(4096);
     return w;
 }
 
@@ -257,18 +369,15 @@ void mlp_forward(const float *theta, const MlpWork &w, int B) {
     hipStream_t st = stream();
     const int M = (B + kRows - 1) / kRows * kRows;
     const int g = M / kRows;
-    k_mlp_gemm<false, kEpiGelu><<<g, 256, 0, st>>>(M, kHid, kIn, w.X, theta + kOffW1, theta + kOffB1, w.H1, w.Z1,
-                                                   nullptr);
-    k_mlp_gemm<false, kEpiGelu><<<g, 256, 0, st>>>(M, kHid, kHid, w.H1, theta + kOffW2, theta + kOffB2, w.H2, w.Z2,
-                                                   nullptr);
-    k_mlp_gemm<false, kEpiNone><<<g, 256, 0, st>>>(M, kOut, kHid, w.H2, theta + kOffW3, theta + kOffB3, w.Y,
-                                                   nullptr, nullptr);
+    k_mlp_gemm<kEpiGelu><<<g, 256, 0, st>>>(M, kHid, kIn, w.X, theta + kOffW1, theta + kOffB1, w.H1);
+    k_mlp_gemm<kEpiGelu><<<g, 256, 0, st>>>(M, kHid, kHid, w.H1, theta + kOffW2, theta + kOffB2, w.H2);
+    k_mlp_gemm<kEpiNone><<<g, 256, 0, st>>>(M, kOut, kHid, w.H2, theta + kOffW3, theta + kOffB3, w.Y);
     HZ_LAUNCH_CHECK();
 }
 
-void mlp_inputs(const float *x, const int *idx, int B, const MlpWork &w) {
+void mlp_inputs(const float *x, int B, const MlpWork &w) {
     const int M = (B + kRows - 1) / kRows * kRows;
-    k_mlp_pad_inputs<<<gsz((long)M * kIn), 256, 0, stream()>>>(B, M, x, idx, w.X);
+    k_mlp_pad_inputs<<<gsz((long)M * kIn), 256, 0, stream()>>>(B, M, x, w.X);
     HZ_LAUNCH_CHECK();
 }
 
@@ -277,34 +386,25 @@ void mlp_outputs(int B, const MlpWork &w, float *y) {
     HZ_LAUNCH_CHECK();
 }
 
-void mlp_targets(const float *t, const int *idx, int B, const MlpWork &w) {
-    k_mlp_gather_targets<<<gsz((long)B * 2), 256, 0, stream()>>>(B, t, idx, w.T);
-    HZ_LAUNCH_CHECK();
+MlpGradWork mlp_grad_work() {
+    MlpGradWork w;
+    w.part = arena().alloc_n<float>((size_t)kMlpGradBlocks * kParams);
+    w.lpart = arena().alloc_n<double>(kMlpGradBlocks);
+    return w;
 }
 
-void mlp_backward(const float *theta, const MlpWork &w, int B, float *grad, float *loss) {
-    hipStream_t st = stream();
-    const int M = (B + kRows - 1) / kRows * kRows;
-    const int g = M / kRows;
-    const int gl = gsz((long)M * kOut);
-    k_mlp_dloss<<<gl, 256, 0, st>>>(M, B, w.Y, w.T, w.dY, w.lpart);
-    k_mlp_loss_final<<<1, 64, 0, st>>>(gl, B, w.lpart, loss);
-    const int gw = std::min(kMlpWgradBlocks, g);
-    auto wgrad = [&](int KA, int ND, const float *A, const float *D, float *gW) {
-        k_mlp_wgrad<<<gw, 256, 0, st>>>(M, KA, ND, A, D, w.part);
-        const int len = KA * ND + ND;   // weights then bias (contiguous in theta)
-        k_mlp_reduce<<<gsz(len), 256, 0, st>>>(gw, len, w.part, gW);
-    };
-    // layer 3
-    wgrad(kHid, kOut, w.H2, w.dY, grad + kOffW3);
-    k_mlp_gemm<true, kEpiGeluGrad><<<g, 256, 0, st>>>(M, kHid, kOut, w.dY, theta + kOffW3, nullptr, w.dZ,
-                                                      nullptr, w.Z2);
-    // layer 2
-    wgrad(kHid, kHid, w.H1, w.dZ, grad + kOffW2);
-    k_mlp_gemm<true, kEpiGeluGrad><<<g, 256, 0, st>>>(M, kHid, kHid, w.dZ, theta + kOffW2, nullptr, w.dH,
-                                                      nullptr, w.Z1);
-    // layer 1
-    wgrad(kIn, kHid, w.X, w.dH, grad + kOffW1);
+void mlp_loss_grad(const float *theta, const float *x, const float *t, const int *idx, int B, const MlpGradWork &w,
+                   float *grad, float *loss) {
+    static const bool ready = [] {
+        HZ_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_mlp_grad),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(GradTile)));
+        return true;
+    }();
+    (void)ready;
+    const int G = std::min(kMlpGradBlocks, (B + kRows - 1) / kRows);
+    k_mlp_grad<<<G, kGradThreads, sizeof(GradTile), stream()>>>(B, theta, x, t, idx, w.part, w.lpart);
+    HZ_LAUNCH_CHECK();
+    k_mlp_reduce<<<(kParams + kWave - 1) / kWave + 1, 256, 0, stream()>>>(G, B, w.part, w.lpart, grad, loss);
     HZ_LAUNCH_CHECK();
 }
 
@@ -337,13 +437,10 @@ int mlp_forward_noalloc(const float *theta, const float *x, int B, float *y, hip
     float *Y = H2 + (size_t)kNoAllocRows * kHid;
     const int M = (B + kRows - 1) / kRows * kRows;
     const int g = M / kRows;
-    k_mlp_pad_inputs<<<gsz((long)M * kIn), 256, 0, st>>>(B, M, x, nullptr, X);
-    k_mlp_gemm<false, kEpiGelu><<<g, 256, 0, st>>>(M, kHid, kIn, X, theta + kOffW1, theta + kOffB1, H1, nullptr,
-                                                   nullptr);
-    k_mlp_gemm<false, kEpiGelu><<<g, 256, 0, st>>>(M, kHid, kHid, H1, theta + kOffW2, theta + kOffB2, H2, nullptr,
-                                                   nullptr);
-    k_mlp_gemm<false, kEpiNone><<<g, 256, 0, st>>>(M, kOut, kHid, H2, theta + kOffW3, theta + kOffB3, Y, nullptr,
-                                                   nullptr);
+    k_mlp_pad_inputs<<<gsz((long)M * kIn), 256, 0, st>>>(B, M, x, X);
+    k_mlp_gemm<kEpiGelu><<<g, 256, 0, st>>>(M, kHid, kIn, X, theta + kOffW1, theta + kOffB1, H1);
+    k_mlp_gemm<kEpiGelu><<<g, 256, 0, st>>>(M, kHid, kHid, H1, theta + kOffW2, theta + kOffB2, H2);
+    k_mlp_gemm<kEpiNone><<<g, 256, 0, st>>>(M, kOut, kHid, H2, theta + kOffW3, theta + kOffB3, Y);
     k_mlp_take_outputs<<<gsz((long)B * 2), 256, 0, st>>>(B, Y, y);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {

@@ -236,3 +236,43 @@ def test_gauss_seidel_forms_bitexact(lib, orc, rows, per_row, symmetric, smoothe
                                   capi.dptr(order, capi.INT), capi.dptr(cptr, capi.INT), nc.value)
         assert np.array_equal(np.sort(order), np.arange(rows))
         assert np.array_equal(xg, xo)
+
+
+# tiles of 64 rows over 256 workgroups: fewer tiles than workgroups, as many, one more, and several a workgroup with a
+# last tile of one row
+@pytest.mark.parametrize("B", [65, 16384, 16385, 40001])
+def test_mlp_gradient_tiles_vs_fp64(lib, B):
+    """Loss and gradient against the same network in FP64: sums of B terms in FP32 over at most 256 partials are within
+    2e-5 of the gradient's norm (64-row tiles: 2^-24 times a few hundred roundings)."""
+    from scipy.special import erf
+    rng = np.random.default_rng(B)
+    th = np.zeros(capi.MLP_PARAMS, np.float32)
+    lib.hz_mlp_init(capi.fptr(th), 3)
+    X = rng.standard_normal((B, capi.MLP_INPUTS)).astype(np.float32)
+    T = rng.standard_normal((B, capi.MLP_OUTPUTS)).astype(np.float32)
+    grad, loss = np.zeros(capi.MLP_PARAMS, np.float32), np.zeros(1, np.float32)
+    assert lib.hz_mlp_loss_grad(capi.fptr(th), capi.fptr(X), capi.fptr(T), B, capi.fptr(grad), capi.fptr(loss)) == 0
+    t = th.astype(np.float64)
+    o = np.cumsum([0, 16 * 64, 64, 64 * 64, 64, 64 * 16, 16])
+    W1, b1, W2, b2, W3, b3 = (t[o[k]:o[k + 1]] for k in range(6))
+    W1, W2, W3 = W1.reshape(16, 64), W2.reshape(64, 64), W3.reshape(64, 16)
+    x = np.pad(X.astype(np.float64), ((0, 0), (0, 4)))
+
+    def cdf(z):
+        return 0.5 * (1.0 + erf(z / np.sqrt(2.0)))
+
+    def dgelu(z):
+        return cdf(z) + z * np.exp(-0.5 * z * z) / np.sqrt(2.0 * np.pi)
+    z1 = x @ W1 + b1
+    h1 = z1 * cdf(z1)
+    z2 = h1 @ W2 + b2
+    h2 = z2 * cdf(z2)
+    d = (h2 @ W3 + b3)[:, :2] - T
+    dy = np.zeros((B, 16))
+    dy[:, :2] = d / B
+    dz2 = (dy @ W3.T) * dgelu(z2)
+    dz1 = (dz2 @ W2.T) * dgelu(z1)
+    ref = np.concatenate([(x.T @ dz1).ravel(), dz1.sum(0), (h1.T @ dz2).ravel(), dz2.sum(0), (h2.T @ dy).ravel(),
+                          dy.sum(0)])
+    assert np.linalg.norm(grad - ref) < 2e-5 * np.linalg.norm(ref)
+    assert abs(loss[0] - (d ** 2).mean()) < 2e-6 * (d ** 2).mean()
