@@ -56,7 +56,11 @@ static_assert(kR == HZ_BATCH_RHS, "C ABI batch width");
 static_assert(kR == 8, "the kernels split the right-hand sides into float4 / double2 groups");
 constexpr int kBlock = 256;
 constexpr int kSlicesPerBlock = kBlock / kWave;
-constexpr int kChunkRows = 2048;       // level-0 rows per reduction chunk (never across systems)
+// level-0 rows per reduction chunk (never across systems).  A chunk is one
+// workgroup's 16 double2 a thread, loaded four at a time; at 2,048 rows, one
+// double at a time, the dots took 24 us and the update 43 on 693,356 rows (of
+// 8 columns) against CHUNKFIG.
+constexpr int kChunkRows = 1024;
 constexpr float kSmallRealF = 1e-20f;
 constexpr int kMaxRestart = 20;        // MAX_RESTART, include/macro.h:33
 constexpr int kCoarseMax = 2048;       // dense coarsest limit (the block's b is staged in 64 KiB of LDS)
@@ -141,16 +145,25 @@ __global__ void k_agg_renumber(int n, const int *__restrict__ blk, const int *__
     }
 }
 
-// dense row-major copy of the diagonal block rows/cols [r0, r0+nb)
-__global__ void k_dense_block(const int *__restrict__ ia, const int *__restrict__ ja, const double *__restrict__ a,
-                              int r0, int nb, double *__restrict__ M) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nb; i += gridDim.x * blockDim.x) {
-        double *row = M + (size_t)i * nb;
-        for (int j = 0; j < nb; ++j) row[j] = 0.0;
-        for (int k = ia[r0 + i]; k < ia[r0 + i + 1]; ++k) {
-            const int j = ja[k] - r0;
-            if (j >= 0 && j < nb) row[j] += a[k];
-        }
+// dense row-major copies of the coarsest diagonal blocks (cleared before):
+// work[w] = (system entry, first row), a thread a row; csr: the levels' arrays
+struct LevelMatrices {
+    const int *ia[HZ_MAX_AMG_LVL], *ja[HZ_MAX_AMG_LVL];
+    const double *a[HZ_MAX_AMG_LVL];
+};
+__global__ __launch_bounds__(kWave) void k_dense_blocks(const long long *__restrict__ tab,
+                                                        const int *__restrict__ level, const int2 *__restrict__ work,
+                                                        LevelMatrices csr, double *__restrict__ W) {
+    const int2 wk = work[blockIdx.x];
+    const int r0 = (int)tab[4 * wk.x], nb = (int)tab[4 * wk.x + 1], l = level[wk.x];
+    const int i = wk.y + threadIdx.x;
+    if (i >= nb) return;
+    const int *ia = csr.ia[l], *ja = csr.ja[l];
+    const double *a = csr.a[l];
+    double *row = W + tab[4 * wk.x + 2] + (size_t)i * nb;
+    for (int k = ia[r0 + i]; k < ia[r0 + i + 1]; ++k) {
+        const int j = ja[k] - r0;
+        if (j >= 0 && j < nb) row[j] += a[k];
     }
 }
 
@@ -213,14 +226,22 @@ struct LaneMap {
     }
 };
 
+template <int kN>
+__device__ __forceinline__ void st_vec(double *p, const float *v) {
+#pragma unroll
+    for (int h = 0; h < kN / 2; ++h)
+        reinterpret_cast<double2 *>(p)[h] = make_double2((double)v[2 * h], (double)v[2 * h + 1]);
+}
+
 // One sweep xout = sweep(x) for live rows (Jacobi weight w / L1DIAG as in
-// the FP32 single-system cycle); dead rows copy x.
-template <int kSm, int kH, int kU>
+// the FP32 single-system cycle); dead rows copy x.  XT double: the cycle's last
+// sweep, writing z.
+template <int kSm, int kH, int kU, class XT>
 __global__ __launch_bounds__(kBlock) void k_bsweep(int n, int nslices, const long long *__restrict__ sptr,
                                                    const int *__restrict__ col, const float *__restrict__ val,
                                                    float wgt, const unsigned char *__restrict__ live,
                                                    const float *__restrict__ b, const float *__restrict__ x,
-                                                   float *__restrict__ xout, const int *__restrict__ rsys,
+                                                   XT *__restrict__ xout, const int *__restrict__ rsys,
                                                    const int *__restrict__ act) {
     constexpr int kN = kR / kH;
     const LaneMap<kH> m;
@@ -333,15 +354,31 @@ __global__ __launch_bounds__(kBlock) void k_bresidual(int n, int nslices, const 
     st_vec<kN>(w + (size_t)r * kR + m.q0, acc);
 }
 
-// bc = R w (member sums in ascending member order), one thread per coarse row
+// x = first sweep from zero of a live row (Jacobi: w b / d, L1DIAG: b / d with d
+// precomputed; w = 0 for a zero start)
+__device__ __forceinline__ void zero_sweep_row(int smoother, float wgt, float di, const float *b, float *x) {
+    float v[kR];
+#pragma unroll
+    for (int q = 0; q < kR; ++q) {
+        v[q] = 0.0f;
+        if (fabsf(di) > kSmallRealF) v[q] = smoother == HZ_SMOOTHER_L1DIAG ? b[q] / di : wgt * b[q] / di;
+    }
+    st_vec<kR>(x, v);
+}
+
+// bc = R w (member sums in ascending member order), one thread per coarse row,
+// and the coarse level's first sweep on it where the system goes on below
 __global__ void k_brestrict(int nc, const int *__restrict__ rptr, const int *__restrict__ rmem,
                             const float *__restrict__ w, float *__restrict__ bc, const int *__restrict__ crsys,
-                            const int *__restrict__ act) {
+                            const int *__restrict__ act, int smoother, float wgt, const float *__restrict__ dc,
+                            const unsigned char *__restrict__ live, float *__restrict__ xc) {
     for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < nc; c += gridDim.x * blockDim.x) {
         if (skip_row(crsys, act, c)) continue;
         float s[kR];
 #pragma unroll
         for (int q = 0; q < kR; ++q) s[q] = 0.0f;
+        const float di = dc[c];
+        const bool go = live[c];
         for (int p = rptr[c]; p < rptr[c + 1]; ++p) {
             float v[kR];
             ld_vec<kR>(w + (size_t)rmem[p] * kR, v);
@@ -349,24 +386,7 @@ __global__ void k_brestrict(int nc, const int *__restrict__ rptr, const int *__r
             for (int q = 0; q < kR; ++q) s[q] = s[q] + v[q];
         }
         st_vec<kR>(bc + (size_t)c * kR, s);
-    }
-}
-
-// x = first sweep from zero for live rows (Jacobi: w b / d, L1DIAG: b / d with d precomputed)
-__global__ void k_bzero_sweep(int n, int smoother, float wgt, const float *__restrict__ d,
-                              const unsigned char *__restrict__ live, const float *__restrict__ b,
-                              float *__restrict__ x, const int *__restrict__ rsys, const int *__restrict__ act) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        if (!live[i] || skip_row(rsys, act, i)) continue;
-        const float di = d[i];
-        float bi[kR], v[kR];
-        ld_vec<kR>(b + (size_t)i * kR, bi);
-#pragma unroll
-        for (int q = 0; q < kR; ++q) {
-            v[q] = 0.0f;
-            if (fabsf(di) > kSmallRealF) v[q] = smoother == HZ_SMOOTHER_L1DIAG ? bi[q] / di : wgt * bi[q] / di;
-        }
-        st_vec<kR>(x + (size_t)i * kR, v);
+        if (go) zero_sweep_row(smoother, wgt, di, s, xc + (size_t)c * kR);
     }
 }
 
@@ -385,54 +405,82 @@ __global__ void k_bprolong(int n, const int *__restrict__ agg, const float *__re
     }
 }
 
-// Systems whose hierarchy ends at this level: x = Ainv b per block (FP64
-// inverse and accumulation, sum over j ascending).  One workgroup per block,
-// a thread per row with all right-hand sides; the block's b staged in LDS;
-// the inverse stored transposed (entry (i, j) at io + j nb + i) so a
-// workgroup's loads of one j are contiguous.  tab[4 k .. 4 k + 3] = row
-// offset, size, inverse offset (in doubles), system.
-__global__ __launch_bounds__(256) void k_bcoarse(const long long *__restrict__ tab, const double *__restrict__ AinvT,
-                                                 const float *__restrict__ b, float *__restrict__ x,
-                                                 const int *__restrict__ act) {
-    extern __shared__ float bs[];
-    const long long r0 = tab[4 * blockIdx.x], nb = tab[4 * blockIdx.x + 1], io = tab[4 * blockIdx.x + 2];
-    if (act && act[tab[4 * blockIdx.x + 3]] == 0) return;
+// The coarse solves x = Ainv b of every system, whatever level its hierarchy
+// ends at, in one launch (FP64 inverse and accumulation): a workgroup takes 64
+// rows of one system, a lane a row with all right-hand sides, its four
+// wavefronts a quarter of the columns each with eight entries' loads in
+// flight; the block's b staged in LDS; the inverse stored transposed (entry
+// (i, j) at io + j nb + i) so a wave's loads of one j are contiguous.  As a
+// launch a level with one workgroup a system the solves took 118 of the 480 us
+// of an iteration of 48 systems, against 14.  tab[4 k .. 4 k + 3] =
+// row offset, size, inverse offset (in doubles), system; level[k]: its level;
+// work[w] = (system entry, first row).
+struct LevelVectors {
+    const float *b[HZ_MAX_AMG_LVL];
+    float *x[HZ_MAX_AMG_LVL];
+};
+__global__ __launch_bounds__(256) void k_bcoarse(const long long *__restrict__ tab, const int *__restrict__ level,
+                                                 const int2 *__restrict__ work, const double *__restrict__ AinvT,
+                                                 LevelVectors lv, const int *__restrict__ act) {
+    extern __shared__ double s_dyn[];
+    constexpr int kParts = 256 / kWave, U = 8;
+    double *red = s_dyn;                                           // kParts x 64 x kR
+    float *bs = reinterpret_cast<float *>(s_dyn + kParts * kWave * kR);   // nb x kR
+    const int2 wk = work[blockIdx.x];
+    const long long r0 = tab[4 * wk.x], nb = tab[4 * wk.x + 1], io = tab[4 * wk.x + 2];
+    if (act && act[tab[4 * wk.x + 3]] == 0) return;
+    const float *b = lv.b[level[wk.x]];
     for (long long e = threadIdx.x; e < nb * kR; e += blockDim.x) bs[e] = b[r0 * kR + e];
     __syncthreads();
-    for (long long i = threadIdx.x; i < nb; i += blockDim.x) {
-        double acc[kR];
+    const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int i = wk.y + lane;
+    const int per = ((int)nb + kParts - 1) / kParts, j1 = min((int)nb, (w + 1) * per);
+    double acc[kR];
 #pragma unroll
-        for (int q = 0; q < kR; ++q) acc[q] = 0.0;
-        const double *Mi = AinvT + io + i;
-        for (long long j = 0; j < nb; ++j) {
-            const double m = Mi[j * nb];
+    for (int q = 0; q < kR; ++q) acc[q] = 0.0;
+    const double *Mi = AinvT + io + min(i, (int)nb - 1);
+    for (int j = w * per; j < j1; j += U) {
+        double m[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) m[u] = j + u < j1 ? Mi[(long long)(j + u) * nb] : 0.0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (j + u >= j1) break;
             float bj[kR];
-            ld_vec<kR>(bs + j * kR, bj);
+            ld_vec<kR>(bs + (j + u) * kR, bj);
 #pragma unroll
-            for (int q = 0; q < kR; ++q) acc[q] += m * (double)bj[q];
+            for (int q = 0; q < kR; ++q) acc[q] += m[u] * (double)bj[q];
         }
+    }
+#pragma unroll
+    for (int q = 0; q < kR; ++q) red[(w * kR + q) * kWave + lane] = acc[q];
+    __syncthreads();
+    if (w == 0 && i < nb) {
         float o[kR];
 #pragma unroll
-        for (int q = 0; q < kR; ++q) o[q] = (float)acc[q];
-        st_vec<kR>(x + (r0 + i) * kR, o);
+        for (int q = 0; q < kR; ++q) {
+            double t = red[q * kWave + lane];
+            for (int k = 1; k < kParts; ++k) t += red[(k * kR + q) * kWave + lane];
+            o[q] = (float)t;
+        }
+        st_vec<kR>(lv.x[level[wk.x]] + (r0 + i) * kR, o);
     }
 }
 
 // Explicit inverses of many small dense matrices at once: workgroup k inverts
-// block k (size tab[4k+1], stored row-major at W + woff[k]) in place by
+// block k (size tab[4k+1], stored row-major at W + tab[4k+2]) in place by
 // Gauss-Jordan elimination without pivoting (the coarsest Galerkin matrices are
 // SPD), the elimination of the single-system coarsest inverse applied to the
 // whole block.  Writes the transpose of the inverse to T + tab[4k+2].  A zero
 // pivot sets status[k] = 1 and leaves the block.
 __global__ __launch_bounds__(1024) void k_batch_gj_inverse(const long long *__restrict__ tab,
-                                                           const long long *__restrict__ woff,
                                                            double *__restrict__ W, double *__restrict__ T,
                                                            int *__restrict__ status) {
     __shared__ double colk[kCoarseMax];
     __shared__ double rowk[kCoarseMax];
     const int blk = blockIdx.x;
     const int nb = (int)tab[4 * blk + 1];
-    double *M = W + woff[blk];
+    double *M = W + tab[4 * blk + 2];
     const int tid = threadIdx.x, nt = blockDim.x;
     for (int k = 0; k < nb; ++k) {
         const double piv = M[(size_t)k * nb + k];
@@ -465,8 +513,11 @@ __global__ __launch_bounds__(1024) void k_batch_gj_inverse(const long long *__re
     }
 }
 
+// b = fl(r), and the first level-0 sweep on it for the live rows
 __global__ void k_enter_b(int n, const double *__restrict__ r, float *__restrict__ b,
-                          const int *__restrict__ rsys, const int *__restrict__ act) {
+                          const int *__restrict__ rsys, const int *__restrict__ act, int smoother, float wgt,
+                          const float *__restrict__ d, const unsigned char *__restrict__ live,
+                          float *__restrict__ x) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         if (skip_row(rsys, act, i)) continue;
         const double2 *rp = reinterpret_cast<const double2 *>(r + (size_t)i * kR);
@@ -478,6 +529,7 @@ __global__ void k_enter_b(int n, const double *__restrict__ r, float *__restrict
             v[2 * h + 1] = (float)t.y;
         }
         st_vec<kR>(b + (size_t)i * kR, v);
+        if (live[i]) zero_sweep_row(smoother, wgt, d[i], v, x + (size_t)i * kR);
     }
 }
 
@@ -553,31 +605,64 @@ __global__ __launch_bounds__(kBlock) void k_spmm64(int n, int nslices, const lon
     for (int q = 0; q < kN; ++q) y[o + q] = kSub == 2 ? b[o + q] - acc[q] : acc[q];
 }
 
-// chunk c: rows [crow[c], crow[c+1]) of one system; partial sums per right-hand side
-struct ChunkDot {
-    __device__ static void store(double *part, int c, double v, double *sh) {
-        // threads t and t + 8k share right-hand side t % 8: reduce per rhs
-        sh[threadIdx.x] = v;
-        __syncthreads();
-        if (threadIdx.x < kR) {
-            double s = 0.0;
-            for (int t = threadIdx.x; t < (int)blockDim.x; t += kR) s += sh[t];
-            part[(size_t)c * kR + threadIdx.x] = s;
-        }
+// chunk c: rows [crow[c], crow[c+1]) of one system; a thread takes every 256th
+// double2 of them, always of right-hand sides 2 (t % 4) and 2 (t % 4) + 1.
+// body(e, u) handles the loaded double2 e (arrays of kChunkU).
+constexpr int kChunkU = 4;
+template <class Load, class Body>
+__device__ __forceinline__ void chunk_loop(const int *__restrict__ crow, int c, Load load, Body body) {
+    const long e0 = (long)crow[c] * (kR / 2), e1 = (long)crow[c + 1] * (kR / 2);
+    for (long e = e0 + threadIdx.x; e < e1; e += kBlock * kChunkU) {
+#pragma unroll
+        for (int u = 0; u < kChunkU; ++u)
+            if (e + u * kBlock < e1) load(e + u * kBlock, u);
+#pragma unroll
+        for (int u = 0; u < kChunkU; ++u)
+            if (e + u * kBlock < e1) body(e + u * kBlock, u);
     }
-};
+}
+
+// partial sums per right-hand side of a chunk: the lanes of a wave that share a
+// pair, then the waves in order
+__device__ __forceinline__ void chunk_store(double *part, int c, double2 v, double2 *sh) {
+#pragma unroll
+    for (int off = 4; off < kWave; off <<= 1) {
+        v.x += __shfl_xor(v.x, off, kWave);
+        v.y += __shfl_xor(v.y, off, kWave);
+    }
+    const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    if (lane < kR / 2) sh[w * (kR / 2) + lane] = v;
+    __syncthreads();
+    if (threadIdx.x < kR / 2) {
+        double2 t = sh[threadIdx.x];
+        for (int i = 1; i < kBlock / kWave; ++i) {
+            t.x += sh[i * (kR / 2) + threadIdx.x].x;
+            t.y += sh[i * (kR / 2) + threadIdx.x].y;
+        }
+        part[(size_t)c * kR + 2 * threadIdx.x] = t.x;
+        part[(size_t)c * kR + 2 * threadIdx.x + 1] = t.y;
+    }
+}
 
 // partial (u, v) per chunk and rhs
-__global__ __launch_bounds__(kBlock) void k_cdot(const int *__restrict__ crow, const double *__restrict__ u,
-                                                 const double *__restrict__ v, double *__restrict__ part,
+__global__ __launch_bounds__(kBlock) void k_cdot(const int *__restrict__ crow, const double *__restrict__ u_,
+                                                 const double *__restrict__ v_, double *__restrict__ part,
                                                  const int *__restrict__ csys, const int *__restrict__ act) {
-    __shared__ double sh[kBlock];
+    __shared__ double2 sh[kBlock / kWave * (kR / 2)];
     const int c = blockIdx.x;
     if (act && act[csys[c]] == 0) return;   // whole workgroup
-    const long e0 = (long)crow[c] * kR, e1 = (long)crow[c + 1] * kR;
-    double s = 0.0;
-    for (long e = e0 + threadIdx.x; e < e1; e += kBlock) s += u[e] * v[e];
-    ChunkDot::store(part, c, s, sh);
+    const double2 *u = reinterpret_cast<const double2 *>(u_), *v = reinterpret_cast<const double2 *>(v_);
+    double2 a[kChunkU], b[kChunkU], s = make_double2(0.0, 0.0);
+    chunk_loop(crow, c,
+               [&](long e, int i) {
+                   a[i] = u[e];
+                   b[i] = v[e];
+               },
+               [&](long, int i) {
+                   s.x += a[i].x * b[i].x;
+                   s.y += a[i].y * b[i].y;
+               });
+    chunk_store(part, c, s, sh);
 }
 
 // Per-column PCG state (column = system * kR + rhs).
@@ -588,72 +673,113 @@ struct ColState {
 
 // u += alpha p, r -= alpha t for unfinished columns; partial ||r||^2
 __global__ __launch_bounds__(kBlock) void k_cupdate(const int *__restrict__ crow, const int *__restrict__ csys,
-                                                    const ColState *__restrict__ st, const double *__restrict__ p,
-                                                    const double *__restrict__ t, double *__restrict__ u,
-                                                    double *__restrict__ r, double *__restrict__ part,
+                                                    const ColState *__restrict__ st, const double *__restrict__ p_,
+                                                    const double *__restrict__ t_, double *__restrict__ u_,
+                                                    double *__restrict__ r_, double *__restrict__ part,
                                                     const int *__restrict__ act) {
-    __shared__ double sh[kBlock];
+    __shared__ double2 sh[kBlock / kWave * (kR / 2)];
     const int c = blockIdx.x;
     if (act && act[csys[c]] == 0) return;
-    const int q = threadIdx.x % kR;
-    const ColState &cs = st[csys[c] * kR + q];
-    const bool active = !cs.done;
-    const double al = cs.alpha;
-    const long e0 = (long)crow[c] * kR, e1 = (long)crow[c + 1] * kR;
-    double s = 0.0;
-    for (long e = e0 + threadIdx.x; e < e1; e += kBlock) {
-        double re = r[e];
-        if (active) {
-            u[e] += al * p[e];
-            re -= al * t[e];
-            r[e] = re;
-        }
-        s += re * re;
-    }
-    ChunkDot::store(part, c, s, sh);
+    const ColState *cs = st + csys[c] * kR + 2 * (threadIdx.x % (kR / 2));
+    const bool on0 = !cs[0].done, on1 = !cs[1].done;
+    const double al0 = cs[0].alpha, al1 = cs[1].alpha;
+    const double2 *p = reinterpret_cast<const double2 *>(p_), *t = reinterpret_cast<const double2 *>(t_);
+    double2 *u = reinterpret_cast<double2 *>(u_), *r = reinterpret_cast<double2 *>(r_);
+    double2 pv[kChunkU], tv[kChunkU], uv[kChunkU], rv[kChunkU], s = make_double2(0.0, 0.0);
+    chunk_loop(crow, c,
+               [&](long e, int i) {
+                   pv[i] = p[e];
+                   tv[i] = t[e];
+                   uv[i] = u[e];
+                   rv[i] = r[e];
+               },
+               [&](long e, int i) {
+                   if (on0) {
+                       uv[i].x += al0 * pv[i].x;
+                       rv[i].x -= al0 * tv[i].x;
+                   }
+                   if (on1) {
+                       uv[i].y += al1 * pv[i].y;
+                       rv[i].y -= al1 * tv[i].y;
+                   }
+                   u[e] = uv[i];
+                   r[e] = rv[i];
+                   s.x += rv[i].x * rv[i].x;
+                   s.y += rv[i].y * rv[i].y;
+               });
+    chunk_store(part, c, s, sh);
 }
 
 // r = t (= b - A u) for candidate columns; partial ||r||^2 of those columns
 __global__ __launch_bounds__(kBlock) void k_creplace(const int *__restrict__ crow, const int *__restrict__ csys,
-                                                     const ColState *__restrict__ st, const double *__restrict__ t,
-                                                     double *__restrict__ r, double *__restrict__ part,
+                                                     const ColState *__restrict__ st, const double *__restrict__ t_,
+                                                     double *__restrict__ r_, double *__restrict__ part,
                                                      const int *__restrict__ gate, const int *__restrict__ act) {
     if (*gate == 0) return;
-    __shared__ double sh[kBlock];
+    __shared__ double2 sh[kBlock / kWave * (kR / 2)];
     const int c = blockIdx.x;
     if (act && act[csys[c]] == 0) return;
-    const int q = threadIdx.x % kR;
-    const bool cand = st[csys[c] * kR + q].cand != 0;
-    const long e0 = (long)crow[c] * kR, e1 = (long)crow[c + 1] * kR;
-    double s = 0.0;
-    for (long e = e0 + threadIdx.x; e < e1; e += kBlock) {
-        if (cand) {
-            const double re = t[e];
-            r[e] = re;
-            s += re * re;
-        }
-    }
-    ChunkDot::store(part, c, s, sh);
+    const ColState *cs = st + csys[c] * kR + 2 * (threadIdx.x % (kR / 2));
+    const bool on0 = cs[0].cand != 0, on1 = cs[1].cand != 0;
+    const double2 *t = reinterpret_cast<const double2 *>(t_);
+    double2 *r = reinterpret_cast<double2 *>(r_);
+    double2 tv[kChunkU], rv[kChunkU], s = make_double2(0.0, 0.0);
+    chunk_loop(crow, c,
+               [&](long e, int i) {
+                   tv[i] = t[e];
+                   rv[i] = r[e];
+               },
+               [&](long e, int i) {
+                   if (on0) {
+                       rv[i].x = tv[i].x;
+                       s.x += tv[i].x * tv[i].x;
+                   }
+                   if (on1) {
+                       rv[i].y = tv[i].y;
+                       s.y += tv[i].y * tv[i].y;
+                   }
+                   r[e] = rv[i];
+               });
+    chunk_store(part, c, s, sh);
 }
 
 // p = z + beta p for unfinished columns
 __global__ __launch_bounds__(kBlock) void k_cdirection(const int *__restrict__ crow, const int *__restrict__ csys,
-                                                       const ColState *__restrict__ st, const double *__restrict__ z,
-                                                       double *__restrict__ p, const int *__restrict__ act) {
+                                                       const ColState *__restrict__ st, const double *__restrict__ z_,
+                                                       double *__restrict__ p_, const int *__restrict__ act) {
     const int c = blockIdx.x;
     if (act && act[csys[c]] == 0) return;
-    const int q = threadIdx.x % kR;
-    const ColState &cs = st[csys[c] * kR + q];
-    if (cs.done) return;
-    const double be = cs.beta;
-    const long e0 = (long)crow[c] * kR, e1 = (long)crow[c + 1] * kR;
-    for (long e = e0 + threadIdx.x; e < e1; e += kBlock) p[e] = z[e] + be * p[e];
+    const ColState *cs = st + csys[c] * kR + 2 * (threadIdx.x % (kR / 2));
+    const bool on0 = !cs[0].done, on1 = !cs[1].done;
+    if (!on0 && !on1) return;
+    const double be0 = cs[0].beta, be1 = cs[1].beta;
+    const double2 *z = reinterpret_cast<const double2 *>(z_);
+    double2 *p = reinterpret_cast<double2 *>(p_);
+    double2 zv[kChunkU], pv[kChunkU];
+    chunk_loop(crow, c,
+               [&](long e, int i) {
+                   zv[i] = z[e];
+                   pv[i] = p[e];
+               },
+               [&](long e, int i) {
+                   if (on0) pv[i].x = zv[i].x + be0 * pv[i].x;
+                   if (on1) pv[i].y = zv[i].y + be1 * pv[i].y;
+                   p[e] = pv[i];
+               });
 }
 
 // column sums of the chunk partials of its system, in chunk order
 __device__ __forceinline__ double col_sum(const double *part, const int *schunk, int sys, int q) {
+    constexpr int U = 16;   // loads issued together
     double s = 0.0;
-    for (int c = schunk[sys]; c < schunk[sys + 1]; ++c) s += part[(size_t)c * kR + q];
+    const int c1 = schunk[sys + 1];
+    for (int c = schunk[sys]; c < c1; c += U) {
+        double a[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) a[u] = c + u < c1 ? part[(size_t)(c + u) * kR + q] : 0.0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) s += a[u];
+    }
     return s;
 }
 
@@ -789,10 +915,6 @@ struct BatchLevel {
     std::vector<int> sys, off;       // blocks: system id, row offsets (nblk + 1)
     unsigned char *live = nullptr;   // rows of systems that continue below
     int *agg = nullptr, nagg = 0, *rptr = nullptr, *rmem = nullptr;
-    int ncoarse = 0;                 // systems solved at this level
-    int cmax = 0;                    // their largest size
-    long long *ctab = nullptr;       // (row offset, size, inverse offset, system) per such system
-    double *Ainv = nullptr;
     float *b = nullptr, *x = nullptr, *xt = nullptr, *w = nullptr;
     int shape = 104;                 // FP32 cycle kernels' shape chosen by the tuner (shape code)
     int spmm_shape = 204;            // level 0: shape of the FP64 PCG SpMM (tuned)
@@ -805,6 +927,13 @@ struct BatchHierarchy {
     float wgt = 1.0f;
     std::vector<int> levels_of;      // per system: number of levels
     int *act = nullptr;              // per system: 1 while any right-hand side iterates (null: all)
+    // coarse solves: (row offset, size, inverse offset, system) and level per
+    // system, 64-row pieces of them, and the inverses
+    int cmax = 0, npieces = 0;
+    long long *ctab = nullptr;
+    int *clevel = nullptr;
+    int2 *cwork = nullptr;
+    double *Ainv = nullptr;
 };
 
 namespace {
@@ -836,17 +965,17 @@ bool valid_shape(int code) {
     return false;
 }
 
-void bsweep(const BatchLevel &L, int sm, float w, const float *b, const float *x, float *xo,
-            const int *act = nullptr) {
+template <class XT>
+void bsweep(const BatchLevel &L, int sm, float w, const float *b, const float *x, XT *xo, const int *act = nullptr) {
     if (L.S.n == 0) return;
     with_shape(L.shape, [&](auto H, auto U) {
         constexpr int kH = decltype(H)::value, kU = decltype(U)::value;
         const int grid = div_up(L.S.nslices * kH, kSlicesPerBlock);
         if (sm == HZ_SMOOTHER_L1DIAG)
-            k_bsweep<HZ_SMOOTHER_L1DIAG, kH, kU><<<grid, kBlock, 0, stream()>>>(
+            k_bsweep<HZ_SMOOTHER_L1DIAG, kH, kU, XT><<<grid, kBlock, 0, stream()>>>(
                 L.S.n, L.S.nslices, L.S.sptr, L.S.col, L.valf, w, L.live, b, x, xo, L.rsys, act);
         else
-            k_bsweep<HZ_SMOOTHER_JACOBI, kH, kU><<<grid, kBlock, 0, stream()>>>(
+            k_bsweep<HZ_SMOOTHER_JACOBI, kH, kU, XT><<<grid, kBlock, 0, stream()>>>(
                 L.S.n, L.S.nslices, L.S.sptr, L.S.col, L.valf, w, L.live, b, x, xo, L.rsys, act);
     });
     HZ_LAUNCH_CHECK();
@@ -947,6 +1076,9 @@ int tune_shape(BatchLevel &L, int sm, float w) {
 
 }  // namespace
 
+// LDS of k_bcoarse for blocks of up to nb rows
+static size_t coarse_lds(int nb) { return sizeof(double) * 256 * kR + sizeof(float) * kR * nb; }
+
 // Setup of the stacked hierarchies.  A0: the level-0 super matrix (device,
 // borrowed), off0: nsys + 1 row offsets.  theta: per system, the caller's
 // strong_coupled (updated per level per system, as amg_setup_ua.c:1325-1328
@@ -971,6 +1103,10 @@ int batch_setup(BatchHierarchy &H, const DevCSR &A0, const std::vector<int> &off
     H.lv[0].sys.resize(nsys);
     for (int s = 0; s < nsys; ++s) H.lv[0].sys[s] = s;
     hipStream_t st = stream();
+    std::vector<long long> ctab;   // the coarse solves of all levels
+    std::vector<int> clevel;
+    std::vector<int2> pieces;
+    long long inv_total = 0;
     for (int lvl = 0;; ++lvl) {
         BatchLevel &L = H.lv[lvl];
         const int n = L.A.n, nblk = (int)L.sys.size();
@@ -1034,9 +1170,7 @@ int batch_setup(BatchHierarchy &H, const DevCSR &A0, const std::vector<int> &off
                 if (nagg_b[k] < 1) keep[k] = 0;   // P.col < MIN_CDOF (amg_setup_ua.c:1340)
             }
         }
-        // systems solved at this level: dense FP64 inverse of their block
-        std::vector<long long> ctab;
-        long long inv_total = 0;
+        // systems solved at this level: a dense FP64 inverse of their block
         for (int k = 0; k < nblk; ++k) {
             if (keep[k]) continue;
             const long long nb = L.off[k + 1] - L.off[k];
@@ -1045,39 +1179,12 @@ int batch_setup(BatchHierarchy &H, const DevCSR &A0, const std::vector<int> &off
                             nb, kCoarseMax);
                 return HZ_ERROR_INPUT_PAR;
             }
-            L.cmax = std::max<int>(L.cmax, (int)nb);
-            ctab.push_back(L.off[k]);
-            ctab.push_back(nb);
-            ctab.push_back(inv_total);
-            ctab.push_back(L.sys[k]);
+            H.cmax = std::max<int>(H.cmax, (int)nb);
+            for (long long i = 0; i < nb; i += kWave) pieces.push_back(make_int2((int)clevel.size(), (int)i));
+            ctab.insert(ctab.end(), {(long long)L.off[k], nb, inv_total, (long long)L.sys[k]});
+            clevel.push_back(lvl);
             inv_total += nb * nb;
             H.levels_of[L.sys[k]] = lvl + 1;
-        }
-        L.ncoarse = (int)(ctab.size() / 4);
-        if (L.ncoarse) {
-            L.Ainv = arena().alloc_n<double>((size_t)inv_total + 1);
-            L.ctab = arena().alloc_n<long long>(ctab.size() + 1);
-            HZ_CHECK(memcpy_sync(L.ctab, ctab.data(), sizeof(long long) * ctab.size(), hipMemcpyHostToDevice));
-            // dense copies of the blocks (work area at the inverses' offsets),
-            // then all inverses in one launch
-            double *W = arena().alloc_n<double>((size_t)inv_total + 1);
-            std::vector<long long> woff(L.ncoarse);
-            for (int c = 0; c < L.ncoarse; ++c) {
-                const int r0 = (int)ctab[4 * c], nb = (int)ctab[4 * c + 1];
-                woff[c] = ctab[4 * c + 2];
-                k_dense_block<<<div_up(nb, 64), 64, 0, st>>>(L.A.ia, L.A.ja, L.A.val, r0, nb, W + woff[c]);
-            }
-            HZ_LAUNCH_CHECK();
-            long long *dwoff = arena().alloc_n<long long>((size_t)L.ncoarse + 1);
-            int *dstat = arena().alloc_n<int>((size_t)L.ncoarse + 1);
-            HZ_CHECK(memcpy_sync(dwoff, woff.data(), sizeof(long long) * L.ncoarse, hipMemcpyHostToDevice));
-            HZ_CHECK(hipMemsetAsync(dstat, 0, sizeof(int) * L.ncoarse, st));
-            k_batch_gj_inverse<<<L.ncoarse, 1024, 0, st>>>(L.ctab, dwoff, W, L.Ainv, dstat);
-            HZ_LAUNCH_CHECK();
-            std::vector<int> hstat(L.ncoarse);
-            HZ_CHECK(memcpy_sync(hstat.data(), dstat, sizeof(int) * L.ncoarse, hipMemcpyDeviceToHost));
-            for (int v : hstat)
-                if (v) return HZ_ERROR_SOLVER_MISC;
         }
         // live rows, renumbered aggregates, next level
         L.live = arena().alloc_n<unsigned char>((size_t)n + 1);
@@ -1126,6 +1233,39 @@ int batch_setup(BatchHierarchy &H, const DevCSR &A0, const std::vector<int> &off
         H.lv.push_back(C);
     }
     H.nl = (int)H.lv.size();
+    // the coarsest blocks of all systems: dense copies, then all inverses in one
+    // launch (a launch a level left most of the chip idle for 2.3-2.7 ms each)
+    const int ncoarse = (int)clevel.size();
+    H.npieces = (int)pieces.size();
+    H.Ainv = arena().alloc_n<double>((size_t)inv_total + 1);
+    H.ctab = arena().alloc_n<long long>(ctab.size() + 1);
+    H.clevel = arena().alloc_n<int>((size_t)ncoarse + 1);
+    H.cwork = arena().alloc_n<int2>((size_t)H.npieces + 1);
+    if (ncoarse) {
+        HZ_CHECK(memcpy_sync(H.ctab, ctab.data(), sizeof(long long) * ctab.size(), hipMemcpyHostToDevice));
+        HZ_CHECK(memcpy_sync(H.clevel, clevel.data(), sizeof(int) * ncoarse, hipMemcpyHostToDevice));
+        HZ_CHECK(memcpy_sync(H.cwork, pieces.data(), sizeof(int2) * H.npieces, hipMemcpyHostToDevice));
+        double *W = arena().alloc_n<double>((size_t)inv_total + 1);
+        int *dstat = arena().alloc_n<int>((size_t)ncoarse + 1);
+        HZ_CHECK(hipMemsetAsync(W, 0, sizeof(double) * inv_total, st));
+        HZ_CHECK(hipMemsetAsync(dstat, 0, sizeof(int) * ncoarse, st));
+        LevelMatrices csr{};
+        for (int l = 0; l < H.nl; ++l) {
+            csr.ia[l] = H.lv[l].A.ia;
+            csr.ja[l] = H.lv[l].A.ja;
+            csr.a[l] = H.lv[l].A.val;
+        }
+        k_dense_blocks<<<H.npieces, kWave, 0, st>>>(H.ctab, H.clevel, H.cwork, csr, W);
+        HZ_LAUNCH_CHECK();
+        k_batch_gj_inverse<<<ncoarse, 1024, 0, st>>>(H.ctab, W, H.Ainv, dstat);
+        HZ_LAUNCH_CHECK();
+        std::vector<int> hstat(ncoarse);
+        HZ_CHECK(memcpy_sync(hstat.data(), dstat, sizeof(int) * ncoarse, hipMemcpyDeviceToHost));
+        for (int v : hstat)
+            if (v) return HZ_ERROR_SOLVER_MISC;
+        HZ_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_bcoarse),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)coarse_lds(kCoarseMax)));
+    }
     H.act = arena().alloc_n<int>((size_t)nsys + 1);
     k_fill_i<<<grid_for(nsys), kBlock, 0, st>>>(nsys, 1, H.act);
     HZ_LAUNCH_CHECK();
@@ -1135,50 +1275,57 @@ int batch_setup(BatchHierarchy &H, const DevCSR &A0, const std::vector<int> &off
 }
 
 // z = B(r) for all columns: one V-cycle from zero (precond_amg with maxit 1,
-// cycle_type V), FP32.  r, z: level-0 interleaved FP64.
+// cycle_type V), FP32.  r, z: level-0 interleaved FP64.  The first sweep of a
+// level is formed where its b is, and the last level-0 sweep writes z.
 void batch_vcycle(BatchHierarchy &H, const double *r, double *z) {
     const int nl = H.nl;
     hipStream_t st = stream();
     BatchLevel &L0 = H.lv[0];
     const int *act = H.act;
-    k_enter_b<<<grid_for(L0.A.n), kBlock, 0, st>>>(L0.A.n, r, L0.b, L0.rsys, act);
+    // without pre-smoothing the live rows start from zero (weight 0)
+    const int sm0 = H.pre > 0 ? H.smoother : HZ_SMOOTHER_JACOBI;
+    const float w0 = H.pre > 0 ? H.wgt : 0.0f;
+    k_enter_b<<<grid_for(L0.A.n), kBlock, 0, st>>>(L0.A.n, r, L0.b, L0.rsys, act, sm0, w0, L0.dsm, L0.live, L0.x);
     HZ_LAUNCH_CHECK();
     // descend
-    for (int l = 0; l < nl; ++l) {
+    for (int l = 0; l + 1 < nl; ++l) {
         BatchLevel &L = H.lv[l];
-        const int n = L.A.n;
-        if (L.ncoarse)
-            k_bcoarse<<<L.ncoarse, 256, sizeof(float) * kR * L.cmax, st>>>(L.ctab, L.Ainv, L.b, L.x, act);
-        if (l == nl - 1) break;
-        if (H.pre > 0) {
-            k_bzero_sweep<<<grid_for(n), kBlock, 0, st>>>(n, H.smoother, H.wgt, L.dsm, L.live, L.b, L.x,
-                                                          L.rsys, act);
-            for (int s = 1; s < H.pre; ++s) {
-                bsweep(L, H.smoother, H.wgt, L.b, L.x, L.xt, act);
-                std::swap(L.x, L.xt);
-            }
-        } else {
-            // x = 0 on live rows: the dead rows hold the coarse solution
-            k_bzero_sweep<<<grid_for(n), kBlock, 0, st>>>(n, HZ_SMOOTHER_JACOBI, 0.0f, L.dsm, L.live, L.b, L.x,
-                                                          L.rsys, act);
+        for (int s = 1; s < H.pre; ++s) {
+            bsweep(L, H.smoother, H.wgt, L.b, L.x, L.xt, act);
+            std::swap(L.x, L.xt);
         }
         bresidual(L, act);
         BatchLevel &C = H.lv[l + 1];
-        const long totc = (long)C.A.n * kR;
-        k_brestrict<<<grid_for(C.A.n), kBlock, 0, st>>>(C.A.n, L.rptr, L.rmem, L.w, C.b, C.rsys, act);
+        k_brestrict<<<grid_for(C.A.n), kBlock, 0, st>>>(C.A.n, L.rptr, L.rmem, L.w, C.b, C.rsys, act, sm0, w0, C.dsm,
+                                                        C.live, C.x);
+        HZ_LAUNCH_CHECK();
+    }
+    if (H.npieces) {
+        LevelVectors lv{};
+        for (int l = 0; l < nl; ++l) {
+            lv.b[l] = H.lv[l].b;
+            lv.x[l] = H.lv[l].x;
+        }
+        k_bcoarse<<<H.npieces, 256, coarse_lds(H.cmax), st>>>(H.ctab, H.clevel, H.cwork, H.Ainv, lv, act);
         HZ_LAUNCH_CHECK();
     }
     // ascend
+    bool z_written = false;
     for (int l = nl - 2; l >= 0; --l) {
         BatchLevel &L = H.lv[l];
         BatchLevel &C = H.lv[l + 1];
         k_bprolong<<<grid_for(L.A.n), kBlock, 0, st>>>(L.A.n, L.agg, C.x, L.x, L.rsys, act);
         for (int s = 0; s < H.post; ++s) {
+            if (l == 0 && s == H.post - 1) {
+                bsweep(L, H.smoother, H.wgt, L.b, L.x, z, act);
+                z_written = true;
+                break;
+            }
             bsweep(L, H.smoother, H.wgt, L.b, L.x, L.xt, act);
             std::swap(L.x, L.xt);
         }
     }
-    k_exit_b<<<grid_for(L0.A.n), kBlock, 0, st>>>(L0.A.n, L0.x, z, L0.rsys, act);
+    if (!z_written) k_exit_b<<<grid_for(L0.A.n), kBlock, 0, st>>>(L0.A.n, L0.x, z, L0.rsys, act);
     HZ_LAUNCH_CHECK();
 }
 

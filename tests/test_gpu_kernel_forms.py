@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from hazmath_amd import capi, problems
-from test_gpu_parity import _solve_both
+from test_gpu_parity import _set_precision, _solve_both
 
 pytestmark = pytest.mark.gpu
 
@@ -276,3 +276,40 @@ def test_mlp_gradient_tiles_vs_fp64(lib, B):
                           dy.sum(0)])
     assert np.linalg.norm(grad - ref) < 2e-5 * np.linalg.norm(ref)
     assert abs(loss[0] - (d ** 2).mean()) < 2e-6 * (d ** 2).mean()
+
+
+# sweeps before and after (a zero start without sweeps, the last sweep writing z or not), and largest coarsest blocks:
+# below 64 rows, above 512; systems of 31^2 + 1 chunk ends: 961 rows (below a chunk of 1,024), 1,024 (one), 1,089 (one
+# and a rest); 25 rows are solved at level 0
+@pytest.mark.parametrize("pre,post,coarse", [(1, 1, 30), (2, 2, 600), (0, 1, 100), (1, 0, 100), (0, 0, 30)])
+def test_batch_cycle_forms_vs_single_system(lib, libc, pre, post, coarse):
+    """Every pair as the single-system solver with the same FP32 cycle.  The cycles round differently, which moves the
+    iterates by 2^-24 relative and the iteration at which 1e-8 is passed by at most one; both solutions are then within
+    1e-8 times the condition number (below 1e4 here) of the true one, 1e-4 of each other."""
+    systems = [problems.aniso2d_p1(m, 0.4 + 0.1 * m, 0.3) for m in (32, 6, 33, 34, 48)]
+    B = [problems.batch_rhs(s[0].size - 1, k, nrhs=3) for k, s in enumerate(systems)]
+    X = [np.zeros_like(b) for b in B]
+
+    def params():
+        it, amg = capi.solver_params(lib, tol=1e-8, maxit=60, aggregation=capi.HEM, smoother=capi.SMOOTHER_JACOBI,
+                                     coarse_dof=coarse, theta=0.04)
+        amg.presmooth_iter, amg.postsmooth_iter = pre, post
+        return it, amg
+    r, iters = capi.batch_solve(lib, systems, B, X, *params())
+    old = _set_precision(lib, 1)
+    try:
+        for k, (ia, ja, va) in enumerate(systems):
+            A = capi.HostCSR(ia, ja, va)
+            for q in range(3):
+                its, amgs = params()
+                x = capi.HostVec(np.zeros(ia.size - 1))
+                libc.srand(1)
+                rs = lib.linear_solver_dcsr_krylov_amg(A.ptr(), capi.HostVec(B[k][q]).ptr(), x.ptr(), C.byref(its),
+                                                       C.byref(amgs))
+                print(f"[batch] {pre},{post},{coarse} system {k} rhs {q}: {iters[k, q]} single {rs}", flush=True)
+                assert (rs > 0) == (iters[k, q] > 0)
+                if rs > 0:
+                    assert abs(int(iters[k, q]) - rs) <= 1
+                    assert np.linalg.norm(X[k][q] - x.arr) <= 1e-4 * np.linalg.norm(x.arr)
+    finally:
+        _set_precision(lib, old)
