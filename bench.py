@@ -574,6 +574,20 @@ def main_learned(a, lib):
     print(json.dumps(line))
 
 
+def distinct_pairs(off, va, stop=255, chunk=1 << 20):
+    """Different (offset, value) pairs among the entries the solve keeps (off-diagonal zeros left out); counting ends
+    above `stop`."""
+    seen = set()
+    for k in range(0, off.size, chunk):
+        o, v = off[k:k + chunk], va[k:k + chunk]
+        keep = (v != 0.0) | (o == 0)
+        for d in np.unique(o[keep]):
+            seen.update((int(d), float(x)) for x in np.unique(v[keep & (o == d)])[:stop + 1])
+        if len(seen) > stop:
+            break
+    return len(seen)
+
+
 def main():
     a = parse()
     if a.gpus != 1:
@@ -713,7 +727,10 @@ def main():
     paired = (a.precision == "fp64" and a.smoother in ("l1", "jacobi") and n >= 65536
               and os.environ.get("HZ_COL16", "1") != "0"
               and int(np.abs(ja.astype(np.int64) - rows).max()) <= 32767)
-    eb = 10 if paired else 12
+    # at most 255 different (offset, value) pairs on such a level: one byte an entry
+    coded = (n >= 65536 and os.environ.get("HZ_COL16", "1") != "0"
+             and distinct_pairs(ja.astype(np.int64) - rows, va) <= 255)
+    eb = 1 if coded else 10 if paired else 12
     # the solve's copies leave stored off-diagonal zeros out: its kernels are
     # priced at the entries they stream
     kept = int(np.count_nonzero((va != 0.0) | (ja == rows)))
@@ -803,7 +820,9 @@ def main():
         "spmv_gbs": spmv_gbs,
         "roofline": {
             "bound": "hbm",
-            "kernel": ("k_spmv: SELL-64 SpMV t=Ap with (t,p) partials, columns as paired 16-bit offsets (10 bytes an "
+            "kernel": ("k_coded: SELL-64 SpMV t=Ap with (t,p) partials, entries as one-byte codes of their "
+                       "(offset, value) pairs" if coded else
+                       "k_spmv: SELL-64 SpMV t=Ap with (t,p) partials, columns as paired 16-bit offsets (10 bytes an "
                        "entry)" if paired else
                        "k_spmv: SELL-64 SpMV t=Ap with (t,p) partials") + f", {kept} of the {nnz} stored entries "
                       "(off-diagonal zeros left out), fine level, in the PCG",

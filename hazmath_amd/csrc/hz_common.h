@@ -169,6 +169,24 @@ __device__ __forceinline__ unsigned short f2bf(float f) {
     return (unsigned short)(r >> 16);
 }
 
+// Entry codes: where a matrix has at most 255 different (column - row, value)
+// pairs -- constant coefficients on a regular grid -- an entry is one byte, its
+// pair's place in a table, four entries of a row to a 32-bit word, the same
+// number of words for every slice of 64 rows, lane-major as its entries are,
+// padding kCodePad.  The table holds the values' own bits (FP32 cycle: those of
+// their FP32 copies).
+enum class code8 : unsigned int {};
+constexpr int kCodes = 256, kCodePad = 255;
+// An entry of the table: the value and the pair's column offset in bytes of a
+// vector of T, so a kernel's address is the row's plus that.
+template <class T>
+struct CodeEntry {
+    T val;
+    int off;
+};
+template <class T>
+using CodeTable = CodeEntry<T>[kCodes];
+
 // 16-bit column offsets from the row, two entries of a row to a 32-bit word:
 // entry 2p of the row in the low half of word p, 2p+1 in the high half, words
 // of a SELL slice lane-major as its entries are, padding kColPad16.  Slice s's

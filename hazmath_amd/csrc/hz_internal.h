@@ -30,6 +30,12 @@ struct DevSELL {
     // the columns again as paired 16-bit offsets (col_base), when the FP64
     // cycle's level has them; null otherwise
     unsigned int *pcol = nullptr;
+    // entry codes (code8 in hz_common.h) and their table, where the matrix has
+    // few enough (offset, value) pairs; null otherwise
+    unsigned int *code = nullptr;
+    int cwords = 0;            // words of a slice's row
+    void *ctab = nullptr;      // CodeEntry<double>[kCodes]
+    void *ctabf = nullptr;     // CodeEntry<float>[kCodes]: the values in FP32
 };
 
 // Entries a round of the masked SELL kernels: 8 where the slices are at most 8
@@ -336,14 +342,18 @@ struct LowMatrix {
     void *csr = nullptr;
     // the SELL column indices again as 16-bit offsets from the row (padding
     // kColPad16), two entries of a row to a 32-bit word, slice s from word
-    // sptr[s] / 2 + 32 s, when every stored entry's fits; null otherwise
+    // sptr[s] / 2 + 32 s, when every stored entry's fits; null otherwise, and
+    // where the matrix has entry codes
     unsigned int *dcol = nullptr;
 };
 void low_values(const DevSELL &S, const DevCSR &A, int kind, LowMatrix &out, bool col16 = false);
 // queue the conversion of S's columns into paired 16-bit offsets (col_base);
 // the device int *misfit is cleared first and set when some offset does not fit
 unsigned int *col16_launch(const DevSELL &S, int *misfit);
-// HZ_COL16=0 switches the 16-bit column offsets off
+// give S its entry codes if it has few enough (offset, value) pairs (waits for
+// the count); returns whether it has them
+bool codes_build(DevSELL &S);
+// HZ_COL16=0 switches the 16-bit column offsets and the entry codes off
 bool col16_enabled();
 // FP32 copy of a CSR matrix's values (smoothed aggregation's P and R).
 float *values_f32(const DevCSR &A);

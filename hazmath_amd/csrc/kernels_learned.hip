@@ -14,7 +14,7 @@
 #include <cmath>
 #include <vector>
 
-#include "hz_internal.h"
+#include "coded.hpp"
 
 namespace hz {
 
@@ -292,8 +292,10 @@ void cheby_apply(const DevSELL &S, const ChebLevel &c, int steps, const double *
             std::swap(x, xt);
             continue;
         }
-        count_bytes(matrix_bytes(S.nnz, S.n) + 48.0 * S.n);
-        if (grp)
+        count_bytes((S.code ? coded_bytes(S) : matrix_bytes(S.nnz, S.n)) + 48.0 * S.n);
+        if (S.code)
+            launch_coded<double>(S, CodedCheb<double, false>{c.diag, b, x, xt, dwork, nullptr, nullptr, c1, c2});
+        else if (grp)
             k_cheb_step_grp<G><<<div_up((long)S.n * G, kBlock), kBlock, 0, stream()>>>(S.n, A->ia, A->ja, A->val,
                                                                                        c.diag, c1, c2, b, x, xt,
                                                                                        dwork);

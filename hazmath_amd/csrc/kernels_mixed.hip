@@ -12,7 +12,7 @@
 #include <algorithm>
 #include <cstdlib>
 
-#include "hz_internal.h"
+#include "coded.hpp"
 
 namespace hz {
 
@@ -64,7 +64,6 @@ __device__ __forceinline__ float zero_sweep(int smoother, float w, float b, floa
     return 0.0f;
 }
 
-// b = fl(r); optionally x = first sweep from zero
 // 16-bit column offsets of a SELL matrix in the paired form ld_cols reads
 // (one wave per slice); any stored entry whose offset from its row needs more
 // sets *misfit
@@ -93,6 +92,196 @@ __global__ __launch_bounds__(kBlock) void k_col16(int nslices, const long long *
     if (bad) *misfit = 1;
 }
 
+// The distinct (column - row, value) pairs of a SELL matrix: a workgroup
+// gathers those of a run of slices in an open-addressing table in LDS (keys of
+// 64 hashed bits; an entry whose key is there costs one LDS read), then adds
+// them to the one in memory, whose slot keeps the pair itself.  More than
+// kCodePad pairs: *count ends above kCodePad and the rest stops early.
+constexpr int kPairSlots = 512;
+struct PairTable {
+    unsigned long long key[kPairSlots];
+    double val[kPairSlots];
+    int off[kPairSlots];
+    int count;
+    int misfit;
+    int widest;
+};
+__device__ __forceinline__ unsigned long long pair_key(int off, double v) {
+    unsigned long long h = (unsigned long long)__double_as_longlong(v) * 0x9E3779B97F4A7C15ull;
+    h = (h ^ (h >> 32) ^ (unsigned long long)(unsigned int)off) * 0xD6E8FEB86659FD93ull;
+    return (h ^ (h >> 32)) | 1ull;
+}
+__device__ __forceinline__ int pair_slot(unsigned long long key) { return (int)(key >> 40) & (kPairSlots - 1); }
+// slot of key in the table, or the free slot it was put in (*fresh); -1: full
+template <class Load, class Cas>
+__device__ __forceinline__ int pair_insert(unsigned long long key, bool *fresh, Load load, Cas cas) {
+    int s = pair_slot(key);
+    *fresh = false;
+    for (int t = 0; t < kPairSlots; ++t, s = (s + 1) & (kPairSlots - 1)) {
+        unsigned long long cur = load(s);
+        if (cur == 0) {
+            cur = cas(s, key);
+            if (cur == 0) {
+                *fresh = true;
+                return s;
+            }
+        }
+        if (cur == key) return s;
+    }
+    return -1;
+}
+
+constexpr int kPairRun = 8;   // slices of a wave
+__global__ __launch_bounds__(kBlock) void k_code_pairs(int nslices, const long long *__restrict__ sptr,
+                                                       const int *__restrict__ col, const double *__restrict__ val,
+                                                       PairTable *__restrict__ g) {
+    __shared__ unsigned long long key[kPairSlots];
+    __shared__ double pv[kPairSlots];
+    __shared__ int po[kPairSlots];
+    __shared__ int count, total;
+    for (int i = threadIdx.x; i < kPairSlots; i += kBlock) key[i] = 0;
+    if (threadIdx.x == 0) {
+        count = 0;
+        total = __hip_atomic_load(&g->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (total > kCodePad) return;   // whole workgroup
+    const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int s0 = (blockIdx.x * kSlicesPerBlock + w) * kPairRun, s1 = min(nslices, s0 + kPairRun);
+    bool full = false;
+    int widest = 0;
+    for (int s = s0; s < s1 && !full; ++s) {
+        const long long base = sptr[s];
+        const int wd = (int)((sptr[s + 1] - base) / kSlice);
+        constexpr int U = 8;
+        widest = max(widest, wd);
+        for (int k = 0; k < wd && !full; k += U) {
+            int c[U];
+            double v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                c[u] = k + u < wd ? col[base + (long long)(k + u) * kSlice + lane] : -1;
+                v[u] = k + u < wd ? val[base + (long long)(k + u) * kSlice + lane] : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (c[u] < 0 || full) continue;
+                const int off = c[u] - (s * kSlice + lane);
+                bool fresh;
+                const int t = pair_insert(
+                    pair_key(off, v[u]), &fresh, [&](int q) { return ((volatile unsigned long long *)key)[q]; },
+                    [&](int q, unsigned long long kk) { return atomicCAS(&key[q], 0ull, kk); });
+                if (fresh) {
+                    pv[t] = v[u];
+                    po[t] = off;
+                    full = atomicAdd(&count, 1) >= kCodePad;
+                } else {
+                    full = t < 0;
+                }
+            }
+            full = __any(full);
+        }
+    }
+    if (lane == 0 && widest > __hip_atomic_load(&g->widest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(&g->widest, widest);
+    __syncthreads();
+    if (count > kCodePad) {
+        if (threadIdx.x == 0) atomicAdd(&g->count, kCodes);
+        return;
+    }
+    for (int i = threadIdx.x; i < kPairSlots; i += kBlock) {
+        if (key[i] == 0) continue;
+        bool fresh;
+        const int t = pair_insert(
+            key[i], &fresh,
+            [&](int q) { return __hip_atomic_load(&g->key[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); },
+            [&](int q, unsigned long long kk) { return atomicCAS(&g->key[q], 0ull, kk); });
+        if (t < 0) {
+            atomicAdd(&g->count, kCodes);
+        } else if (fresh) {
+            g->val[t] = pv[i];
+            g->off[t] = po[i];
+            atomicAdd(&g->count, 1);
+        }
+    }
+}
+
+// codes of the used slots in slot order, and the tables the kernels read
+__global__ __launch_bounds__(kPairSlots) void k_code_table(const PairTable *__restrict__ g,
+                                                           CodeEntry<double> *__restrict__ tab,
+                                                           CodeEntry<float> *__restrict__ tabf,
+                                                           unsigned char *__restrict__ code) {
+    __shared__ int cnt[kPairSlots / kWave];
+    const int i = threadIdx.x, w = i / kWave, lane = i % kWave;
+    if (i < kCodes) {
+        tab[i] = {0.0, 0};
+        tabf[i] = {0.0f, 0};
+    }
+    const bool used = g->key[i] != 0;
+    const unsigned long long m = __ballot(used);
+    if (lane == 0) cnt[w] = __popcll(m);
+    __syncthreads();
+    int c = __popcll(m & ((1ull << lane) - 1));
+    for (int q = 0; q < w; ++q) c += cnt[q];
+    if (used && c < kCodePad) {
+        tab[c] = {g->val[i], (int)(g->off[i] * sizeof(double))};
+        tabf[c] = {(float)g->val[i], (int)(g->off[i] * sizeof(float))};
+        code[i] = (unsigned char)c;
+    }
+}
+
+// the entries' codes; one whose pair is not its key's (two pairs with equal
+// hashes) sets *misfit
+__global__ __launch_bounds__(kBlock) void k_code_fill(int nslices, const long long *__restrict__ sptr,
+                                                      const int *__restrict__ col, const double *__restrict__ val,
+                                                      PairTable *__restrict__ g,
+                                                      const unsigned char *__restrict__ code, int words,
+                                                      unsigned int *__restrict__ d) {
+    __shared__ unsigned long long key[kPairSlots];
+    __shared__ long long pv[kPairSlots];
+    __shared__ int po[kPairSlots], pc[kPairSlots];
+    for (int i = threadIdx.x; i < kPairSlots; i += kBlock) {
+        key[i] = g->key[i];
+        pv[i] = __double_as_longlong(g->val[i]);
+        po[i] = g->off[i];
+        pc[i] = code[i];
+    }
+    __syncthreads();
+    const int s = blockIdx.x * kSlicesPerBlock + threadIdx.x / kWave;
+    const int lane = threadIdx.x % kWave;
+    if (s >= nslices) return;
+    const int r = s * kSlice + lane;
+    const long long base = sptr[s];
+    const int wd = (int)((sptr[s + 1] - base) / kSlice);
+    bool bad = false;
+    for (int k = 0; k < 4 * words; k += 4) {
+        int c[4];
+        double v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            c[u] = k + u < wd ? col[base + (long long)(k + u) * kSlice + lane] : -1;
+            v[u] = k + u < wd ? val[base + (long long)(k + u) * kSlice + lane] : 0.0;
+        }
+        unsigned int w = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            unsigned int h = kCodePad;
+            if (c[u] >= 0) {
+                const unsigned long long kk = pair_key(c[u] - r, v[u]);
+                int t = pair_slot(kk);
+                for (int q = 0; q < kPairSlots && key[t] != kk && key[t] != 0; ++q) t = (t + 1) & (kPairSlots - 1);
+                const bool same = key[t] == kk && po[t] == c[u] - r && pv[t] == __double_as_longlong(v[u]);
+                bad = bad || !same;
+                h = (unsigned int)pc[t];
+            }
+            w |= h << (8 * u);
+        }
+        d[((size_t)s * words + k / 4) * kSlice + lane] = w;
+    }
+    if (bad) g->misfit = 1;
+}
+
+// b = fl(r); optionally x = first sweep from zero
 __global__ void k_enter(int n, const double *__restrict__ r, int smoother, float w, const float *__restrict__ d,
                         float *__restrict__ b, float *__restrict__ x, float c2, float *__restrict__ dcheb) {
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
@@ -525,6 +714,11 @@ __global__ __launch_bounds__(256) void k_gemv_m(int n, const double *__restrict_
 template <int kSm, bool kPro, bool kOut, class MT>
 void launch_sweep_m(const DevSELL &S, const MT *val, float w, const int *agg, const float *xc, const float *b,
                     const float *x, float *xout, double *out64, const double *r64, double *partials) {
+    if constexpr (!kPro && std::is_same_v<MT, float>)
+        if (S.code) {
+            launch_coded<float>(S, CodedSweep<float, kSm, kOut>{b, x, xout, out64, r64, w}, partials);
+            return;
+        }
     const int grid = div_up(S.nslices, kSlicesPerBlock);
     // the last level-0 sweep (z in FP64) precedes the FP64 PCG SpMV, which
     // shares the column indices: they are loaded with ordinary loads and stay
@@ -565,6 +759,7 @@ static bool grp_level(const DevSELL &S, const DevCSR *A) {
 // offsets where the level has them
 static double low_matrix_bytes(const DevSELL &S, const LowMatrix &M) {
     const int vb = M.kind == kLowF32 ? 4 : 2;
+    if (S.code && M.kind == kLowF32) return coded_bytes(S);
     return M.dcol ? (double)S.nnz * (vb + 2) + 4.0 * (S.n + 1) : matrix_bytes(S.nnz, S.n, vb);
 }
 
@@ -596,13 +791,45 @@ void low_values(const DevSELL &S, const DevCSR &A, int kind, LowMatrix &out, boo
     // last-level cache and its smaller levels through the fused restriction:
     // building them there cost 0.8 ms of setup and saved nothing.
     out.dcol = nullptr;
-    if (!col16 || !col16_enabled() || ne == 0 || grp_level(S, &A)) return;
+    if (!col16 || !col16_enabled() || ne == 0 || grp_level(S, &A) || (S.code && kind == kLowF32)) return;
     int *misfit = arena().alloc_n<int>(1);
     unsigned int *d = col16_launch(S, misfit);
     int h = 1;
     HZ_CHECK(hipMemcpyAsync(&h, misfit, sizeof(int), hipMemcpyDeviceToHost, stream()));
     HZ_CHECK(hipStreamSynchronize(stream()));
     if (h == 0) out.dcol = d;
+}
+
+bool codes_build(DevSELL &S) {
+    if (S.n >= 1 << 28) return false;   // byte offsets of FP64 vectors in 31 bits
+    PairTable *g = arena().alloc_n<PairTable>(1);
+    unsigned char *code = arena().alloc_n<unsigned char>(kPairSlots);
+    auto *tab = arena().alloc_n<CodeEntry<double>>(kCodes);
+    auto *tabf = arena().alloc_n<CodeEntry<float>>(kCodes);
+    hipStream_t st = stream();
+    HZ_CHECK(hipMemsetAsync(g, 0, sizeof(PairTable), st));
+    k_code_pairs<<<div_up(S.nslices, kSlicesPerBlock * kPairRun), kBlock, 0, st>>>(S.nslices, S.sptr, S.col, S.val, g);
+    HZ_LAUNCH_CHECK();
+    k_code_table<<<1, kPairSlots, 0, st>>>(g, tab, tabf, code);
+    HZ_LAUNCH_CHECK();
+    int h[3] = {0, 0, 0};   // count, misfit, widest
+    HZ_CHECK(hipMemcpyAsync(h, &g->count, sizeof(h), hipMemcpyDeviceToHost, st));
+    HZ_CHECK(hipStreamSynchronize(st));
+    // slices of much the same width (a regular grid's): their padding to the
+    // widest one at most doubles the entries
+    const int words = (h[2] + 3) / 4;
+    if (h[0] > kCodePad || h[2] == 0 || 4LL * words * kSlice * S.nslices > 2 * S.nent) return false;
+    unsigned int *d = arena().alloc_n<unsigned int>((size_t)words * kSlice * S.nslices);
+    k_code_fill<<<div_up(S.nslices, kSlicesPerBlock), kBlock, 0, st>>>(S.nslices, S.sptr, S.col, S.val, g, code, words, d);
+    HZ_LAUNCH_CHECK();
+    HZ_CHECK(hipMemcpyAsync(h, &g->count, sizeof(h), hipMemcpyDeviceToHost, st));
+    HZ_CHECK(hipStreamSynchronize(st));
+    if (h[1]) return false;
+    S.code = d;
+    S.cwords = words;
+    S.ctab = tab;
+    S.ctabf = tabf;
+    return true;
 }
 
 bool col16_enabled() {
@@ -648,8 +875,8 @@ void sweep_m(const DevSELL &S, const LowMatrix &M, int smoother, float w, const 
              const float *b, const float *x, float *xout, double *out64, const double *r64, double *dot_out,
              const ReduceWs &ws) {
     if (S.n == 0) return;
-    count_bytes(matrix_bytes(S.nnz, S.n, M.kind == kLowF32 ? 4 : 2) + 12.0 * S.n + (agg ? 4.0 * S.n : 0.0) +
-                (out64 ? 12.0 * S.n : 0.0));
+    count_bytes((S.code && !agg ? low_matrix_bytes(S, M) : matrix_bytes(S.nnz, S.n, M.kind == kLowF32 ? 4 : 2)) + 12.0 * S.n +
+                (agg ? 4.0 * S.n : 0.0) + (out64 ? 12.0 * S.n : 0.0));
     double *partials = out64 ? ws.dots() : nullptr;
     if (M.kind == kLowF32) {
         const float *v = static_cast<const float *>(M.sell);
@@ -672,7 +899,9 @@ void residual_m(const DevSELL &S, const LowMatrix &M, const float *b, const floa
     const unsigned int *dcol = M.dcol;
     count_bytes(low_matrix_bytes(S, M) + 12.0 * S.n);
     const int grid = div_up(S.nslices, kSlicesPerBlock);
-    if (grp_level(S, A)) {
+    if (S.code && M.kind == kLowF32) {
+        launch_coded<float>(S, CodedResidual<float>{b, x, w});
+    } else if (grp_level(S, A)) {
         constexpr int G = 16;
         const int g = div_up((long)S.n * G, kBlock);
         if (M.kind == kLowF32)
@@ -762,8 +991,15 @@ void cheby_apply_m(const DevSELL &S, const DevCSR &A, const LowMatrix &M, const 
         // product took 42.4 us on the int32 columns that product leaves in the
         // last-level cache, 40.0 us on the offsets (128^3 level 0).
         const unsigned int *dcol = (last64 && !S.pcol) ? nullptr : M.dcol;
-        count_bytes((dcol ? low_matrix_bytes(S, M) : matrix_bytes(S.nnz, S.n, M.kind == kLowF32 ? 4 : 2)) +
+        const bool coded = S.code && M.kind == kLowF32;
+        count_bytes((dcol || coded ? low_matrix_bytes(S, M) : matrix_bytes(S.nnz, S.n, M.kind == kLowF32 ? 4 : 2)) +
                     24.0 * S.n + (last64 ? 16.0 * S.n : 0.0));
+        if (last64 && coded) {
+            launch_coded<float>(S, CodedCheb<float, true>{diag, b, x, nullptr, dwork, out64, r64, (float)c1, (float)c2},
+                                ws.dots());
+            if (dot_out) finish_dot(ws, grid, dot_out);
+            return;
+        }
         if (last64 && dcol) {
             if (M.kind == kLowF32)
                 k_cheb_step_m<true, float, unsigned int><<<grid, kBlock, 0, stream()>>>(
@@ -798,6 +1034,9 @@ void cheby_apply_m(const DevSELL &S, const DevCSR &A, const LowMatrix &M, const 
                 k_cheb_step_grp_m<G, unsigned short><<<div_up((long)S.n * G, kBlock), kBlock, 0, stream()>>>(
                     S.n, A.ia, A.ja, static_cast<const unsigned short *>(M.csr), diag, (float)c1, (float)c2, b, x, xt,
                     dwork);
+        } else if (coded) {
+            launch_coded<float>(S, CodedCheb<float, false>{diag, b, x, xt, dwork, nullptr, nullptr, (float)c1,
+                                                           (float)c2});
         } else if (M.kind == kLowF32 && dcol) {
             k_cheb_step_m<false, float, unsigned int><<<grid, kBlock, 0, stream()>>>(
                 S.n, S.nslices, S.sptr, dcol, static_cast<const float *>(M.sell), diag, (float)c1, (float)c2, b, x,

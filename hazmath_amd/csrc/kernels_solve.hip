@@ -12,7 +12,7 @@
 #include <rocprim/device/device_scan.hpp>
 #include <rocprim/device/device_radix_sort.hpp>
 
-#include "hz_internal.h"
+#include "coded.hpp"
 
 namespace hz {
 
@@ -814,9 +814,10 @@ void sell_from_csr(const DevCSR &A, DevSELL &S, bool drop_zeros) {
     }
 }
 
-// matrix stream of an FP64 SELL launch: 2-byte columns where it reads the
-// paired offsets
+// matrix stream of an FP64 SELL launch: a byte an entry where it reads the
+// codes, 2-byte columns where it reads the paired offsets
 static double sell_bytes(const DevSELL &S, bool paired) {
+    if (S.code) return coded_bytes(S);
     return paired ? (double)S.nnz * 10 + 4.0 * (S.n + 1) : matrix_bytes(S.nnz, S.n);
 }
 
@@ -830,6 +831,12 @@ void spmv(const DevSELL &S, const double *x, double *y, double *dot_out, const R
     const int grid = div_up(S.nslices, kSlicesPerBlock);
     if (dot_out) {
         if (timer) timer->begin();
+        if (S.code) {
+            launch_coded<double>(S, CodedProduct{x, y}, ws.dots());
+            if (timer) timer->end();
+            finish_dot(ws, grid, dot_out);
+            return;
+        }
         // the PCG's SpMV: masked rounds, the second half of each with ordinary
         // loads that stay in the last-level cache for the cycle's residual
         // (ahead of an FP32 cycle: every column index, no value)
@@ -859,6 +866,11 @@ void residual(const DevSELL &S, const double *b, const double *x, double *w, Lau
     if (S.n == 0) return;
     count_bytes(sell_bytes(S, S.pcol) + 24.0 * S.n);
     if (timer) timer->begin();
+    if (S.code) {
+        launch_coded<double>(S, CodedResidual<double>{b, x, w});
+        if (timer) timer->end();
+        return;
+    }
     const int g = div_up(S.nslices, kSlicesPerBlock);
     // a matrix that fits the 256 MB last-level cache with room to spare is
     // loaded with ordinary loads: the same level's post-sweep, after the
@@ -883,6 +895,11 @@ namespace {
 template <int kSm, bool kProlong, bool kDot>
 void launch_sweep_sm(const DevSELL &S, double w, const int *agg, const double *xc, double alpha,
                      const double *alpha_dev, const double *b, const double *x, double *xout, double *partials) {
+    if constexpr (!kProlong)
+        if (S.code) {
+            launch_coded<double>(S, CodedSweep<double, kSm, kDot>{b, x, xout, nullptr, nullptr, w}, partials);
+            return;
+        }
     const int grid = div_up(S.nslices, kSlicesPerBlock);
     const bool paired = !kProlong && S.pcol;
     by_round(S, [&](auto u) {
@@ -901,7 +918,7 @@ template <bool kProlong, bool kDot>
 void launch_sweep(const DevSELL &S, int smoother, double w, const int *agg, const double *xc,
                   double alpha, const double *alpha_dev, const double *b, const double *x, double *xout,
                   double *partials) {
-    count_bytes(sell_bytes(S, !kProlong && S.pcol) + 24.0 * S.n + (kProlong ? 4.0 * S.n : 0.0));
+    count_bytes((kProlong ? matrix_bytes(S.nnz, S.n) : sell_bytes(S, S.pcol)) + 24.0 * S.n + (kProlong ? 4.0 * S.n : 0.0));
     if (smoother == HZ_SMOOTHER_L1DIAG)
         launch_sweep_sm<HZ_SMOOTHER_L1DIAG, kProlong, kDot>(S, w, agg, xc, alpha, alpha_dev, b, x, xout, partials);
     else
