@@ -25,7 +25,7 @@ namespace hz {
 namespace {
 
 constexpr int kDeg = 31, kSep = 3, kMaxTypes = 5;
-constexpr int kChunk = 31 * 128;     // outputs per GPU thread (whole 31-step cycles)
+constexpr int kChunk = 64 * 64;      // outputs per wavefront: 64 steps of 64 outputs
 constexpr int kBlock = 256;
 
 using Mat = std::vector<uint32_t>;   // 31 x 31, row-major
@@ -131,30 +131,85 @@ void advance_libc_state(const LibcState &st, const uint32_t *window_K, long K) {
     setstate(st.buf);
 }
 
-// Each thread expands one chunk of the stream from its start window and
-// writes the shuffle targets H_k = k + o_k / (RAND_MAX / (n - k) + 1).
-__global__ void k_glibc_targets(long K, int n, int nchunks, const uint32_t *__restrict__ starts,
-                                int *__restrict__ H) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nchunks) return;
-    uint32_t w[kDeg];
+// A wavefront expands one chunk of the stream from its start window, 64 outputs
+// a step: output t of a step is a fixed combination of the window's 31 words
+// (row t of the coefficients, from the recurrence itself), so the lanes form
+// their outputs side by side and the last 31 are the next window.  Each writes
+// its shuffle target H_k = k + o_k / (RAND_MAX / (n - k) + 1).  A thread a chunk,
+// one output after the other, took 430 us however few the rows; this 16-28.
+__global__ __launch_bounds__(kWave) void k_glibc_targets(long K, int n, const uint32_t *__restrict__ starts,
+                                                         int *__restrict__ H) {
+    __shared__ uint32_t coef[kWave][kDeg + 1], win[kDeg + 1];
+    const int lane = threadIdx.x;
+    for (int t = 0; t < kWave; ++t) {
+        if (lane < kDeg) {
+            const uint32_t far = t < kDeg ? (lane == t) : coef[t - kDeg][lane];
+            const uint32_t near = t < kSep ? (lane == kDeg - kSep + t) : coef[t - kSep][lane];
+            coef[t][lane] = far + near;
+        }
+        __syncthreads();
+    }
+    uint32_t c[kDeg];
 #pragma unroll
-    for (int i = 0; i < kDeg; ++i) w[i] = starts[(long)t * kDeg + i];
-    long k = (long)t * kChunk;
-    for (int cyc = 0; cyc < kChunk / kDeg; ++cyc) {
+    for (int j = 0; j < kDeg; ++j) c[j] = coef[lane][j];
+    if (lane < kDeg) win[lane] = starts[(long)blockIdx.x * kDeg + lane];
+    __syncthreads();
+    const long k0 = (long)blockIdx.x * kChunk, k1 = K < k0 + kChunk ? K : k0 + kChunk;
+    for (long kb = k0; kb < k1; kb += kWave) {
+        uint32_t e = 0;
 #pragma unroll
-        for (int i = 0; i < kDeg; ++i) {
-            const uint32_t e = w[i] + w[(i + kDeg - kSep) % kDeg];
-            w[i] = e;
-            const long kk = k + i;
-            if (kk < K) {
-                const int o = (int)(e >> 1);
-                const int rem = n - (int)kk;
-                H[kk] = (int)kk + o / (RAND_MAX / rem + 1);
+        for (int j = 0; j < kDeg; ++j) e += c[j] * win[j];
+        __syncthreads();
+        if (lane >= kWave - kDeg) win[lane - (kWave - kDeg)] = e;
+        __syncthreads();
+        const long k = kb + lane;
+        if (k < k1) H[k] = (int)k + (int)(e >> 1) / (RAND_MAX / (n - (int)k) + 1);
+    }
+}
+
+// The shuffle of up to kLdsRows positions by one workgroup: the rounds of
+// k_reserve / k_commit with the reservations, targets and positions in LDS (8
+// bytes a row), a thread's open iterations in a bit mask, a barrier between
+// the two halves of a round.  Keys: round, then the lower index first; a round
+// commits at least the lowest open iteration, so there are fewer than 65,536.
+// 16,129 rows: 51 us against 24-32 rounds of two launches and a wait every
+// eighth (about 250).
+constexpr int kLdsThreads = 1024, kLdsRows = 19 * kLdsThreads;
+__global__ __launch_bounds__(kLdsThreads) void k_shuffle_lds(int n, const int *__restrict__ H,
+                                                             int *__restrict__ perm_out) {
+    extern __shared__ uint32_t s_res[];
+    unsigned short *tgt = reinterpret_cast<unsigned short *>(s_res + n);
+    unsigned short *perm = tgt + n;
+    const int K = n - 1;
+    uint32_t open = 0;
+    for (int j = 0, i = threadIdx.x; i < n; ++j, i += kLdsThreads) {
+        s_res[i] = 0;
+        perm[i] = (unsigned short)i;
+        tgt[i] = (unsigned short)(i < K ? H[i] : i);
+        if (i < K) open |= 1u << j;
+    }
+    for (uint32_t round = 1; round < 65536u; ++round) {
+        __syncthreads();
+        for (uint32_t m = open; m; m &= m - 1) {
+            const int i = threadIdx.x + kLdsThreads * (__ffs(m) - 1);
+            const uint32_t key = (round << 16) | (0xFFFFu - (uint32_t)i);
+            atomicMax(&s_res[i], key);
+            atomicMax(&s_res[tgt[i]], key);
+        }
+        __syncthreads();
+        for (uint32_t m = open; m; m &= m - 1) {
+            const int j = __ffs(m) - 1, i = threadIdx.x + kLdsThreads * j, h = tgt[i];
+            const uint32_t key = (round << 16) | (0xFFFFu - (uint32_t)i);
+            if (s_res[i] == key && s_res[h] == key) {   // no other iteration of the round holds either position
+                const unsigned short a = perm[i];
+                perm[i] = perm[h];
+                perm[h] = a;
+                open &= ~(1u << j);
             }
         }
-        k += kDeg;
+        if (!__syncthreads_or(open != 0)) break;
     }
+    for (int i = threadIdx.x; i < n; i += kLdsThreads) perm_out[i] = perm[i];
 }
 
 __global__ void k_iota(int n, int *__restrict__ p) {
@@ -240,13 +295,24 @@ void hec_turn_order(int n, int *perm_dev, int rng_source) {
 
     uint32_t *dstarts = arena().alloc_n<uint32_t>(starts.size() + 1);
     int *H = arena().alloc_n<int>((size_t)K + 1);
+    HZ_CHECK(hipMemcpyAsync(dstarts, starts.data(), sizeof(uint32_t) * starts.size(), hipMemcpyHostToDevice, s));
+    k_glibc_targets<<<nchunks, kWave, 0, s>>>(K, n, dstarts, H);
+    HZ_LAUNCH_CHECK();
+    if (n <= kLdsRows) {
+        const size_t lds = 8 * (size_t)n;
+        HZ_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_shuffle_lds),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, 8 * kLdsRows));
+        k_shuffle_lds<<<1, kLdsThreads, lds, s>>>(n, H, perm_dev);
+        HZ_LAUNCH_CHECK();
+        HZ_CHECK(hipStreamSynchronize(s));
+        advance_libc_state(st, wk, K);
+        return;
+    }
     int *done = arena().alloc_n<int>((size_t)K + 1);
     unsigned long long *R = arena().alloc_n<unsigned long long>((size_t)n + 1);
     int *remaining = arena().alloc_n<int>(1);
-    HZ_CHECK(hipMemcpyAsync(dstarts, starts.data(), sizeof(uint32_t) * starts.size(), hipMemcpyHostToDevice, s));
     HZ_CHECK(hipMemsetAsync(done, 0, sizeof(int) * (size_t)K, s));
     HZ_CHECK(hipMemsetAsync(R, 0, sizeof(unsigned long long) * (size_t)n, s));
-    k_glibc_targets<<<(nchunks + kBlock - 1) / kBlock, kBlock, 0, s>>>(K, n, nchunks, dstarts, H);
     k_iota<<<grid_for(n), kBlock, 0, s>>>(n, perm_dev);
     HZ_LAUNCH_CHECK();
     const int g = grid_for(K);

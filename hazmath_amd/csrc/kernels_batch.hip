@@ -59,7 +59,7 @@ constexpr int kSlicesPerBlock = kBlock / kWave;
 // level-0 rows per reduction chunk (never across systems).  A chunk is one
 // workgroup's 16 double2 a thread, loaded four at a time; at 2,048 rows, one
 // double at a time, the dots took 24 us and the update 43 on 693,356 rows (of
-// 8 columns) against CHUNKFIG.
+// 8 columns) against 8 and 18.
 constexpr int kChunkRows = 1024;
 constexpr float kSmallRealF = 1e-20f;
 constexpr int kMaxRestart = 20;        // MAX_RESTART, include/macro.h:33

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 from hazmath_amd import capi, problems
-from test_gpu_parity import _set_precision, _solve_both
+from test_gpu_parity import _hierarchies, _set_precision, _solve_both
 
 pytestmark = pytest.mark.gpu
 
@@ -370,3 +370,17 @@ def test_entry_codes_bitexact(lib, libc, monkeypatch, n, offsets, classes, diags
     assert np.array_equal(out["0"][1], out["1"][1])
     saved = (out["0"][2] - out["1"][2]) / (A.ja.size * out["1"][0])
     assert (saved > 10.5) == coded
+
+
+# outputs of the generator: below and at a step of 64, a whole chunk of 4,096 and one more; rows: the most the shuffle in
+# LDS takes, and one more
+@pytest.mark.parametrize("n", [3, 65, 66, 4097, 4098, 19456, 19457])
+def test_hec_turn_order_sizes_vs_oracle(lib, orc, libc, n):
+    """The aggregates of a chain depend on every position of the turn order: the same as the oracle's, whose order is
+    the loop over rand(), and rand() goes on from the same place."""
+    A = capi.HostCSR(*_banded(n, [1], 97, 1))
+    (lg, _, rg), (lo, _, ro) = _hierarchies(lib, orc, libc, A, capi.HEC, 0.0, coarse_dof=2)
+    assert rg == ro and len(lg) == len(lo)
+    for g, o in zip(lg, lo):
+        if "agg" in o:
+            assert np.array_equal(g["agg"], o["agg"])
