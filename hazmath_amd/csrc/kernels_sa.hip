@@ -297,8 +297,8 @@ __global__ void k_rap_rows(int r0, int r1, const int *__restrict__ rows, const l
 // A entry) pairs are staged in LDS in traversal order, whole A rows at a
 // time and at most max_pairs pairs per stage, with the prefix of their P-row
 // lengths; each stage's candidates (q1, q2, q3) are then taken 64 at a time
-// in that order.  The lanes of a round are grouped by column (one ballot per
-// distinct column); a column's first lane folds the round's values of that
+// in that order.  The lanes of a round are grouped by column (a bit mask a
+// slot of the column table); a column's first lane folds the round's values of that
 // column into the column's running sum in lane order, so every sum keeps the
 // sequential order; new columns take output slots in order of first
 // appearance, after the diagonal (slot 0, summed from 0.0).  The column table
@@ -306,8 +306,13 @@ __global__ void k_rap_rows(int r0, int r1, const int *__restrict__ rows, const l
 // the rows it cannot take (more than max_cols columns, or one A row longer
 // than a stage); the per-thread kernel takes those and the fill pass skips
 // them.
-// 256 pairs and 256 columns keep the LDS at 12.8 KB: twelve single-wavefront
-// workgroups per CU hide the rounds' gathers from P (with 512 / 512, six).
+// A round's cost is its chain of LDS steps, so a round is a few: the column's
+// slot, one atomic that tells each lane which lanes share it, the sums.  With a
+// ballot a column, reads one by one, and a stage's pairs fetched a lane an A
+// row, the products of the 250,047-row and 2,048,383-row anisotropic hierarchies
+// took 2.08 ms (432 rows of 59-entry A rows), 0.78 (15,470 rows) and 5.68 ms
+// (174,080), 2.27 (15,218); now 0.94, 0.62, 4.32, 1.43.  256 pairs and 256
+// columns keep the LDS at 17.4 KB: nine single-wavefront workgroups a CU.
 constexpr int kRapwPairs = 256;
 constexpr double kRapSlotBytes = 4e9;   // slots of the one-pass form: at most 4 GB
 constexpr int kRapwCols = 256;
@@ -329,7 +334,7 @@ __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
     return v;
 }
 
-// kCols: the table's columns and the stage's pairs (LDS 50 kCols bytes)
+// kCols: the table's columns and the stage's pairs (LDS 66 kCols bytes and 1 KB)
 template <bool kFill, bool kSlots = false, int kCols = kRapwCols>
 __global__ __launch_bounds__(kWave) void k_rapw(int nc, const int *__restrict__ ria, const int *__restrict__ rja,
                                                 const double *__restrict__ rval, const int *__restrict__ aia,
@@ -341,8 +346,10 @@ __global__ __launch_bounds__(kWave) void k_rapw(int nc, const int *__restrict__ 
     constexpr int kPairs = kCols, kHash = 2 * kCols;   // at most kCols + 64 keys: probing ends
     __shared__ int s_pst[kPairs];              // P-row start of each pair
     __shared__ int s_off[kPairs];          // its P-row length, then its first candidate
+    __shared__ int s_first[kWave], s_a0[kWave];   // of the A rows being staged: first pair, first entry
     __shared__ double s_ra[kFill ? kPairs : 1];
     __shared__ int s_key[kHash], s_pos[kHash];
+    __shared__ unsigned long long s_mask[kHash];   // lanes of a round with the slot's column
     __shared__ double s_val[kFill ? kHash : 1];
     __shared__ double s_rv[kFill ? kWave : 1];
     const int lane = threadIdx.x;
@@ -353,6 +360,7 @@ __global__ __launch_bounds__(kWave) void k_rapw(int nc, const int *__restrict__ 
     for (int t = lane; t < kHash; t += kWave) {
         s_key[t] = -1;
         s_pos[t] = -1;
+        s_mask[t] = 0ull;
     }
     __syncthreads();
     if (lane == 0) {
@@ -386,18 +394,49 @@ __global__ __launch_bounds__(kWave) void k_rapw(int nc, const int *__restrict__ 
                 if (np == 0) big = true;   // one A row longer than a stage
                 break;
             }
-            if (lane < nfit) {
-                const int first = np + incl - alen;
-                for (int k = 0; k < alen; ++k) {
-                    const int q2 = a0 + k;
-                    const int i2 = aja[q2];
-                    const int ps = pia[i2];
-                    s_pst[first + k] = ps;
-                    s_off[first + k] = pia[i2 + 1] - ps;
-                    if (kFill) s_ra[first + k] = r * aval[q2];
+            // the rows' entries over all lanes (a lane a row walked 59-entry
+            // rows one dependent load after the other, with 4 lanes at work)
+            const int tot = __shfl(incl, nfit - 1, kWave);
+            s_first[lane] = incl - alen;
+            s_a0[lane] = a0;
+            if (kFill) s_rv[lane] = r;
+            __syncthreads();
+            constexpr int kEach = kPairs / kWave;
+            int q2[kEach], ps[kEach], pe[kEach], row[kEach];
+#pragma unroll
+            for (int u = 0; u < kEach; ++u) {
+                const int idx = u * kWave + lane;
+                int lo = 0, hi = nfit - 1;   // last row whose first entry is <= idx
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (s_first[mid] <= idx) lo = mid;
+                    else hi = mid - 1;
                 }
+                row[u] = lo;
+                q2[u] = idx < tot ? s_a0[lo] + (idx - s_first[lo]) : -1;
             }
-            np += __shfl(incl, nfit - 1, kWave);
+            int i2[kEach];
+            double av[kEach];
+#pragma unroll
+            for (int u = 0; u < kEach; ++u) {
+                i2[u] = q2[u] >= 0 ? aja[q2[u]] : -1;
+                av[u] = kFill && q2[u] >= 0 ? aval[q2[u]] : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < kEach; ++u) {
+                ps[u] = i2[u] >= 0 ? pia[i2[u]] : 0;
+                pe[u] = i2[u] >= 0 ? pia[i2[u] + 1] : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < kEach; ++u) {
+                const int idx = u * kWave + lane;
+                if (idx >= tot) continue;
+                s_pst[np + idx] = ps[u];
+                s_off[np + idx] = pe[u] - ps[u];
+                if (kFill) s_ra[np + idx] = s_rv[row[u]] * av[u];
+            }
+            __syncthreads();
+            np += tot;
             q1 += nfit;
             if (nfit < kWave) break;   // the stage is full or the row is done
         }
@@ -413,13 +452,14 @@ __global__ __launch_bounds__(kWave) void k_rapw(int nc, const int *__restrict__ 
             L += __shfl(incl, kWave - 1, kWave);
         }
         __syncthreads();
-        // 2) the stage's candidates in rounds of a wavefront
-        for (int base = 0; !big && base < L; base += kWave) {   // uniform
+        // 2) the stage's candidates in rounds of a wavefront, the next round's
+        // gathers in flight while this one's columns are grouped and summed
+        int ncol = -1;
+        double npv = 0.0, nra = 0.0;
+        const auto gather = [&](int base) {
             const int p = base + lane;
-            const bool has = p < L;
-            int col = -1;
-            double v = 0.0;
-            if (has) {
+            ncol = -1;
+            if (p < L) {
                 int lo = 0, hi = np - 1;   // last pair whose first candidate is <= p
                 while (lo < hi) {
                     const int mid = (lo + hi + 1) >> 1;
@@ -427,29 +467,38 @@ __global__ __launch_bounds__(kWave) void k_rapw(int nc, const int *__restrict__ 
                     else hi = mid - 1;
                 }
                 const int q3 = s_pst[lo] + (p - s_off[lo]);
-                col = pja[q3];
-                if (kFill) v = s_ra[lo] * pval[q3];
+                ncol = pja[q3];
+                if (kFill) {
+                    npv = pval[q3];
+                    nra = s_ra[lo];
+                }
             }
+        };
+        gather(0);
+        for (int base = 0; !big && base < L; base += kWave) {   // uniform
+            const bool has = base + lane < L;
+            const int col = ncol;
+            const double v = kFill && has ? nra * npv : 0.0;
+            gather(base + kWave);
             if (kFill) s_rv[lane] = v;
-            // the lanes of each distinct column (one ballot per column)
-            unsigned long long mine = 0;
-            for (unsigned long long todo = __ballot(has); todo;) {   // uniform
-                const int l = __builtin_ctzll(todo);
-                const int c = __builtin_amdgcn_readlane(col, l);
-                const unsigned long long m = __ballot(has && col == c);
-                if (has && col == c) mine = m;
-                todo &= ~m;
-            }
-            const bool lead = has && __builtin_ctzll(mine) == lane;
+            // the lanes of each distinct column: they find its slot and set their
+            // bits there; the lowest of them leads (a ballot a column took 20-40
+            // times as many instructions)
             unsigned slot = 0;
-            if (lead) {   // distinct columns: only the first lane of each probes
+            if (has) {
                 slot = rapw_hash<kHash>(col);
                 while (true) {
                     const int prev = atomicCAS(&s_key[slot], -1, col);
                     if (prev == -1 || prev == col) break;
                     slot = (slot + 1) & (kHash - 1u);
                 }
+                atomicOr(&s_mask[slot], 1ull << lane);
             }
+            __syncthreads();
+            const unsigned long long mine = has ? s_mask[slot] : 0ull;
+            __syncthreads();
+            const bool lead = has && __builtin_ctzll(mine) == lane;
+            if (lead) s_mask[slot] = 0ull;
             const bool fresh = lead && s_pos[slot] < 0;
             const unsigned long long mf = __ballot(fresh);
             if (fresh) s_pos[slot] = next + __popcll(mf & ((1ull << lane) - 1ull));
@@ -457,8 +506,20 @@ __global__ __launch_bounds__(kWave) void k_rapw(int nc, const int *__restrict__ 
             __syncthreads();
             if (kFill && lead) {
                 double acc = fresh ? v : s_val[slot] + v;
-                for (unsigned long long rest = mine & (mine - 1); rest; rest &= rest - 1)
-                    acc = acc + s_rv[__builtin_ctzll(rest)];
+                for (unsigned long long rest = mine & (mine - 1); rest;) {   // four reads at once
+                    constexpr int kAtOnce = 4;
+                    double rv[kAtOnce];
+                    bool on[kAtOnce];
+#pragma unroll
+                    for (int u = 0; u < kAtOnce; ++u) {
+                        on[u] = rest != 0;
+                        rv[u] = s_rv[on[u] ? __builtin_ctzll(rest) : lane];
+                        rest &= rest - 1;   // 0 stays 0
+                    }
+#pragma unroll
+                    for (int u = 0; u < kAtOnce; ++u)
+                        if (on[u]) acc = acc + rv[u];
+                }
                 s_val[slot] = acc;
             }
             if (next > max_cols) big = true;   // uniform; at most max_cols + 64 keys so far
