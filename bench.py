@@ -59,7 +59,9 @@ def _counter_rows(outdir):
 
 # fine-level kernels whose HBM traffic the counter passes report: the graded
 # SpMV, and the V-cycle's fine-level residual and last sweep (largest grid)
-TRAFFIC_KERNELS = {"spmv": r"\bk_spmv<true", "residual": r"\bk_residual<", "sweep_dot": r"\bk_sweep<10, false, true"}
+# over columns and values, or over entry codes (k_coded with the operation as its last argument)
+TRAFFIC_KERNELS = {"spmv": r"\bk_spmv<true|\bk_coded<.*CodedProduct", "residual": r"\bk_residual<|\bk_coded<.*CodedResidual",
+                   "sweep_dot": r"\bk_sweep<10, false, true|\bk_coded<.*CodedSweep<double, 10, true>"}
 
 
 def measure_traffic(a):
