@@ -29,20 +29,18 @@ __global__ __launch_bounds__(kCodedBlock) void k_coded(int n, int nslices, int w
     __shared__ CodeEntry<T> tab[kCodes];
     __shared__ double sh[kCodedBlock / kWave];
     const int blk = xcd_block_id();
-    const int s = blk * kCodedSlices + threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const int r = s * kSlice + lane;
-    const bool in = r < n;
-    const code8 *c = code + (size_t)min(s, nslices - 1) * words * kSlice + lane;
+    const CodedLane l = coded_lane(blk * kCodedSlices + threadIdx.x / kWave, threadIdx.x % kWave, n, nslices, words,
+                                   sizeof(T));
+    const int r = l.row;
     const auto load = [&](int k, unsigned int (&w)[U / 4]) {
 #pragma unroll
-        for (int u = 0; u < U / 4; ++u) w[u] = k + u < words ? (unsigned int)c[(k + u) * kSlice] : 0xFFFFFFFFu;
+        for (int u = 0; u < U / 4; ++u) w[u] = coded_word(l, code, k + u, words);
     };
     unsigned int w[U / 4];
     load(0, w);
-    if (in) op.begin(r);
+    if (l.in) op.begin(r);
     for (int i = threadIdx.x; i < kCodes; i += kCodedBlock) tab[i] = table[i];
     __syncthreads();
-    const unsigned int rb = (unsigned int)(min(r, n - 1) * sizeof(T));   // padding reads the row's own entry
     for (int k = 0; k < words; k += U / 4) {
         if (k > 0) load(k, w);
         T vv[U], xx[U];
@@ -50,11 +48,11 @@ __global__ __launch_bounds__(kCodedBlock) void k_coded(int n, int nslices, int w
         bool pad[U], diag[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const unsigned int h = (w[u / 4] >> (8 * (u % 4))) & 0xFFu;
+            const unsigned int h = coded_entry(w[u / 4], u % 4);
             const CodeEntry<T> e = tab[h];
-            pad[u] = h == kCodePad;
+            pad[u] = h == (unsigned int)kCodePad;
             diag[u] = e.off == 0;
-            at[u] = rb + (unsigned int)e.off;
+            at[u] = l.base + (unsigned int)e.off;   // padding reads the row's own entry
             vv[u] = e.val;
         }
 #pragma unroll
@@ -63,7 +61,7 @@ __global__ __launch_bounds__(kCodedBlock) void k_coded(int n, int nslices, int w
 #pragma unroll
         for (int u = 0; u < U; ++u) op.entry(pad[u], diag[u], vv[u], xx[u]);
     }
-    const double prod = in ? op.end(r) : 0.0;
+    const double prod = l.in ? op.end(r) : 0.0;
     if constexpr (Op::kDot) {
         const double bs = block_sum<kCodedBlock>(prod, sh);
         if (threadIdx.x == 0) partials[blk] = bs;

@@ -10,6 +10,7 @@
 #include <cstdlib>
 #include <vector>
 
+#include "coded_lane.h"
 #include "hazmath_mi355x.h"
 
 namespace hz {
@@ -176,7 +177,7 @@ __device__ __forceinline__ unsigned short f2bf(float f) {
 // padding kCodePad.  The table holds the values' own bits (FP32 cycle: those of
 // their FP32 copies).
 enum class code8 : unsigned int {};
-constexpr int kCodes = 256, kCodePad = 255;
+static_assert(kCodeRows == kSlice, "a slice of codes is a slice of the SELL copy");
 // An entry of the table: the value and the pair's column offset in bytes of a
 // vector of T, so a kernel's address is the row's plus that.
 template <class T>

@@ -334,9 +334,11 @@ def _banded(n, offsets, classes, diags):
 
 
 # pairs: 255 have codes, 256 do not; words of a row: 1, 2 (8 entries at once), 3 (16), 5 (a second round of 16: 19
-# entries); rows: 65,536 (full slices) and 65,601 (a last slice of one row)
+# entries); rows: 65,536 (full slices), 65,601 (a last slice of one row) and 65,576 (three wavefronts past a last slice
+# of 40 rows, whose entries above the diagonal would lead past the vectors)
 @pytest.mark.parametrize("n,offsets,classes,diags,coded", [
     (65601, [1], 127, 1, True), (65601, [1], 127, 2, False), (65536, [1, 50, 51], 1, 1, True),
+    (65576, [1, 30, 31], 1, 1, True),
     (65601, [1, 50, 51, 700], 2, 3, True), (65601, [1, 2, 3, 50, 51, 52, 900, 901, 902], 3, 1, True)])
 @pytest.mark.parametrize("precision", [0, 1])
 @pytest.mark.parametrize("smoother", ["jacobi", "l1", "cheb", "sgs"])
