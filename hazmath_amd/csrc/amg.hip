@@ -373,8 +373,6 @@ void amg_prepare_cycle(Hierarchy &H, const AMG_param *param) {
     cp.coarse_tol = 1e-6 * 1e-2;
     cp.maxit = param->maxit;
     const int n0 = H.lv[0].A.n;
-    int maxgrid = std::max(8192, div_up(H.lv[0].S.nslices, 4) + 1);
-    H.ws.partials = arena().alloc_n<double>((size_t)maxgrid * ReduceWs::kSlots);
     H.ws.tickets = arena().alloc_n<unsigned int>(64);
     HZ_CHECK(hipMemsetAsync(H.ws.tickets, 0, 64 * sizeof(unsigned int), stream()));
     H.sc = arena().alloc_n<PcgScalars>(1);
@@ -454,6 +452,11 @@ void amg_prepare_cycle(Hierarchy &H, const AMG_param *param) {
         }
         fused_prepare(small, kinds, cp.smoother);
     }
+    // a dot leaves a partial a workgroup: of the vector kernels, of those over
+    // level 0's slices, or of the fused kernel on level 0, whose workgroups
+    // follow from the aggregates (2,100,000 rows in pairs: 8,750, of slices 8,204)
+    H.ws.room = std::max({(int)ReduceWs::kMaxBlocks, div_up(H.lv[0].S.nslices, 4) + 1, H.lv[0].F.nblk});
+    H.ws.partials = arena().alloc_n<double>((size_t)H.ws.room * ReduceWs::kSlots);
     // the FP64 Jacobi / L1 cycle and the PCG's product read 16-bit column
     // offsets on levels of 65,536 rows or more where every offset fits: one
     // conversion a level, one wait for all of them
@@ -1012,12 +1015,11 @@ PcgResult pcg_solve(Hierarchy &H, const DevSELL &A, const double *b, double *u, 
         if (!amg_precond(H, rr_, zz_, sc_zr, first_done)) dot(m, zz_, rr_, sc_zr, H.ws);
     };
     // partials of (A p, p) and (z, r) that the next vector kernel sums itself
-    const size_t maxgrid = (size_t)std::max(8192, div_up(A.nslices, 4) + 1);
     int n_ap = 0, n_zr = 0;
     ReduceWs ws_ap = H.ws;
-    ws_ap.dot_part = arena().alloc_n<double>(maxgrid);
+    ws_ap.dot_part = arena().alloc_n<double>((size_t)H.ws.room);
     ws_ap.npart = &n_ap;
-    double *zr_part = arena().alloc_n<double>(maxgrid);
+    double *zr_part = arena().alloc_n<double>((size_t)H.ws.room);
     // the PCG update forms the preconditioner's first level-0 sweep when the
     // preconditioner is queued right behind it
     FirstSweep first;

@@ -746,7 +746,8 @@ INT hz_time_fine_kernels(INT n, INT nnz, const INT *dIA, const INT *dJA, const R
         fill(x, 1.0, n);
         fill(b, 0.5, n);
         ReduceWs ws;
-        ws.partials = arena().alloc_n<double>((size_t)std::max(8192, div_up(S.nslices, 4) + 1) * 4);
+        ws.room = std::max(8192, div_up(S.nslices, 4) + 1);
+        ws.partials = arena().alloc_n<double>((size_t)ws.room * 4);
         ws.tickets = arena().alloc_n<unsigned int>(64);
         HZ_CHECK(hipMemsetAsync(ws.tickets, 0, 64 * sizeof(unsigned int), stream()));
         hipEvent_t e0, e1;

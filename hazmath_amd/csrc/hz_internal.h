@@ -80,14 +80,23 @@ inline double matrix_bytes(long long nnz, long n, int vb = 8) { return (double)n
 constexpr int kSelfSum = 256;
 
 struct ReduceWs {
-    double *partials = nullptr;   // kMaxBlocks * kSlots
+    double *partials = nullptr;   // room * kSlots
+    int room = 0;                 // largest grid whose partials of a dot fit
     unsigned int *tickets = nullptr;
-    // when npart is set, a dot's partials go to dot_part (room for the
-    // largest grid) and stay there if they are few enough: *npart is their count, or 0 when the
-    // total was formed as usual
+    // when npart is set, a dot's partials go to dot_part (room of them) and stay
+    // there if they are few enough: *npart is their count, or 0 when the total
+    // was formed as usual
     double *dot_part = nullptr;
     int *npart = nullptr;
-    double *dots() const { return npart ? dot_part : partials; }
+    // where a launch of `grid` workgroups leaves its partials; a larger grid
+    // than there is room for is an error before the launch
+    double *dots(int grid) const {
+        if (grid > room) {
+            std::fprintf(stderr, "hazmath_mi355x: %d partials of a dot, room for %d\n", grid, room);
+            throw DeviceError{hipErrorInvalidValue, "ReduceWs::dots"};
+        }
+        return npart ? dot_part : partials;
+    }
     static constexpr int kMaxBlocks = 8192;
     static constexpr int kSlots = 4;
 };

@@ -384,7 +384,7 @@ static void fused_up_impl(const Level &L, int smoother, double w, const VT *dsm,
     const int vb = F.kind == 0 ? 8 : (F.kind == kLowF32 ? 4 : 2);
     // (the merged entries are counted as the row's own)
     count_bytes((vb + 4.0) * L.S.nnz + (8.0 + 4.0 * sizeof(VT)) * L.A.n + (out64 ? 16.0 * L.A.n : 0.0));
-    double *part = dot_out || out64 ? ws.dots() : nullptr;
+    double *part = dot_out || out64 ? ws.dots(F.nblk) : nullptr;
     const VT wgt = smoother == HZ_SMOOTHER_L1DIAG ? VT(1) : (VT)w;
     by_width(F.amax, F.awidth != nullptr, [&](auto u) {
         constexpr int U = decltype(u)::value;

@@ -877,7 +877,7 @@ void sweep_m(const DevSELL &S, const LowMatrix &M, int smoother, float w, const 
     if (S.n == 0) return;
     count_bytes((S.code && !agg ? low_matrix_bytes(S, M) : matrix_bytes(S.nnz, S.n, M.kind == kLowF32 ? 4 : 2)) + 12.0 * S.n +
                 (agg ? 4.0 * S.n : 0.0) + (out64 ? 12.0 * S.n : 0.0));
-    double *partials = out64 ? ws.dots() : nullptr;
+    double *partials = out64 ? ws.dots(div_up(S.nslices, kSlicesPerBlock)) : nullptr;
     if (M.kind == kLowF32) {
         const float *v = static_cast<const float *>(M.sell);
         if (smoother == HZ_SMOOTHER_L1DIAG)
@@ -996,7 +996,7 @@ void cheby_apply_m(const DevSELL &S, const DevCSR &A, const LowMatrix &M, const 
                     24.0 * S.n + (last64 ? 16.0 * S.n : 0.0));
         if (last64 && coded) {
             launch_coded<float>(S, CodedCheb<float, true>{diag, b, x, nullptr, dwork, out64, r64, (float)c1, (float)c2},
-                                ws.dots());
+                                ws.dots(grid));
             if (dot_out) finish_dot(ws, grid, dot_out);
             return;
         }
@@ -1004,11 +1004,11 @@ void cheby_apply_m(const DevSELL &S, const DevCSR &A, const LowMatrix &M, const 
             if (M.kind == kLowF32)
                 k_cheb_step_m<true, float, unsigned int><<<grid, kBlock, 0, stream()>>>(
                     S.n, S.nslices, S.sptr, dcol, static_cast<const float *>(M.sell), diag, (float)c1, (float)c2, b,
-                    x, nullptr, dwork, out64, r64, ws.dots());
+                    x, nullptr, dwork, out64, r64, ws.dots(grid));
             else
                 k_cheb_step_m<true, unsigned short, unsigned int><<<grid, kBlock, 0, stream()>>>(
                     S.n, S.nslices, S.sptr, dcol, static_cast<const unsigned short *>(M.sell), diag, (float)c1,
-                    (float)c2, b, x, nullptr, dwork, out64, r64, ws.dots());
+                    (float)c2, b, x, nullptr, dwork, out64, r64, ws.dots(grid));
             HZ_LAUNCH_CHECK();
             if (dot_out) finish_dot(ws, grid, dot_out);
             return;
@@ -1017,11 +1017,11 @@ void cheby_apply_m(const DevSELL &S, const DevCSR &A, const LowMatrix &M, const 
             if (M.kind == kLowF32)
                 k_cheb_step_m<true, float><<<grid, kBlock, 0, stream()>>>(
                     S.n, S.nslices, S.sptr, S.col, static_cast<const float *>(M.sell), diag, (float)c1, (float)c2, b,
-                    x, nullptr, dwork, out64, r64, ws.dots());
+                    x, nullptr, dwork, out64, r64, ws.dots(grid));
             else
                 k_cheb_step_m<true, unsigned short><<<grid, kBlock, 0, stream()>>>(
                     S.n, S.nslices, S.sptr, S.col, static_cast<const unsigned short *>(M.sell), diag, (float)c1,
-                    (float)c2, b, x, nullptr, dwork, out64, r64, ws.dots());
+                    (float)c2, b, x, nullptr, dwork, out64, r64, ws.dots(grid));
             HZ_LAUNCH_CHECK();
             if (dot_out) finish_dot(ws, grid, dot_out);
             return;

@@ -755,7 +755,7 @@ void finish_dot(const ReduceWs &ws, int grid, double *out) {
     const bool left = ws.npart && grid <= kSelfSum;
     if (ws.npart) *ws.npart = left ? grid : 0;
     if (left) return;
-    k_final_sum<<<1, kFinBlock, 0, stream()>>>(ws.dots(), grid, out);
+    k_final_sum<<<1, kFinBlock, 0, stream()>>>(ws.dots(grid), grid, out);
     HZ_LAUNCH_CHECK();
 }
 
@@ -832,7 +832,7 @@ void spmv(const DevSELL &S, const double *x, double *y, double *dot_out, const R
     if (dot_out) {
         if (timer) timer->begin();
         if (S.code) {
-            launch_coded<double>(S, CodedProduct{x, y}, ws.dots());
+            launch_coded<double>(S, CodedProduct{x, y}, ws.dots(grid));
             if (timer) timer->end();
             finish_dot(ws, grid, dot_out);
             return;
@@ -844,13 +844,13 @@ void spmv(const DevSELL &S, const double *x, double *y, double *dot_out, const R
             constexpr int U = decltype(u)::value;
             if (paired)
                 k_spmv<true, U, 1, unsigned int><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.pcol, S.val,
-                                                                                 x, y, ws.dots());
+                                                                                 x, y, ws.dots(grid));
             else if (cols_only)
                 k_spmv<true, U, 4><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, x, y,
-                                                                   ws.dots());
+                                                                   ws.dots(grid));
             else
                 k_spmv<true, U, 1><<<grid, kBlock, 0, stream()>>>(S.n, S.nslices, S.sptr, S.col, S.val, x, y,
-                                                                   ws.dots());
+                                                                   ws.dots(grid));
         });
         if (timer) timer->end();
         HZ_LAUNCH_CHECK();
@@ -936,7 +936,8 @@ void smooth_sweep_dot(const DevSELL &S, int smoother, double w, const double *b,
                       double *xout, double *dot_out, const ReduceWs &ws, LaunchTimer *timer) {
     if (S.n == 0) return;
     if (timer) timer->begin();
-    launch_sweep<false, true>(S, smoother, w, nullptr, nullptr, 1.0, nullptr, b, x, xout, ws.dots());
+    launch_sweep<false, true>(S, smoother, w, nullptr, nullptr, 1.0, nullptr, b, x, xout,
+                             ws.dots(div_up(S.nslices, kSlicesPerBlock)));
     if (timer) timer->end();
     finish_dot(ws, div_up(S.nslices, kSlicesPerBlock), dot_out);
 }
@@ -989,7 +990,8 @@ void up_fused(const DevSELL &S, int smoother, double w, const int *agg, const do
               double *dot_out, const ReduceWs &ws) {
     if (S.n == 0) return;
     if (dot_out) {
-        launch_sweep<true, true>(S, smoother, w, agg, xc, alpha, alpha_dev, b, x, xout, ws.dots());
+        launch_sweep<true, true>(S, smoother, w, agg, xc, alpha, alpha_dev, b, x, xout,
+                                 ws.dots(div_up(S.nslices, kSlicesPerBlock)));
         finish_dot(ws, div_up(S.nslices, kSlicesPerBlock), dot_out);
     } else {
         launch_sweep<true, false>(S, smoother, w, agg, xc, alpha, alpha_dev, b, x, xout, nullptr);
@@ -1039,7 +1041,7 @@ void pcg_update(int n, PcgScalars *s, const double *dot_part, int npart, const d
 void dot(int n, const double *x, const double *y, double *out, const ReduceWs &ws) {
     const int G = stream_grid(n);
     count_bytes(x == y ? 8.0 * n : 16.0 * n);
-    k_dot<<<G, kBlock, 0, stream()>>>(n, x, y, ws.dots());
+    k_dot<<<G, kBlock, 0, stream()>>>(n, x, y, ws.dots(G));
     HZ_LAUNCH_CHECK();
     finish_dot(ws, G, out);
 }

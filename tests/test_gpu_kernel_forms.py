@@ -386,3 +386,55 @@ def test_hec_turn_order_sizes_vs_oracle(lib, orc, libc, n):
     for g, o in zip(lg, lo):
         if "agg" in o:
             assert np.array_equal(g["agg"], o["agg"])
+
+
+_ABOVE_LIMIT = """
+import ctypes as C, sys
+import numpy as np
+sys.path[:0] = [sys.argv[1], sys.argv[1] + "/tests"]
+from hazmath_amd import capi, problems
+from test_gpu_kernel_forms import _banded
+from test_gpu_parity import _set_precision
+lib = capi.load_library()
+o = capi.hz_options()
+lib.hz_get_options(C.byref(o))
+o.return_on_fatal = 1
+lib.hz_set_options(C.byref(o))
+n = int(sys.argv[2])
+A = capi.HostCSR(*_banded(n, [1], 1, 1))
+b = problems.uniform_rhs(n, seed=3)
+out = {}
+for precision in (0, 1):
+    _set_precision(lib, precision)
+    x = capi.HostVec(np.zeros(n))
+    it, amg = capi.solver_params(lib, tol=1e-8, maxit=60, aggregation=capi.HEM, smoother=capi.SMOOTHER_L1DIAG,
+                                 coarse_dof=1000)
+    r = lib.linear_solver_dcsr_krylov_amg(A.ptr(), capi.HostVec(b).ptr(), x.ptr(), C.byref(it), C.byref(amg))
+    out["r%d" % precision], out["x%d" % precision] = r, x.arr
+np.savez(sys.argv[3], **out)
+"""
+
+
+def test_fused_levels_above_their_default_limit(lib, tmp_path):
+    """HZ_FUSE_DOWN_MAX puts a chain's first level of 2,100,000 rows in pairs on the fused kernels: C = 120 coarse rows a
+    workgroup are 8,750 workgroups, a partial each, more than the n / 256 + 1 = 8,204 of the kernels over slices.  Two
+    solutions below 1e-8 of a system of condition 7 / 3 (diagonal 5, off-diagonal entries -1)."""
+    import os
+    import subprocess
+    import sys
+    from pathlib import Path
+    n = 2_100_000
+    assert n // 240 > max(8192, n // 256 + 1)
+    root = str(Path(__file__).resolve().parents[1])
+    out = {}
+    for limit in ("300000", "4000000"):
+        f = tmp_path / f"x{limit}.npz"
+        r = subprocess.run([sys.executable, "-c", _ABOVE_LIMIT, root, str(n), str(f)], timeout=110, capture_output=True,
+                           text=True, env=dict(os.environ, HZ_FUSE_DOWN_MAX=limit))
+        assert r.returncode == 0, r.stdout[-500:] + r.stderr[-2000:]
+        out[limit] = dict(np.load(f))
+    for precision in (0, 1):
+        a, c = out["300000"], out["4000000"]
+        assert a[f"r{precision}"] > 0 and abs(int(a[f"r{precision}"]) - int(c[f"r{precision}"])) <= 1
+        xa, xc = a[f"x{precision}"], c[f"x{precision}"]
+        assert np.linalg.norm(xa - xc) <= 5e-8 * np.linalg.norm(xa)
