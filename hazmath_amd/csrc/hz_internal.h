@@ -417,7 +417,8 @@ struct GsLevel {
     int *dsl0 = nullptr;     // sl0 on the device
     int *order = nullptr;    // rows colour by colour (ascending inside a colour)
     int *rows = nullptr;     // row at a position, -1 where a colour's last slice is not full
-    int *width = nullptr;    // per slice, or null: W everywhere
+    int *place = nullptr;    // per slice, in units of kSlice entries (nslices + 1), or null: W apart
+    bool stream = false;     // the entries do not stay in the caches between colour visits
     int *col = nullptr;
     double *val = nullptr;   // off-diagonal entries, slice column-major (col: positions)
     double *diag = nullptr;  // a_ii per position

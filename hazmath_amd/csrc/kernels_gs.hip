@@ -17,8 +17,11 @@
 // off-diagonal entries column-major as positions (entry k of lane t at
 // 64 (W slice + k) + t, CSR order inside the row, W the longest row, padding a
 // zero entry on the lane's own position) and the diagonal a_ii separately, so
-// that nothing has to be loaded to find a slice's data.  Stored zeros are left
-// out.  A wave handles one slice; one launch per colour, or on levels whose x
+// that nothing has to be loaded to find a slice's data.  Where the padding to W
+// costs more than that (large levels, or rows of very different lengths) every
+// slice has the width of its own longest row, and its place is loaded: with one
+// width a row of 30,000 entries among 1,000,000 would ask for 360 GB.  Stored
+// zeros are left out.  A wave handles one slice; one launch per colour, or on levels whose x
 // fits LDS one workgroup for the whole smoothing call.
 //
 // What bounds a sweep on all but the largest levels is the chain of a colour
@@ -36,6 +39,7 @@
 #include <vector>
 
 #include <rocprim/device/device_radix_sort.hpp>
+#include <rocprim/device/device_scan.hpp>
 
 #include "hz_internal.h"
 
@@ -141,10 +145,16 @@ __global__ void k_jp_round(int n, const int *__restrict__ ia, const int *__restr
     }
 }
 
-// *bad is set when some entry (i, j) has no (j, i)
+// *bad is set when some entry (i, j) has no (j, i).  16 lanes a row: a lane a
+// row spent row length x row length dependent steps on a long one (a row of
+// 30,000 entries: 15 ms).
+constexpr int kSymmetricLanes = 16;
 __global__ void k_gs_symmetric(int n, const int *__restrict__ ia, const int *__restrict__ ja, int *__restrict__ bad) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        for (int k = ia[i]; k < ia[i + 1]; ++k) {
+    const int lane = threadIdx.x % kSymmetricLanes;
+    const int step = gridDim.x * blockDim.x / kSymmetricLanes;
+    for (int i = (blockIdx.x * blockDim.x + threadIdx.x) / kSymmetricLanes; i < n; i += step) {
+        const int k1 = ia[i + 1];
+        for (int k = ia[i] + lane; k < k1; k += kSymmetricLanes) {
             const int j = ja[k];
             if (j == i) continue;
             bool found = false;
@@ -161,6 +171,7 @@ __global__ void k_gs_symmetric(int n, const int *__restrict__ ia, const int *__r
                 return;
             }
         }
+    }
 }
 
 // rows per colour and info[0] = the largest colour; keys and idx for the sort
@@ -190,7 +201,7 @@ __global__ __launch_bounds__(kBlock) void k_color_hist(int n, const int *__restr
 // One wave per slice: the rows at its positions, their positions, and the
 // widest row's off-diagonal entries that a sweep reads (stored zeros are left
 // out; the colouring sees the whole pattern).  cptr: first sorted row of each
-// colour, sl0: first slice.
+// colour, sl0: first slice.  width: nslices + 1, the last 0.
 __global__ __launch_bounds__(kBlock) void k_gs_place(int nslices, int nc, const int *__restrict__ cptr,
                                                      const int *__restrict__ sl0, const int *__restrict__ sorted,
                                                      const int *__restrict__ ia, const int *__restrict__ ja,
@@ -218,6 +229,7 @@ __global__ __launch_bounds__(kBlock) void k_gs_place(int nslices, int nc, const 
     for (int off = kWave / 2; off > 0; off >>= 1) w = max(w, __shfl_xor(w, off, kWave));
     if (lane == 0) {
         width[s] = w;
+        if (s == 0) width[nslices] = 0;
         if (w > info[1]) atomicMax(info + 1, w);
     }
 }
@@ -225,12 +237,15 @@ __global__ __launch_bounds__(kBlock) void k_gs_place(int nslices, int nc, const 
 // Slice fill: one thread per position.  Columns are stored as positions
 // (pos_of[j]): the sweeps work on vectors in that order, where the rows a
 // colour's slice reads lie close together, as they do in the natural order.
-__global__ void k_gs_fill(int nslices, int W, const int *__restrict__ rows, const int *__restrict__ pos_of,
+__global__ void k_gs_fill(int nslices, int W, const int *__restrict__ place, const int *__restrict__ rows,
+                          const int *__restrict__ pos_of,
                           const int *__restrict__ ia, const int *__restrict__ ja, const double *__restrict__ a,
                           int *__restrict__ col, double *__restrict__ val, double *__restrict__ diag) {
     const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= (long)nslices * kSlice) return;
-    const long long base = p / kSlice * W * kSlice + p % kSlice;
+    const int s = (int)(p / kSlice);
+    const long long base = (place ? (long long)place[s] : (long long)s * W) * kSlice + p % kSlice;
+    const int wd = place ? place[s + 1] - place[s] : W;
     const int i = rows[p];
     int k2 = 0;
     double d = 0.0;
@@ -246,7 +261,7 @@ __global__ void k_gs_fill(int nslices, int W, const int *__restrict__ rows, cons
             }
         }
     diag[p] = d;   // 0.0 at an empty position, whose value then stays
-    for (; k2 < W; ++k2) {
+    for (; k2 < wd; ++k2) {
         col[base + (long long)k2 * kSlice] = (int)p;
         val[base + (long long)k2 * kSlice] = 0.0;
     }
@@ -306,9 +321,9 @@ __device__ __forceinline__ double gs_subtract(double t, const GsEntries<U> &e, c
 // One colour (slices s0 .. s0 + ns - 1); a wave per slice.  xout (optional):
 // the new values in the rows' own order as well (the colour's last visit).
 // kNt: the entries stream past the caches (levels whose matrix does not stay
-// there from one colour visit to the next).
-template <int kMode, int U, bool kNt>
-__global__ void __launch_bounds__(kBlock) k_gs_color(int s0, int ns, int W, const int *__restrict__ width,
+// there from one colour visit to the next).  kPlaces: the slices' own widths.
+template <int kMode, int U, bool kNt, bool kPlaces>
+__global__ void __launch_bounds__(kBlock) k_gs_color(int s0, int ns, int W, const int *__restrict__ place,
                                                      const int *__restrict__ rows, const int *__restrict__ col,
                                                      const double *__restrict__ val, const double *__restrict__ diag,
                                                      const double *__restrict__ bp, double *__restrict__ xp, double w,
@@ -317,9 +332,10 @@ __global__ void __launch_bounds__(kBlock) k_gs_color(int s0, int ns, int W, cons
     const int lane = threadIdx.x % kSlice;
     if (sl >= ns) return;
     const int s = s0 + sl, p = s * kSlice + lane;
-    const int wd = width ? width[s] : W;
-    const int *cp = col + (long long)s * W * kSlice + lane;
-    const double *vp = val + (long long)s * W * kSlice + lane;
+    const int q0 = kPlaces ? place[s] : s;
+    const int wd = kPlaces ? place[s + 1] - q0 : W;
+    const int *cp = col + (kPlaces ? (long long)q0 : (long long)s * W) * kSlice + lane;
+    const double *vp = val + (kPlaces ? (long long)q0 : (long long)s * W) * kSlice + lane;
     const double bi = bp[p], d = diag[p], xo = xp[p];
     const int row = xout ? rows[p] : -1;
     double t = bi;
@@ -348,9 +364,10 @@ struct GsProgram {
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // kMixed: the passes differ in mode or weight (looked up per colour visit).
-template <int U, int kThreads, bool kMixed>
-__global__ void __launch_bounds__(kThreads) k_gs_lds(int npos, int ncolors, int W, int steps,
-                                                     const int *__restrict__ sl0, const int *__restrict__ rows,
+// kPlaces: the slices' own widths (their places are kept in LDS).
+template <int U, int kThreads, bool kMixed, bool kPlaces>
+__global__ void __launch_bounds__(kThreads) k_gs_lds(int npos, int ncolors, int W, const int *__restrict__ place,
+                                                     int steps, const int *__restrict__ sl0, const int *__restrict__ rows,
                                                      const int *__restrict__ col, const double *__restrict__ val,
                                                      const double *__restrict__ diag, double *__restrict__ bp,
                                                      const double *__restrict__ b, const double *__restrict__ x,
@@ -358,6 +375,7 @@ __global__ void __launch_bounds__(kThreads) k_gs_lds(int npos, int ncolors, int 
     extern __shared__ double xs[];
     __shared__ int ph_s0[kGsMaxPhase], ph_s1[kGsMaxPhase];
     __shared__ unsigned char ph_pass[kMixed ? kGsMaxPhase : 1];
+    __shared__ int s_place[kPlaces ? kGsLdsPos / kSlice + 1 : 1];
     int nph = 0;
     for (int ps = 0; ps < prog.npass; ++ps) {
         const int count = ncolors - prog.skip[ps];
@@ -369,6 +387,8 @@ __global__ void __launch_bounds__(kThreads) k_gs_lds(int npos, int ncolors, int 
         }
         nph += count;
     }
+    if (kPlaces)
+        for (int s = threadIdx.x; s <= npos / kSlice; s += kThreads) s_place[s] = place[s];
     for (int p = threadIdx.x; p < npos; p += kThreads) {
         const int i = rows[p];
         xs[p] = x && i >= 0 ? x[i] : 0.0;
@@ -386,6 +406,10 @@ __global__ void __launch_bounds__(kThreads) k_gs_lds(int npos, int ncolors, int 
     const int total = nph * steps;   // a colour takes `steps` slices a wave at most
     const int mode0 = prog.mode[0];
     const double w0 = prog.w[0];
+    const auto first = [&](int s) {   // of a lane's entries in slice s
+        return (kPlaces ? (long long)s_place[s] : (long long)s * W) * kSlice + lane;
+    };
+    const auto width = [&](int s) { return kPlaces ? s_place[s + 1] - s_place[s] : W; };
     // the visit that is loaded next: colour visit ph, its step j
     int ph = 0, j = 0;
     auto load = [&](Slice &S) {
@@ -402,16 +426,18 @@ __global__ void __launch_bounds__(kThreads) k_gs_lds(int npos, int ncolors, int 
         S.p = s * kSlice + lane;
         S.bi = bp[S.p];
         S.d = diag[S.p];
-        gs_load<false>(S.e, col + (long long)s * W * kSlice + lane, val + (long long)s * W * kSlice + lane, 0, W, S.p);
+        const long long base = first(s);
+        gs_load<false>(S.e, col + base, val + base, 0, width(s), S.p);
     };
     int done = 0;   // steps of the current visit
     auto compute = [&](Slice &S) {
         if (S.on) {
             double t = gs_subtract(S.bi, S.e, xs);
-            const long long base = (long long)(S.p / kSlice) * W * kSlice + lane;
-            for (int k = U; k < W; k += U) {
+            const long long base = first(S.p / kSlice);
+            const int wd = width(S.p / kSlice);
+            for (int k = U; k < wd; k += U) {
                 GsEntries<U> e;
-                gs_load<false>(e, col + base, val + base, k, W, S.p);
+                gs_load<false>(e, col + base, val + base, k, wd, S.p);
                 t = gs_subtract(t, e, xs);
             }
             const int mode = kMixed ? prog.mode[S.pass] : mode0;
@@ -458,7 +484,7 @@ void gs_prepare(const DevCSR &A, GsLevel &G) {
     int *left = arena().alloc_n<int>(1);
     int h = 0;
     HZ_CHECK(hipMemsetAsync(left, 0, sizeof(int), st));
-    k_gs_symmetric<<<grid_rows(n), kBlock, 0, st>>>(n, A.ia, A.ja, left);
+    k_gs_symmetric<<<grid_rows((long)n * kSymmetricLanes), kBlock, 0, st>>>(n, A.ia, A.ja, left);
     HZ_LAUNCH_CHECK();
     HZ_CHECK(memcpy_sync(&h, left, sizeof(int), hipMemcpyDeviceToHost));
     DevCSR AT;
@@ -523,25 +549,40 @@ void gs_prepare(const DevCSR &A, GsLevel &G) {
     HZ_CHECK(hipMemcpyAsync(dtab, tables.data(), sizeof(int) * tables.size(), hipMemcpyHostToDevice, st));
     G.dsl0 = dtab + nc + 1;
     G.rows = arena().alloc_n<int>((size_t)G.npos);
-    int *width = arena().alloc_n<int>((size_t)ns);
+    // widths of the slices (and 0), then their places in units of kSlice entries
+    int *width = arena().alloc_n<int>((size_t)ns + 1), *place = arena().alloc_n<int>((size_t)ns + 1);
     int *pos_of = c1;   // scratch: the colouring buffers are free now
     k_gs_place<<<div_up(ns, kSlicesPerBlock), kBlock, 0, st>>>(ns, nc, dtab, G.dsl0, sorted, A.ia, A.ja, A.val, G.rows,
                                                                 pos_of, width, info);
     HZ_LAUNCH_CHECK();
     HZ_CHECK(memcpy_sync(&G.W, info + 1, sizeof(int), hipMemcpyDeviceToHost));
-    const size_t room = (size_t)G.npos * std::max(1, G.W);
+    // one width for all where it pads little, and on levels whose sweeps are
+    // chains of loads while it adds no round of loads (16 entries) or at most
+    // doubles the entries; else the slices' own
+    bool one_width = n <= 65536 && G.W <= 16;
+    int total = 0;   // of kSlice entries
+    if (!one_width) {
+        HZ_CHECK(rocprim::exclusive_scan(nullptr, tmp_bytes, width, place, 0, (size_t)ns + 1, rocprim::plus<int>(), st));
+        tmp = arena().alloc(tmp_bytes);
+        HZ_CHECK(rocprim::exclusive_scan(tmp, tmp_bytes, width, place, 0, (size_t)ns + 1, rocprim::plus<int>(), st));
+        HZ_CHECK(memcpy_sync(&total, place + ns, sizeof(int), hipMemcpyDeviceToHost));   // at most the matrix's entries
+        one_width = (long long)ns * G.W <= (n <= 65536 ? 2.0 : 1.25) * total;
+    }
+    G.place = one_width ? nullptr : place;
+    G.stream = n > 65536;
+    const size_t room = (one_width ? (size_t)ns * G.W : (size_t)total) * kSlice + 1;
+    if (trace_enabled())
+        std::fprintf(stderr, "[hz]   Gauss-Seidel n=%d: %d colours, %d slices, longest row %d, %s\n", n, nc, ns, G.W,
+                     one_width ? "one width" : "widths by slice");
     G.diag = arena().alloc_n<double>((size_t)G.npos);
     G.col = arena().alloc_n<int>(room);
     G.val = arena().alloc_n<double>(room);
     G.xp = arena().alloc_n<double>((size_t)G.npos);
     G.bp = arena().alloc_n<double>((size_t)G.npos);
-    k_gs_fill<<<div_up(G.npos, kBlock), kBlock, 0, st>>>(ns, G.W, G.rows, pos_of, A.ia, A.ja, A.val, G.col, G.val,
+    k_gs_fill<<<div_up(G.npos, kBlock), kBlock, 0, st>>>(ns, G.W, G.place, G.rows, pos_of, A.ia, A.ja, A.val, G.col, G.val,
                                                          G.diag);
     HZ_LAUNCH_CHECK();
-    // one workgroup where x and the rest fit LDS; else per-slice widths where
-    // the padding to the longest row is worth the load that skips it
-    G.in_lds = G.npos <= kGsLdsPos;
-    G.width = n > 65536 ? width : nullptr;
+    G.in_lds = G.npos <= kGsLdsPos;   // one workgroup where x and the rest fit LDS
 }
 
 namespace {
@@ -606,14 +647,15 @@ void color_launch(const GsLevel &G, int c, int mode, double w, double *xout) {
     const int s0 = G.sl0[c], ns = G.sl0[c + 1] - G.sl0[c];
     if (ns == 0) return;
     const int grid = div_up(ns, kSlicesPerBlock);
+    auto launch = [&](auto m, auto u, auto nt, auto places) {
+        k_gs_color<decltype(m)::value, decltype(u)::value, decltype(nt)::value, decltype(places)::value>
+            <<<grid, kBlock, 0, stream()>>>(s0, ns, G.W, G.place, G.rows, G.col, G.val, G.diag, G.bp, G.xp, w, xout);
+    };
     auto go = [&](auto m, auto u) {
-        constexpr int M = decltype(m)::value, U = decltype(u)::value;
-        if (G.width)
-            k_gs_color<M, U, true><<<grid, kBlock, 0, stream()>>>(s0, ns, G.W, G.width, G.rows, G.col, G.val, G.diag,
-                                                                  G.bp, G.xp, w, xout);
-        else
-            k_gs_color<M, U, false><<<grid, kBlock, 0, stream()>>>(s0, ns, G.W, G.width, G.rows, G.col, G.val, G.diag,
-                                                                   G.bp, G.xp, w, xout);
+        if (G.stream && G.place) launch(m, u, std::true_type{}, std::true_type{});
+        else if (G.stream) launch(m, u, std::true_type{}, std::false_type{});
+        else if (G.place) launch(m, u, std::false_type{}, std::true_type{});
+        else launch(m, u, std::false_type{}, std::false_type{});
     };
     auto by_mode = [&](auto u) {
         if (mode == 0) go(std::integral_constant<int, 0>{}, u);
@@ -626,18 +668,25 @@ void color_launch(const GsLevel &G, int c, int mode, double w, double *xout) {
 
 // The one-workgroup form: 16 waves with eight entries in flight for short
 // rows, 8 waves with sixteen for longer ones (registers).
-template <int U, int kThreads, bool kMixed>
-void lds_launch(const GsLevel &G, const double *b, const double *x, double *xout, const GsProgram &gp) {
+template <int U, int kThreads, bool kMixed, bool kPlaces>
+void lds_launch_form(const GsLevel &G, const double *b, const double *x, double *xout, const GsProgram &gp) {
     static const bool ready = [] {
-        HZ_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gs_lds<U, kThreads, kMixed>),
+        HZ_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_gs_lds<U, kThreads, kMixed, kPlaces>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, kGsLdsPos * (int)sizeof(double)));
         return true;
     }();
     (void)ready;
     const int steps = std::max(1, div_up(G.most_slices, kThreads / kSlice));
-    k_gs_lds<U, kThreads, kMixed><<<1, kThreads, sizeof(double) * G.npos, stream()>>>(
-        G.npos, G.ncolors, G.W, steps, G.dsl0, G.rows, G.col, G.val, G.diag, G.bp, b, x, xout, gp);
+    k_gs_lds<U, kThreads, kMixed, kPlaces><<<1, kThreads, sizeof(double) * G.npos, stream()>>>(
+        G.npos, G.ncolors, G.W, G.place, steps, G.dsl0, G.rows, G.col, G.val, G.diag, G.bp, b, x, xout, gp);
     HZ_LAUNCH_CHECK();
+}
+
+template <int U, int kThreads, bool kMixed>
+void lds_launch(const GsLevel &G, const double *b, const double *x, double *xout, const GsProgram &gp) {
+    if constexpr (U > 8)   // levels of short rows have one width
+        if (G.place) return lds_launch_form<U, kThreads, kMixed, true>(G, b, x, xout, gp);
+    lds_launch_form<U, kThreads, kMixed, false>(G, b, x, xout, gp);
 }
 
 }  // namespace

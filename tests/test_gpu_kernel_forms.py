@@ -203,27 +203,28 @@ def test_coarse_gmres_after_small_cg_vs_oracle(lib, orc, m):
     assert np.linalg.norm(x - xo) <= 1e-6 * np.linalg.norm(xo)
 
 
-# positions (64 per slice, colours padded): one workgroup up to 18,432, colour launches above; rows of up to 8, up to
-# 16 and over 16 off-diagonal entries; a nonsymmetric pattern; more than 65,536 rows: widths by slice
-@pytest.mark.parametrize("rows,per_row,symmetric", [(1, 0, True), (70, 6, True), (3000, 6, True), (3000, 14, True),
-                                                    (3000, 30, True), (3000, 8, False), (21000, 6, True),
-                                                    (21000, 20, False), (70001, 6, True)])
-@pytest.mark.parametrize("smoother", [capi.SMOOTHER_GS, capi.SMOOTHER_SGS, capi.SMOOTHER_SGSOR])
-def test_gauss_seidel_forms_bitexact(lib, orc, rows, per_row, symmetric, smoother):
-    """Smoothing calls (two sweeps, before and after the coarse correction) in the library's colour order, bit for bit
-    as the oracle sweeps the rows in that order, on every form that the level's size and rows choose."""
+def _gs_matrix(rows, per_row, symmetric, long_row=0):
+    """Diagonally dominant matrix with about per_row off-diagonal entries a row within 300 of the diagonal, and row
+    rows / 2 coupled to `long_row` others spread over all rows."""
     import scipy.sparse as sp
     rng = np.random.default_rng(rows + per_row)
     i = np.repeat(np.arange(rows), per_row // 2 if symmetric else per_row)
     j = (i + rng.integers(1, max(2, min(rows, 300)), i.size)) % rows
     off = sp.csr_matrix((rng.uniform(-1.0, 1.0, i.size), (i, j)), shape=(rows, rows))
+    if long_row:
+        j = np.linspace(0, rows - 1, long_row).astype(np.int64)
+        off = off + sp.csr_matrix((rng.uniform(-1.0, 1.0, long_row), (np.full(long_row, rows // 2), j)),
+                                  shape=(rows, rows))
     if symmetric:
         off = off + off.T
     off.setdiag(0.0)
     off.eliminate_zeros()
     A = (off + sp.diags(1.0 + np.asarray(np.abs(off).sum(axis=1)).ravel())).tocsr()
     A.sort_indices()
-    M = capi.HostCSR(A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data.astype(np.float64))
+    return capi.HostCSR(A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data.astype(np.float64)), rng
+
+
+def _gs_bitexact(lib, orc, M, rows, rng, smoother):
     b, x0 = rng.standard_normal(rows), rng.standard_normal(rows)
     for post in (0, 1):
         order, cptr = np.zeros(rows, np.int32), np.zeros(rows + 2, np.int32)
@@ -236,6 +237,32 @@ def test_gauss_seidel_forms_bitexact(lib, orc, rows, per_row, symmetric, smoothe
                                   capi.dptr(order, capi.INT), capi.dptr(cptr, capi.INT), nc.value)
         assert np.array_equal(np.sort(order), np.arange(rows))
         assert np.array_equal(xg, xo)
+
+
+# positions (64 per slice, colours padded): one workgroup up to 18,432, colour launches above; rows of up to 8, up to
+# 16 and over 16 off-diagonal entries; a nonsymmetric pattern; more than 65,536 rows: widths by slice
+@pytest.mark.parametrize("rows,per_row,symmetric", [(1, 0, True), (70, 6, True), (3000, 6, True), (3000, 14, True),
+                                                    (3000, 30, True), (3000, 8, False), (21000, 6, True),
+                                                    (21000, 20, False), (70001, 6, True)])
+@pytest.mark.parametrize("smoother", [capi.SMOOTHER_GS, capi.SMOOTHER_SGS, capi.SMOOTHER_SGSOR])
+def test_gauss_seidel_forms_bitexact(lib, orc, rows, per_row, symmetric, smoother):
+    """Smoothing calls (two sweeps, before and after the coarse correction) in the library's colour order, bit for bit
+    as the oracle sweeps the rows in that order, on every form that the level's size and rows choose."""
+    M, rng = _gs_matrix(rows, per_row, symmetric)
+    _gs_bitexact(lib, orc, M, rows, rng, smoother)
+
+
+# one workgroup, colour launches, and more than 65,536 rows; the long row's slices alone are that wide
+@pytest.mark.parametrize("rows,long_row", [(3000, 2000), (15000, 9000), (21000, 9000), (70001, 30000)])
+@pytest.mark.parametrize("symmetric", [True, False])
+@pytest.mark.parametrize("smoother", [capi.SMOOTHER_GS, capi.SMOOTHER_SGSOR])
+def test_gauss_seidel_long_row(lib, orc, rows, long_row, symmetric, smoother):
+    """One row far longer than the others: the same bits as the oracle, and memory for the slices' own widths (at the
+    longest row's everywhere the entries alone would take 12 rows long_row bytes, up to 25 GB)."""
+    M, rng = _gs_matrix(rows, 6, symmetric, long_row)
+    lib.hz_release_device_memory()
+    _gs_bitexact(lib, orc, M, rows, rng, smoother)
+    assert lib.hz_device_pool_bytes() <= 512 << 20   # two of the pool's chunks
 
 
 # tiles of 64 rows over 256 workgroups: fewer tiles than workgroups, as many, one more, and several a workgroup with a
