@@ -364,14 +364,15 @@ struct GsProgram {
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // kMixed: the passes differ in mode or weight (looked up per colour visit).
-// kPlaces: the slices' own widths (their places are kept in LDS).
+// kPlaces: the slices' own widths (their places are kept in LDS).  x and xout
+// may be one vector: it is read into LDS before anything is written.
 template <int U, int kThreads, bool kMixed, bool kPlaces>
 __global__ void __launch_bounds__(kThreads) k_gs_lds(int npos, int ncolors, int W, const int *__restrict__ place,
                                                      int steps, const int *__restrict__ sl0, const int *__restrict__ rows,
                                                      const int *__restrict__ col, const double *__restrict__ val,
                                                      const double *__restrict__ diag, double *__restrict__ bp,
-                                                     const double *__restrict__ b, const double *__restrict__ x,
-                                                     double *__restrict__ xout, GsProgram prog) {
+                                                     const double *__restrict__ b, const double *x, double *xout,
+                                                     GsProgram prog) {
     extern __shared__ double xs[];
     __shared__ int ph_s0[kGsMaxPhase], ph_s1[kGsMaxPhase];
     __shared__ unsigned char ph_pass[kMixed ? kGsMaxPhase : 1];
