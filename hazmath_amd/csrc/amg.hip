@@ -345,10 +345,11 @@ int amg_setup(Hierarchy &H, const DevCSR &A0, AMG_param *param, bool) {
 namespace {
 // Levels up to this many rows are latency-bound: they use the fused kernels
 // (HZ_FUSE_DOWN_MAX overrides the default).  PCG ms by limit, 128^3 Poisson /
-// 76^3 anisotropic (438,976 rows) / 128^3 FP32 cycle: 300,000 rows 13.76 /
-// 16.35 / 24.41; 600,000 13.76 / 18.09 / 24.37; every level 14.42 / 18.07 /
-// 24.79.  Above it a level's kernels are bandwidth-bound, and a finest level
-// shares its matrix with the PCG's product through the last-level cache.
+// 76^3 anisotropic (438,976 rows) / 128^3 coefficient jumps with the FP32 cycle:
+// 300,000 rows 12.11 / 13.73 / 24.27; 600,000 12.15 / 16.88 / 24.24; every level
+// 13.72 / 16.89 / 24.59.  Above it a level's kernels are bandwidth-bound, and a
+// finest level has its entry codes and shares its matrix with the PCG's product
+// through the last-level cache.
 int fused_down_max_rows() {
     static int v = -1;
     if (v < 0) {

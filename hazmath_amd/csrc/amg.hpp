@@ -14,7 +14,10 @@ struct FusedLevel {
     int C = 0, K = 0;         // coarse rows and slices of a workgroup
     int nblk = 0;             // workgroups
     int wmax = 0, amax = 0;   // longest row of A and of A P
-    int *width = nullptr, *awidth = nullptr;   // per slice, or null: wmax / amax everywhere
+    int slices = 0;           // nblk K
+    // per slice, where their widths differ: first entry in units of kWave entries
+    // (slices + 1, of A and of A P), or null: wmax apart; width of A P
+    int *place = nullptr, *awidth = nullptr;
     int *prow = nullptr, *pagg = nullptr;      // per position: row (-1: none) and its aggregate
     int *col = nullptr;       // A by position
     void *val = nullptr;

@@ -10,9 +10,12 @@
 // column, aggregate of the column, coarse x).  Here the rows lie in the order
 // in which the restriction adds them: a workgroup owns C consecutive coarse
 // rows, its positions (their member rows, members ascending) are cut into K
-// slices of 64, lane t of a slice holds one row, entry k of it at
-// (64 slice + t) + 64 k of the slice's piece, and every slice's piece has room
-// for the level's longest row, so that its place is computed and not loaded.
+// slices of 64, lane t of a slice holds one row, entry k of it at t + 64 k of
+// the slice's piece, and every slice's piece has room for the level's longest
+// row, so that its place is computed and not loaded.  Where that padding costs
+// more than the load (fused_prepare) the pieces are as wide as their own longest
+// row instead: one row of 60 entries in a level of 287,496 rows of 15 would
+// otherwise take four times the level's memory, twice.
 // Down is then (row, column, value) -> x -> LDS -> store, the row sums formed
 // in the same order as over CSR.  It keeps the rows' residuals w, and up uses
 // them: after the correction the residual is w - alpha (A P) xc, so the sweep
@@ -26,6 +29,8 @@
 // 21.2 -> 16.4 ms.
 #include <algorithm>
 #include <vector>
+
+#include <rocprim/device/device_scan.hpp>
 
 #include "amg.hpp"
 
@@ -66,20 +71,41 @@ __device__ __forceinline__ MT narrow_value(double v) {
     else return (MT)v;
 }
 
+// Width of every slice (and 0 after the last): its longest row.
+__global__ __launch_bounds__(kBlock) void k_fused_width(int slices, int nc, int C, int K, const int *__restrict__ rptr,
+                                                        const int *__restrict__ rmem, const int *__restrict__ len,
+                                                        int *__restrict__ width) {
+    const int s = blockIdx.x * kWaves + threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    if (s >= slices) return;
+    const int blk = s / K, c0 = blk * C, c1 = min(nc, c0 + C);
+    const int q = rptr[c0] + (s - blk * K) * kWave + lane;
+    int w = q < rptr[c1] ? len[rmem[q]] : 0;
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) w = max(w, __shfl_xor(w, off, kWave));
+    if (lane == 0) {
+        width[s] = w;
+        if (s == 0) width[slices] = 0;
+    }
+}
+
+// First entry of slice s: places in units of kWave entries, or wmax apart.
+__device__ __forceinline__ long long slice_base(const int *place, int s, int wmax) {
+    return (place ? (long long)place[s] : (long long)s * wmax) * kWave;
+}
+
 // One wave per slice (and workgroup): its rows' entries from the SELL copy, and
 // the same merged by the aggregate of their column, in order of its first
 // entry, each sum in stored order (the merge runs in LDS).  amax: the longest
 // merged row; *dup: set when a row stores its diagonal more than once.
 constexpr int kMergeMax = 64;
 template <class MT>
-__global__ __launch_bounds__(kWave) void k_fused_fill(int nc, int C, int K, int wmax, int uniform,
+__global__ __launch_bounds__(kWave) void k_fused_fill(int nc, int C, int K, int wmax, const int *__restrict__ place,
                                                       const int *__restrict__ rptr, const int *__restrict__ rmem,
                                                       const int *__restrict__ agg, const int *__restrict__ len,
                                                       const long long *__restrict__ sptr,
                                                       const int *__restrict__ scol, const double *__restrict__ sval,
                                                       int *__restrict__ prow, int *__restrict__ pagg,
-                                                      int *__restrict__ width, int *__restrict__ awidth,
-                                                      int *__restrict__ col, MT *__restrict__ val,
+                                                      int *__restrict__ awidth, int *__restrict__ col, MT *__restrict__ val,
                                                       int *__restrict__ acol, MT *__restrict__ aval,
                                                       int *__restrict__ amax, int *__restrict__ dup) {
     extern __shared__ double s_merge[];   // wmax x 64 sums, then wmax x 64 aggregates
@@ -93,12 +119,10 @@ __global__ __launch_bounds__(kWave) void k_fused_fill(int nc, int C, int K, int 
     pagg[s * kWave + lane] = row >= 0 ? agg[row] : -1;
     const int l = row >= 0 ? len[row] : 0;
     const long long src = row >= 0 ? sptr[row / kSlice] + row % kSlice : 0;
-    const long long dst = (long long)s * kWave * wmax + lane;
-    int w = l;
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) w = max(w, __shfl_xor(w, off, kWave));
+    const long long dst = slice_base(place, s, wmax) + lane;
+    const int w = place ? place[s + 1] - place[s] : wmax;
     int m = 0, ndiag = 0;   // merged entries, stored diagonals
-    for (int k = 0; k < (uniform ? wmax : w); ++k) {
+    for (int k = 0; k < w; ++k) {
         const bool ok = k < l;
         const int c = ok ? scol[src + (long long)k * kSlice] : -1;
         const double a = ok ? sval[src + (long long)k * kSlice] : 0.0;
@@ -121,12 +145,11 @@ __global__ __launch_bounds__(kWave) void k_fused_fill(int nc, int C, int K, int 
     int wa = m;
 #pragma unroll
     for (int off = kWave / 2; off > 0; off >>= 1) wa = max(wa, __shfl_xor(wa, off, kWave));
-    for (int k = 0; k < (uniform ? wmax : wa); ++k) {
+    for (int k = 0; k < (place ? wa : wmax); ++k) {
         acol[dst + (long long)k * kWave] = k < m ? m_agg[k * kWave + lane] : -1;
         aval[dst + (long long)k * kWave] = narrow_value<MT>(k < m ? m_val[k * kWave + lane] : 0.0);
     }
     if (lane == 0) {
-        width[s] = w;
         awidth[s] = wa;
         if (wa > *amax) atomicMax(amax, wa);   // most waves find the maximum there already
     }
@@ -162,8 +185,8 @@ __device__ __forceinline__ void ld_entries(const int *__restrict__ idx, const MT
 
 // wpos = b - A x by position, bc = R (b - A x) and optionally xc = the coarse
 // level's first sweep from zero.
-template <class VT, class MT, int U>
-__global__ __launch_bounds__(kBlock) void k_fused_down(int nc, int C, int K, int wmax, const int *__restrict__ width,
+template <class VT, class MT, int U, bool kPlaces>
+__global__ __launch_bounds__(kBlock) void k_fused_down(int nc, int C, int K, int wmax, const int *__restrict__ place,
                                                        const int *__restrict__ rptr, const int *__restrict__ prow,
                                                        const int *__restrict__ col, const MT *__restrict__ val,
                                                        const VT *__restrict__ b, const VT *__restrict__ x,
@@ -182,8 +205,8 @@ __global__ __launch_bounds__(kBlock) void k_fused_down(int nc, int C, int K, int
     for (int sl = wv; sl < K; sl += kWaves) {
         const int s = blk * K + sl;
         const int row = prow[s * kWave + lane];
-        const int wd = width ? width[s] : wmax;
-        const long long base = (long long)s * kWave * wmax + lane;
+        const int wd = kPlaces ? place[s + 1] - place[s] : wmax;
+        const long long base = slice_base(kPlaces ? place : nullptr, s, wmax) + lane;
         const VT bi = row >= 0 ? b[row] : VT(0);
         VT t = 0;
         for (int k = 0; k < wd; k += U) {
@@ -211,8 +234,9 @@ __global__ __launch_bounds__(kBlock) void k_fused_down(int nc, int C, int K, int
 //   Jacobi  x' + w r / d,  L1DIAG  x' + r / d  (rows with |d| <= SMALLREAL keep x').
 // kOut 1: also partials of sum xout b; kOut 2: the result in FP64 to out64
 // instead, with partials of sum out64 r64.
-template <class VT, class MT, int kOut, int U>
-__global__ __launch_bounds__(kBlock) void k_fused_up(int K, int wmax, int wd0, const int *__restrict__ awidth,
+template <class VT, class MT, int kOut, int U, bool kPlaces>
+__global__ __launch_bounds__(kBlock) void k_fused_up(int K, int wmax, int wd0, const int *__restrict__ place,
+                                                     const int *__restrict__ awidth,
                                                      const int *__restrict__ prow, const int *__restrict__ pagg,
                                                      const int *__restrict__ acol, const MT *__restrict__ aval,
                                                      VT wgt, const VT *__restrict__ dsm, const VT *__restrict__ xc,
@@ -230,8 +254,8 @@ __global__ __launch_bounds__(kBlock) void k_fused_up(int K, int wmax, int wd0, c
         const int s = blk * K + sl;
         const int row = prow[s * kWave + lane], g = pagg[s * kWave + lane];
         const VT w = wpos[s * kWave + lane];
-        const int wd = awidth ? awidth[s] : wd0;
-        const long long base = (long long)s * kWave * wmax + lane;
+        const int wd = kPlaces ? awidth[s] : wd0;
+        const long long base = slice_base(kPlaces ? place : nullptr, s, wmax) + lane;
         VT x0 = 0, xg0 = 0, d = 0, bi = 0;
         double ri = 0.0;
         VT t = 0;
@@ -272,14 +296,19 @@ __global__ __launch_bounds__(kBlock) void k_fused_up(int K, int wmax, int wd0, c
     }
 }
 
-// Entries a round: the longest row's, up to 32 where the whole row is one
-// round of loads on the levels with a common width (latency-bound: a second
-// round doubles the chain), up to 16 where the widths differ.
+// Entries a round, and whether the slices have places: the longest row's, up
+// to 32 where the whole row is one round of loads on the levels with a common
+// width (latency-bound: a second round doubles the chain), up to 16 where the
+// widths differ.
 template <class F>
-void by_width(int longest, bool differ, F &&launch) {
-    if (longest <= 8) launch(std::integral_constant<int, 8>{});
-    else if (longest <= 16 || differ) launch(std::integral_constant<int, 16>{});
-    else launch(std::integral_constant<int, 32>{});
+void by_width(int longest, bool places, F &&launch) {
+    const auto go = [&](auto u) {
+        if (places) launch(u, std::true_type{});
+        else launch(u, std::false_type{});
+    };
+    if (longest <= 8) go(std::integral_constant<int, 8>{});
+    else if (longest <= 16 || places) go(std::integral_constant<int, 16>{});
+    else launch(std::integral_constant<int, 32>{}, std::false_type{});
 }
 
 template <class F>
@@ -311,6 +340,8 @@ void fused_prepare(std::vector<Level *> &levels, const std::vector<int> &kinds, 
     }
     std::vector<int> h((size_t)nl * kInfo);
     HZ_CHECK(memcpy_sync(h.data(), info, sizeof(int) * nl * kInfo, hipMemcpyDeviceToHost));
+    std::vector<int> total(nl, 0);   // of kWave entries
+    bool placed = false;
     for (int i = 0; i < nl; ++i) {
         Level &L = *levels[i];
         FusedLevel &F = L.F;
@@ -323,27 +354,52 @@ void fused_prepare(std::vector<Level *> &levels, const std::vector<int> &kinds, 
         // list-walking kernels
         if (h[kInfo * i + 2] != L.A.n || F.K > kMaxSlices || F.wmax > kMergeMax || room > 8 * L.S.nent + (1 << 20))
             continue;
-        // a common width where the padding costs little or the level is tiny
-        const bool uniform = L.A.n <= 65536 || room <= L.S.nent + L.S.nent / 4;
+        F.slices = (int)slices;
+        // a common width where the padding costs little, or on the latency-bound
+        // levels while it is not many times the entries (measured: 1.1 to 3.7
+        // times); else the slices' own widths
+        if (L.A.n <= 65536 ? room > 4 * L.S.nent + (1 << 16) : room > L.S.nent + L.S.nent / 4) {
+            int *width = arena().alloc_n<int>((size_t)slices + 1);
+            F.place = arena().alloc_n<int>((size_t)slices + 1);
+            k_fused_width<<<div_up(slices, kWaves), kBlock, 0, st>>>(F.slices, L.nagg, F.C, F.K, L.rptr, L.rmem, L.S.len,
+                                                                     width);
+            HZ_LAUNCH_CHECK();
+            size_t tmp_bytes = 0;
+            HZ_CHECK(rocprim::exclusive_scan(nullptr, tmp_bytes, width, F.place, 0, (size_t)slices + 1,
+                                             rocprim::plus<int>(), st));
+            void *tmp = arena().alloc(tmp_bytes);
+            HZ_CHECK(rocprim::exclusive_scan(tmp, tmp_bytes, width, F.place, 0, (size_t)slices + 1,
+                                             rocprim::plus<int>(), st));
+            placed = true;
+            HZ_CHECK(hipMemcpyAsync(&total[i], F.place + slices, sizeof(int), hipMemcpyDeviceToHost, st));
+        } else {
+            total[i] = (int)(slices * F.wmax);   // at most 8 S.nent + 2^20 entries of kWave
+        }
+        F.on = true;
+    }
+    if (placed) HZ_CHECK(hipStreamSynchronize(st));
+    for (int i = 0; i < nl; ++i) {
+        Level &L = *levels[i];
+        FusedLevel &F = L.F;
+        if (!F.on) continue;
+        const int slices = F.slices;
+        const size_t room = (size_t)total[i] * kWave;
         F.prow = arena().alloc_n<int>((size_t)slices * kWave);
         F.pagg = arena().alloc_n<int>((size_t)slices * kWave);
-        int *width = arena().alloc_n<int>((size_t)slices), *awidth = arena().alloc_n<int>((size_t)slices);
-        F.col = arena().alloc_n<int>((size_t)room);
-        F.acol = arena().alloc_n<int>((size_t)room);
-        F.width = uniform ? nullptr : width;
-        F.awidth = uniform ? nullptr : awidth;
+        F.awidth = arena().alloc_n<int>((size_t)slices);
+        F.col = arena().alloc_n<int>(room);
+        F.acol = arena().alloc_n<int>(room);
         F.wpos = arena().alloc((size_t)slices * kWave * (F.kind == 0 ? sizeof(double) : sizeof(float)));
         by_kind(F.kind, [&](auto m) {
             using MT = decltype(m);
-            MT *v = arena().alloc_n<MT>((size_t)room), *av = arena().alloc_n<MT>((size_t)room);
+            MT *v = arena().alloc_n<MT>(room), *av = arena().alloc_n<MT>(room);
             F.val = v;
             F.aval = av;
-            k_fused_fill<MT><<<(int)slices, kWave, (size_t)F.wmax * kWave * (sizeof(double) + sizeof(int)), st>>>(
-                L.nagg, F.C, F.K, F.wmax, uniform ? 1 : 0, L.rptr, L.rmem, L.agg, L.S.len, L.S.sptr, L.S.col, L.S.val,
-                F.prow, F.pagg, width, awidth, F.col, v, F.acol, av, info + kInfo * i + 3, info + kInfo * i + 4);
+            k_fused_fill<MT><<<slices, kWave, (size_t)F.wmax * kWave * (sizeof(double) + sizeof(int)), st>>>(
+                L.nagg, F.C, F.K, F.wmax, F.place, L.rptr, L.rmem, L.agg, L.S.len, L.S.sptr, L.S.col, L.S.val, F.prow,
+                F.pagg, F.awidth, F.col, v, F.acol, av, info + kInfo * i + 3, info + kInfo * i + 4);
         });
         HZ_LAUNCH_CHECK();
-        F.on = true;
     }
     HZ_CHECK(memcpy_sync(h.data(), info, sizeof(int) * nl * kInfo, hipMemcpyDeviceToHost));
     for (int i = 0; i < nl; ++i) {
@@ -361,12 +417,13 @@ static void fused_down_impl(const Level &L, const VT *b, const VT *x, VT *bc, in
     const int vb = F.kind == 0 ? 8 : (F.kind == kLowF32 ? 4 : 2);
     count_bytes((vb + 4.0) * L.S.nnz + (4.0 + 3.0 * sizeof(VT)) * L.A.n + 4.0 * (L.nagg + 1) +
                 (xc ? 3.0 : 1.0) * sizeof(VT) * L.nagg);
-    by_width(F.wmax, F.width != nullptr, [&](auto u) {
+    by_width(F.wmax, F.place != nullptr, [&](auto u, auto places) {
         constexpr int U = decltype(u)::value;
+        constexpr bool kPlaces = decltype(places)::value;
         auto go = [&](auto m) {
             using MT = decltype(m);
-            k_fused_down<VT, MT, U><<<F.nblk, kBlock, sizeof(VT) * F.K * kWave, stream()>>>(
-                L.nagg, F.C, F.K, F.wmax, F.width, L.rptr, F.prow, F.col, static_cast<const MT *>(F.val), b, x,
+            k_fused_down<VT, MT, U, kPlaces><<<F.nblk, kBlock, sizeof(VT) * F.K * kWave, stream()>>>(
+                L.nagg, F.C, F.K, F.wmax, F.place, L.rptr, F.prow, F.col, static_cast<const MT *>(F.val), b, x,
                 static_cast<VT *>(F.wpos), bc, smoother, (VT)w, dc, xc);
         };
         if constexpr (sizeof(VT) == 8) go(double{});
@@ -386,13 +443,14 @@ static void fused_up_impl(const Level &L, int smoother, double w, const VT *dsm,
     count_bytes((vb + 4.0) * L.S.nnz + (8.0 + 4.0 * sizeof(VT)) * L.A.n + (out64 ? 16.0 * L.A.n : 0.0));
     double *part = dot_out || out64 ? ws.dots(F.nblk) : nullptr;
     const VT wgt = smoother == HZ_SMOOTHER_L1DIAG ? VT(1) : (VT)w;
-    by_width(F.amax, F.awidth != nullptr, [&](auto u) {
+    by_width(F.amax, F.place != nullptr, [&](auto u, auto places) {
         constexpr int U = decltype(u)::value;
+        constexpr bool kPlaces = decltype(places)::value;
         auto launch = [&](auto m, auto out) {
             using MT = decltype(m);
-            k_fused_up<VT, MT, decltype(out)::value, U><<<F.nblk, kBlock, 0, stream()>>>(
-                F.K, F.wmax, F.amax, F.awidth, F.prow, F.pagg, F.acol, static_cast<const MT *>(F.aval), wgt, dsm, xc,
-                alpha, alpha_dev, static_cast<const VT *>(F.wpos), b, x, xout, out64, r64, part);
+            k_fused_up<VT, MT, decltype(out)::value, U, kPlaces><<<F.nblk, kBlock, 0, stream()>>>(
+                F.K, F.wmax, F.amax, F.place, F.awidth, F.prow, F.pagg, F.acol, static_cast<const MT *>(F.aval), wgt, dsm,
+                xc, alpha, alpha_dev, static_cast<const VT *>(F.wpos), b, x, xout, out64, r64, part);
         };
         if constexpr (sizeof(VT) == 8) {
             if (dot_out) launch(double{}, std::integral_constant<int, 1>{});

@@ -67,6 +67,18 @@ def _dirichlet_rows(m):
     return M.indptr.astype(np.int32), M.indices.astype(np.int32), M.data
 
 
+def _star(ia, ja, va, entries):
+    """The matrix with `entries` weak couplings of row 0, spread over all rows, added."""
+    import scipy.sparse as sp
+    n = ia.size - 1
+    j = np.linspace(n // 3, n - 1, entries).astype(np.int64)
+    S = sp.coo_matrix((np.full(entries, -1e-3), (np.zeros(entries, np.int64), j)), shape=(n, n)).tocsr()
+    S = S + S.T
+    M = (sp.csr_matrix((va, ja, ia), shape=(n, n)) + S - sp.diags(np.asarray(S.sum(axis=1)).ravel())).tocsr()
+    M.sort_indices()
+    return M.indptr.astype(np.int32), M.indices.astype(np.int32), M.data
+
+
 def _long_row(m, entries):
     """2-D Laplacian with `entries` weak couplings of row 0 added (symmetric, diagonally dominant)."""
     import scipy.sparse as sp
@@ -103,6 +115,7 @@ FUSED = {
     "kuhn_hem": (lambda: problems.poisson3d_kuhn(22), capi.HEM),      # pairs, zeros left out
     "aniso_hec": (lambda: problems.aniso3d_kuhn(24, 0.7, 0.05), capi.HEC),   # rows of over 16 entries below
     "large_hem": (lambda: problems.aniso3d_kuhn(46, 0.7, 0.05), capi.HEM),   # 91,125 rows: widths by slice
+    "row45": (lambda: _star(*problems.aniso3d_kuhn(46, 0.7, 0.05), 45), capi.HEM),   # places, one wide slice a level
     "dirichlet": (lambda: _dirichlet_rows(50), capi.HEC),             # rows in no aggregate: the list-walking kernels
     "row64": (lambda: _long_row(40, 59), capi.HEC),                   # the longest row that the merge takes
     "two_diagonals": (lambda: _two_diagonals(40), capi.HEC),          # Jacobi: the list-walking kernels
@@ -158,6 +171,28 @@ def test_fused_cycle_kernels_vs_oracle(lib, orc, libc, case, smoother):
     assert off(0, "oracle") < 1e-12
     assert off(1, 0) < 2e-5
     assert off(2, 0) < 5e-2
+
+
+def test_fused_layout_memory_with_a_long_row(lib, libc):
+    """A row of 60 entries in a level of 287,496 rows of 15 costs the fused layout its own slice's padding: the solve's
+    pool grows by no more than one of its chunks (with the longest row's room in every slice, A and A P took 24 bytes
+    times 45 more entries a row there and as many again on the levels below, 600 MB)."""
+    base = problems.aniso3d_kuhn(67, 0.7, 0.05)
+    held = []
+    for ia, ja, va in (base, _star(*base, 45)):
+        A = capi.HostCSR(ia, ja, va)
+        n = ia.size - 1
+        lib.hz_release_device_memory()
+        b, x = capi.HostVec(problems.uniform_rhs(n, seed=4)), capi.HostVec(np.zeros(n))
+        it, amg = capi.solver_params(lib, tol=1e-6, maxit=200, aggregation=capi.HEM, smoother=capi.SMOOTHER_L1DIAG,
+                                     coarse_dof=1000, theta=0.04)
+        libc.srand(1)
+        r = lib.linear_solver_dcsr_krylov_amg(A.ptr(), b.ptr(), x.ptr(), C.byref(it), C.byref(amg))
+        assert r > 0
+        held.append(lib.hz_device_pool_bytes())
+    lib.hz_release_device_memory()
+    print(f"[fused] pool {held[0] >> 20} MB, with the long row {held[1] >> 20} MB", flush=True)
+    assert held[1] - held[0] <= 256 << 20
 
 
 # thread counts of the one-row-a-thread CG are 64, 256, 512 and 1,024; 1,025 rows run the general form; 20
