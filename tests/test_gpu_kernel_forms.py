@@ -345,34 +345,43 @@ def test_mlp_gradient_tiles_vs_fp64(lib, B):
 # and a rest); 25 rows are solved at level 0
 @pytest.mark.parametrize("pre,post,coarse", [(1, 1, 30), (2, 2, 600), (0, 1, 100), (1, 0, 100), (0, 0, 30)])
 def test_batch_cycle_forms_vs_single_system(lib, libc, pre, post, coarse):
-    """Every pair as the single-system solver with the same FP32 cycle.  The cycles round differently, which moves the
-    iterates by 2^-24 relative and the iteration at which 1e-8 is passed by at most one; both solutions are then within
-    1e-8 times the condition number (below 1e4 here) of the true one, 1e-4 of each other."""
+    """Every pair as the single-system solver with the same FP32 cycle.  Three iterations on every form of the cycle,
+    also those whose iteration does not converge: the iterates differ by what the cycles' applications do, each at most
+    2e-5 (the FP32 cycle's bound against FP64) and each step from the one before, 1e-4 in all.  Solves to 1e-8 with
+    smoothing on both sides: the iteration at which it is passed moves by at most one; both solutions are within 1e-8
+    times the condition number (below 1e4 here) of the true one, 1e-4 of each other."""
     systems = [problems.aniso2d_p1(m, 0.4 + 0.1 * m, 0.3) for m in (32, 6, 33, 34, 48)]
     B = [problems.batch_rhs(s[0].size - 1, k, nrhs=3) for k, s in enumerate(systems)]
-    X = [np.zeros_like(b) for b in B]
 
-    def params():
-        it, amg = capi.solver_params(lib, tol=1e-8, maxit=60, aggregation=capi.HEM, smoother=capi.SMOOTHER_JACOBI,
+    def params(maxit):
+        it, amg = capi.solver_params(lib, tol=1e-8, maxit=maxit, aggregation=capi.HEM, smoother=capi.SMOOTHER_JACOBI,
                                      coarse_dof=coarse, theta=0.04)
         amg.presmooth_iter, amg.postsmooth_iter = pre, post
         return it, amg
-    r, iters = capi.batch_solve(lib, systems, B, X, *params())
+
     old = _set_precision(lib, 1)
     try:
-        for k, (ia, ja, va) in enumerate(systems):
-            A = capi.HostCSR(ia, ja, va)
-            for q in range(3):
-                its, amgs = params()
-                x = capi.HostVec(np.zeros(ia.size - 1))
-                libc.srand(1)
-                rs = lib.linear_solver_dcsr_krylov_amg(A.ptr(), capi.HostVec(B[k][q]).ptr(), x.ptr(), C.byref(its),
-                                                       C.byref(amgs))
-                print(f"[batch] {pre},{post},{coarse} system {k} rhs {q}: {iters[k, q]} single {rs}", flush=True)
-                assert (rs > 0) == (iters[k, q] > 0)
-                if rs > 0:
-                    assert abs(int(iters[k, q]) - rs) <= 1
-                    assert np.linalg.norm(X[k][q] - x.arr) <= 1e-4 * np.linalg.norm(x.arr)
+        for maxit in (3, 60) if pre and post else (3,):
+            X = [np.zeros_like(b) for b in B]
+            r, iters = capi.batch_solve(lib, systems, B, X, *params(maxit))
+            for k, (ia, ja, va) in enumerate(systems):
+                A = capi.HostCSR(ia, ja, va)
+                direct = ia.size - 1 <= coarse   # solved by the coarsest inverse alone: one step, or two
+                for q in range(3):
+                    its, amgs = params(maxit)
+                    x, b = capi.HostVec(np.zeros(ia.size - 1)), capi.HostVec(B[k][q])
+                    libc.srand(1)
+                    rs = lib.linear_solver_dcsr_krylov_amg(A.ptr(), b.ptr(), x.ptr(), C.byref(its), C.byref(amgs))
+                    off = np.linalg.norm(X[k][q] - x.arr) / np.linalg.norm(x.arr)
+                    print(f"[batch] {pre},{post},{coarse} {maxit} system {k} rhs {q}: {iters[k, q]} single {rs}, {off:.1e}",
+                          flush=True)
+                    if direct:
+                        assert rs > 0 and 0 < iters[k, q] <= rs + 1
+                    elif maxit == 3 or k == 4:   # system 4's anisotropy needs more than 60
+                        assert rs == iters[k, q] == -48
+                    else:
+                        assert rs > 0 and abs(int(iters[k, q]) - rs) <= 1
+                    assert off <= 1e-4 or (k == 4 and maxit == 60)
     finally:
         _set_precision(lib, old)
 
@@ -402,9 +411,10 @@ def _banded(n, offsets, classes, diags):
     (65601, [1], 127, 1, True), (65601, [1], 127, 2, False), (65536, [1, 50, 51], 1, 1, True),
     (65576, [1, 30, 31], 1, 1, True),
     (65601, [1, 50, 51, 700], 2, 3, True), (65601, [1, 2, 3, 50, 51, 52, 900, 901, 902], 3, 1, True)])
-@pytest.mark.parametrize("precision", [0, 1])
-@pytest.mark.parametrize("smoother", ["jacobi", "l1", "cheb", "sgs"])
-def test_entry_codes_bitexact(lib, libc, monkeypatch, n, offsets, classes, diags, coded, precision, smoother):
+# (the FP32 cycle has no Gauss-Seidel)
+@pytest.mark.parametrize("smoother,precision", [("jacobi", 0), ("jacobi", 1), ("l1", 0), ("l1", 1), ("cheb", 0),
+                                                ("cheb", 1), ("sgs", 0)])
+def test_entry_codes_bitexact(lib, libc, monkeypatch, n, offsets, classes, diags, coded, smoother, precision):
     """The kernels over entry codes add the same products in the same order as those over columns and values: the same
     iterations and solution bits with the codes off (HZ_COL16=0).  Where the matrix has them an iteration's product alone
     streams 11 bytes an entry fewer; 16-bit column offsets alone save 2 in each of at most 3 kernels."""
@@ -413,8 +423,6 @@ def test_entry_codes_bitexact(lib, libc, monkeypatch, n, offsets, classes, diags
     kw = dict(tol=1e-8, maxit=30, aggregation=capi.HEM, coarse_dof=500,
               smoother=dict(jacobi=capi.SMOOTHER_JACOBI, l1=capi.SMOOTHER_L1DIAG, cheb=capi.SMOOTHER_CHEBY,
                             sgs=capi.SMOOTHER_SGS)[smoother])
-    if smoother == "sgs" and precision == 1:
-        pytest.skip("the FP32 cycle has no Gauss-Seidel")
     out = {}
     old = _set_precision(lib, precision)
     try:
