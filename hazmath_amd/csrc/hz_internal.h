@@ -20,6 +20,7 @@ struct DevSELL {
     int n = 0, nslices = 0;
     long long nnz = 0;         // entries without the padding (algorithmic bytes count these)
     long long nent = 0;        // padded entries
+    int nwide = 0;             // slices wider than kWideSlice, where counted (without zeros)
     long long *sptr = nullptr; // nslices+1 offsets
     int *len = nullptr;        // entries of each row
     int *col = nullptr;
@@ -39,11 +40,14 @@ struct DevSELL {
 };
 
 // Entries a round of the masked SELL kernels: 8 where the slices are at most 8
-// wide on average (stored zeros left out: 7-point rows), else 16.  launch takes
-// the count as a std::integral_constant.
+// wide on average (stored zeros left out: 7-point rows), else 16; 16 also where
+// a slice is much wider, since its rounds then bound the launch (59,319 rows
+// of 7 and one of 307 entries: product 38.5 us in rounds of 8, 32.4 of 16).
+// launch takes the count as a std::integral_constant.
+constexpr int kWideSlice = 32;
 template <class F>
 void by_round(const DevSELL &S, F &&launch) {
-    if (S.nent <= 8LL * kSlice * S.nslices) launch(std::integral_constant<int, 8>{});
+    if (S.nent <= 8LL * kSlice * S.nslices && S.nwide == 0) launch(std::integral_constant<int, 8>{});
     else launch(std::integral_constant<int, 16>{});
 }
 

@@ -49,8 +49,10 @@ constexpr int kSellStage = 1024;
 // one bit an entry in LDS, and each lane counts its row's bits; the column of
 // a zero entry is looked at to keep diagonal ones.  kept: entries kept, over
 // kKeptParts counters in lines of their own (with one counter for all waves
-// its atomics took 70 of the 97 us at 438,976 rows).
-constexpr int kKeptParts = 32, kKeptStride = 8;
+// its atomics took 70 of the 97 us at 438,976 rows), and from bit kWideShift on
+// the slices that by_round counts as wide (one atomic a wave for both: a second
+// one, or a look at a maximum first, cost 50 us a level at 128^3).
+constexpr int kKeptParts = 32, kKeptStride = 8, kWideShift = 40;
 __global__ __launch_bounds__(kBlock) void k_slice_width_nz(int n, const int *__restrict__ ia,
                                                            const int *__restrict__ ja,
                                                            const double *__restrict__ val,
@@ -93,7 +95,8 @@ __global__ __launch_bounds__(kBlock) void k_slice_width_nz(int n, const int *__r
     }
     if (lane == 0) {
         wcount[s] = (long long)widest * kSlice;
-        if (len) atomicAdd(kept + (s % kKeptParts) * kKeptStride, (unsigned long long)len);
+        const unsigned long long wide = widest > kWideSlice ? 1ull << kWideShift : 0ull;
+        if (len) atomicAdd(kept + (s % kKeptParts) * kKeptStride, (unsigned long long)len + wide);
     }
 }
 
@@ -794,7 +797,10 @@ void sell_from_csr(const DevCSR &A, DevSELL &S, bool drop_zeros) {
     S.nent = tail[0];
     if (drop_zeros) {
         S.nnz = 0;
-        for (int p = 0; p < kParts; p += kKeptStride) S.nnz += tail[1 + p];
+        for (int p = 0; p < kParts; p += kKeptStride) {
+            S.nnz += tail[1 + p] & ((1ll << kWideShift) - 1);
+            S.nwide += (int)(tail[1 + p] >> kWideShift);
+        }
     }
     S.col = arena().alloc_n<int>((size_t)S.nent + 1);
     S.val = arena().alloc_n<double>((size_t)S.nent + 1);
