@@ -732,16 +732,18 @@ def main():
     # at most 255 different (offset, value) pairs on such a level: one byte an entry
     coded = (n >= 65536 and os.environ.get("HZ_COL16", "1") != "0"
              and distinct_pairs(ja.astype(np.int64) - rows, va) <= 255)
-    eb = 1 if coded else 10 if paired else 12
+    eb = 10 if paired else 12
     # the solve's copies leave stored off-diagonal zeros out: its kernels are
     # priced at the entries they stream
     kept = int(np.count_nonzero((va != 0.0) | (ja == rows)))
-    bytes_spmv = eb * kept + 4 * (n + 1) + 16 * n
+    # (the kernels over codes read no row pointers)
+    matrix = kept if coded else eb * kept + 4 * (n + 1)
+    bytes_spmv = matrix + 16 * n
     bytes_jacobi = 12 * nnz + 4 * (n + 1) + 24 * n
     # residual w = b - A x: matrix, x and b read, w written; last sweep: matrix, b (= r) and x
     # read, x' written ((x', r) needs no other array)
-    bytes_res = eb * kept + 4 * (n + 1) + 24 * n
-    bytes_sweep_dot = eb * kept + 4 * (n + 1) + 24 * n
+    bytes_res = matrix + 24 * n
+    bytes_sweep_dot = matrix + 24 * n
     spmv_gbs = bytes_spmv / (pcg_spmv_ms * 1e-3) / 1e9
     jac_gbs = bytes_jacobi / (kt.jacobi_ms * 1e-3) / 1e9 if kt.jacobi_ms > 0 else None
 

@@ -18,9 +18,10 @@ constexpr int kCodedBlock = 256, kCodedSlices = kCodedBlock / kWave;
 // residual 31 -> 17, last sweep 38 -> 21; 15-entry rows FP32 Chebyshev step 39
 // -> 16, FP64 product 63 -> 25; 438,976 rows of 15: 15.5 -> 7.4-10.  With the
 // slices' places loaded first the Chebyshev step took 20 us, with 64-bit
-// addresses as well 24; several slices in turn by a workgroup gained nothing.  Entries are added in stored
-// order and the partial of a workgroup is that of its 256 rows, as in the kernels
-// that read columns and values: results and dots are bit-identical to theirs.
+// addresses as well 24; several slices in turn by a workgroup gained nothing.
+// Entries are added in stored order and the partial of a workgroup is that of
+// its 256 rows, as in the kernels that read columns and values: results and dots
+// are bit-identical to theirs.
 template <int U, class T, class Op>
 __global__ __launch_bounds__(kCodedBlock) void k_coded(int n, int nslices, int words, const code8 *__restrict__ code,
                                                        const CodeEntry<T> *__restrict__ table, Op op,
@@ -80,8 +81,9 @@ void launch_coded(const DevSELL &S, const Op &op, double *partials = nullptr) {
     HZ_LAUNCH_CHECK();
 }
 
-// bytes of the codes and row lengths a coded kernel reads
-inline double coded_bytes(const DevSELL &S) { return (double)S.nnz + 4.0 * (S.n + 1); }
+// bytes of the matrix a coded kernel cannot do without: a code an entry (padding
+// ends a row, so no row pointers or lengths are read)
+inline double coded_bytes(const DevSELL &S) { return (double)S.nnz; }
 
 // w = b - A x
 template <class T>

@@ -185,8 +185,6 @@ struct CodeEntry {
     T val;
     int off;
 };
-template <class T>
-using CodeTable = CodeEntry<T>[kCodes];
 
 // 16-bit column offsets from the row, two entries of a row to a 32-bit word:
 // entry 2p of the row in the low half of word p, 2p+1 in the high half, words

@@ -417,7 +417,7 @@ def _banded(n, offsets, classes, diags):
 def test_entry_codes_bitexact(lib, libc, monkeypatch, n, offsets, classes, diags, coded, smoother, precision):
     """The kernels over entry codes add the same products in the same order as those over columns and values: the same
     iterations and solution bits with the codes off (HZ_COL16=0).  Where the matrix has them an iteration's product alone
-    streams 11 bytes an entry fewer; 16-bit column offsets alone save 2 in each of at most 3 kernels."""
+    streams 11 bytes an entry fewer and no row pointers; 16-bit column offsets alone save 2 in each of at most 3 kernels."""
     A = capi.HostCSR(*_banded(n, offsets, classes, diags))
     b = problems.uniform_rhs(n, seed=5)
     kw = dict(tol=1e-8, maxit=30, aggregation=capi.HEM, coarse_dof=500,
