@@ -30,9 +30,9 @@
 // rounds of 8 or 16 masked loads (rows of 6 entries took six dependent pairs of
 // loads when only whole rounds of eight were batched), and the one-workgroup
 // form loads a wave's next two slices ahead.  Measured on the 64^3 Poisson
-// hierarchy (SGS, 11 colours): a colour's launch 7.5 -> 4.1 us, the one-workgroup
-// call on 7,811 / 3,902 / 1,950 rows 165 / 90 / 65 -> 62 / 40 / 29 us, PCG
-// 42.5 -> 26.2 ms; the preparation (rows sorted and placed on the GPU, no
+// hierarchy (SGS, 11 colours): a colour's launch 7.5 -> 3.5-4.0 us, the
+// one-workgroup call on 7,811 / 3,902 / 1,950 rows 165 / 90 / 65 -> 62 / 40 / 29
+// us, PCG 42.5 -> 25.8 ms; the preparation (rows sorted and placed on the GPU, no
 // transpose where the pattern is symmetric) 9 -> 5 ms over eight levels.
 #include <algorithm>
 #include <type_traits>
