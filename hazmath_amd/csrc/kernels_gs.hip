@@ -21,8 +21,8 @@
 // costs more than that (large levels, or rows of very different lengths) every
 // slice has the width of its own longest row, and its place is loaded: with one
 // width a row of 30,000 entries among 1,000,000 would ask for 360 GB.  Stored
-// zeros are left out.  A wave handles one slice; one launch per colour, or on levels whose x
-// fits LDS one workgroup for the whole smoothing call.
+// zeros are left out.  A wave handles one slice; one launch per colour, or on
+// levels whose x fits LDS one workgroup for the whole smoothing call.
 //
 // What bounds a sweep on all but the largest levels is the chain of a colour
 // visit: a launch or a barrier, the entries' loads, the gathers, the division
